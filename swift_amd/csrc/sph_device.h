@@ -80,6 +80,7 @@ __device__ __forceinline__ float kernel_dw(float u) {
 __device__ __forceinline__ bool pair_frame(const int o[3], const int ci[3],
                                            const int cj[3], const double t[3],
                                            const double w[3], double *fo) {
+#pragma clang fp contract(off)
   const int sid = 9 * (o[0] + 1) + 3 * (o[1] + 1) + (o[2] + 1);
   const bool up_j = sid > 13;
 #pragma unroll

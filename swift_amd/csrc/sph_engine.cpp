@@ -97,7 +97,7 @@ struct swsph_engine {
     int *d_start = nullptr, *d_cell_chunk = nullptr, *d_chunk_cell = nullptr;
     double *d_bbox = nullptr;
     float *d_hg2max = nullptr;
-    // boxes of the pre-test records (the tables of the sparse tiles)
+    // boxes of the pre-test records
     float4 *d_fbox = nullptr;
     // positions the boxes were formed from (engine pos_gen; 0: unknown)
     uint64_t pos_gen = 0;
@@ -126,6 +126,7 @@ struct swsph_engine {
   TileScratch ts{};
   size_t tile_cap = 0;  // entries of ts.tile_start / ts.tile_cell
   int tiles_c = 0;  // capacity of the all-active tile table in ts, 0: none
+  int tiles_n = -1;  // tiles of the table in ts (-1: not read back)
   // Steps with few active particles per cell (fewer than sparse_per_cell on
   // average) run their pass with tiles of sparse_ci against chunks of
   // sparse_cj in all three loops; 0 disables.
@@ -298,6 +299,10 @@ LoopArgs loop_args(const swsph_engine *e) {
   la.pos_eps = pos_eps(e);
   la.cmask = e->cmask_on ? e->d_cmask : nullptr;
   la.fresh = 0;
+  for (int k = 0; k < 3; k++) {
+    la.w[k] = e->grid.dim[k] / e->grid.nc[k];
+    la.magic[k] = (unsigned int)((1ull << 32) / (unsigned long long)e->grid.nc[k]);
+  }
   return la;
 }
 
@@ -331,6 +336,14 @@ GhostArgs ghost_args(const swsph_engine *e) {
   g.grad_rec = 0;
   g.force_rec = 0;
   return g;
+}
+
+// The ghost of the batched passes.
+GhostArgs batched_ghost_args(const swsph_engine *e) {
+  GhostArgs ga = ghost_args(e);
+  ga.fresh_grad = 1;  // the batched gradient loop starts its own sums
+  ga.grad_rec = 1;    // and reads the records the ghost writes
+  return ga;
 }
 
 void free_dev(swsph_engine *e) {
@@ -461,8 +474,7 @@ swsph_engine::ChunkTable *chunk_table(swsph_engine *e, int C, int *rc) {
         dalloc(&t.d_chunk_cell, nk) != hipSuccess ||
         dalloc(&t.d_bbox, 6 * nk) != hipSuccess ||
         dalloc(&t.d_hg2max, nk) != hipSuccess ||
-        ((C == kSparseChunk || C == kSparseSub) &&
-         dalloc(&t.d_fbox, 2 * nk) != hipSuccess)) {
+        dalloc(&t.d_fbox, 2 * nk) != hipSuccess) {
       *rc = fail(2, "allocation of chunk table failed");
       return nullptr;
     }
@@ -795,12 +807,19 @@ TileArgs tile_args(const swsph_engine *e) {
   return ta;
 }
 
+// The density tiles iterate the smoothing lengths themselves (sph_tile.h):
+// one launch instead of a round of ghost, tile build and density each.
+bool iterates(const swsph_engine *e) {
+  return e->schedule >= 1 && !e->use_lists &&
+         e->loop_c[(int)LoopKind::Density] == 16;
+}
+
 // A batched loop through the work queue: tiles of the particles selected by
 // `mode` (0 active, 1 active and flagged, 2 flagged without a usable
 // neighbour list), drained by persistent waves; `build` rebuilds the lists
 // of the selected particles while doing their density.
 int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
-               bool build) {
+               bool build, bool iter = false) {
   int rc = 0;
   const int C = build ? kListChunk : e->loop_c[(int)k];
   const int CJ = build ? kListChunk : e->loop_cj[(int)k];
@@ -836,6 +855,7 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
     HIPCHK(sphk::launch_build_tiles(e->d, la, (int)e->n, e->ncells, C, mode,
                                     flag, e->ts, e->st));
     e->tiles_c = mode == 0 ? C : 0;
+    e->tiles_n = -1;
   } else if (e->schedule == 2) {
     HIPCHK(sphk::launch_zero_u32((unsigned int *)e->ts.heads, 8 * 64, e->st));
   }
@@ -843,11 +863,17 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
   bool persistent = e->schedule == 2, rest = false;
   if (!e->capturing && e->schedule == 1) {
     // Eager: one wave per tile of the device-side count (a grid for the
-    // largest possible count would mostly be waves that exit at once).
-    HIPCHK(hipMemcpyAsync(e->h_ntiles, ta.ntiles, sizeof(int),
-                          hipMemcpyDeviceToHost, e->st));
-    HIPCHK(hipStreamSynchronize(e->st));
-    max_tiles = *e->h_ntiles;
+    // largest possible count would mostly be waves that exit at once), read
+    // once per table.
+    if (subset || e->tiles_n < 0) {
+      HIPCHK(hipMemcpyAsync(e->h_ntiles, ta.ntiles, sizeof(int),
+                            hipMemcpyDeviceToHost, e->st));
+      HIPCHK(hipStreamSynchronize(e->st));
+      if (!subset) e->tiles_n = *e->h_ntiles;
+      max_tiles = *e->h_ntiles;
+    } else {
+      max_tiles = e->tiles_n;
+    }
   } else if (e->capturing && e->schedule == 1) {
     // Captured: the all-active tiles are counted before the capture (the
     // count holds for every replay of this configuration), with a small
@@ -871,6 +897,11 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
     HIPCHK(sphk::launch_sparse(k, e->d, la, chunk_args(t1), chunk_args(t), ta,
                                persistent, e->queue_waves, max_tiles, rest,
                                e->st));
+  else if ((max_tiles > 0 || rest) && C == 16 && !build)
+    HIPCHK(sphk::launch_tile16(k, iter, e->d, la, chunk_args(t), ta,
+                               batched_ghost_args(e), e->props.max_iter,
+                               e->d_redo, persistent, e->queue_waves, max_tiles,
+                               rest, e->st));
   else if (max_tiles > 0 || rest)
     HIPCHK(sphk::launch_queue(k, build, e->d, la, chunk_args(t), ta, e->nl, C,
                               CJ, persistent, e->queue_waves, max_tiles, rest,
@@ -1482,6 +1513,13 @@ namespace {
 // hydro_init_part on the active particles and the first density round (with
 // lists: a fresh neighbour list for every active particle).
 int phase_start(swsph_engine *e) {
+  if (iterates(e)) {
+    // the tiles hold the ghost's brackets and flags in registers
+    HIPCHK(sphk::launch_zero_u64(e->d_redo, kGhostCounters, e->st));
+    e->launches++;
+    e->tiles_c = 0;  // activity may have changed since the last pass
+    return queue_loop(e, LoopKind::Density, 0, nullptr, false, true);
+  }
   HIPCHK(sphk::launch_init_density(e->d, 0, (int)e->n, e->props.max_active_bin,
                                    e->props.h_max, e->st, nullptr, nullptr,
                                    true));
@@ -1513,9 +1551,7 @@ const int *queue_list(const swsph_engine *e, const int **cnt) {
 int phase_ghost(swsph_engine *e) {
   const int *cnt;
   const int *list = queue_list(e, &cnt);
-  GhostArgs ga = ghost_args(e);
-  ga.fresh_grad = 1;  // the batched gradient loop starts its own sums
-  ga.grad_rec = 1;    // and reads the records the ghost writes
+  const GhostArgs ga = batched_ghost_args(e);
   HIPCHK(sphk::launch_ghost(e->d, ga, 0, (int)e->n, e->d_redo, e->st, list,
                             cnt));
   e->launches += 2;
@@ -1605,6 +1641,17 @@ int finish_stats(swsph_engine *e, swsph_pass_stats *stats, int rounds,
   return collect_timing(e);
 }
 
+// The end of a pass whose density tiles iterated: their counters are read
+// once the whole pass is enqueued.
+int finish_iterated(swsph_engine *e, swsph_pass_stats *stats, int64_t l0) {
+  int redo = 0;
+  if (int rc = read_redo(e, &redo)) return rc;
+  if (redo > 0)
+    return fail(3, "Smoothing length failed to converge on %d particles", redo);
+  e->last_rounds = std::max(1, (int)e->h_redo[kGhostRounds]);
+  return finish_stats(e, stats, e->last_rounds, l0);
+}
+
 // Captures the launches of fn on the engine stream into an executable graph.
 template <class F>
 int capture(swsph_engine *e, hipGraphExec_t *out, F fn) {
@@ -1691,6 +1738,10 @@ int pass_batched_locked(swsph_engine *e, swsph_pass_stats *stats) {
   if ((rc = ensure_records(e))) return rc;
   e->last_pass_mab = e->props.max_active_bin;
   if ((rc = phase_start(e))) return rc;
+  if (iterates(e)) {
+    if ((rc = phase_finish(e))) return rc;
+    return finish_iterated(e, stats, l0);
+  }
   int redo = 0, it = 0;
   for (; it < e->props.max_iter; it++) {
     if ((rc = phase_ghost(e))) return rc;
@@ -2760,9 +2811,11 @@ static int pass_graph_locked(swsph_engine *e, swsph_pass_stats *stats) {
   e->last_pass_mab = e->props.max_active_bin;
   // Re-runs captured: as many as the last pass needed.
   // (at most kHistRounds - 1: one redo count per captured ghost round)
-  const int reruns = std::min(
-      swsph_engine::kHistRounds - 1,
-      std::max(1, std::min(e->props.max_iter, e->last_rounds) - 1));
+  const int reruns =
+      iterates(e) ? 0
+                  : std::min(swsph_engine::kHistRounds - 1,
+                             std::max(1, std::min(e->props.max_iter,
+                                                  e->last_rounds) - 1));
   if (!e->g_density || e->graph_gen != e->gen || e->graph_reruns != reruns) {
     drop_graphs(e);
     // chunk tables must exist before capture (they allocate)
@@ -2793,6 +2846,14 @@ static int pass_graph_locked(swsph_engine *e, swsph_pass_stats *stats) {
                             hipMemcpyDeviceToDevice, e->st));
       return 0;
     };
+    if (iterates(e)) {
+      // no rounds to count: the pass is one graph
+      if ((rc = capture(e, &e->g_density, [&]() -> int {
+             const int r = phase_start(e);
+             return r ? r : phase_finish(e);
+           })))
+        return rc;
+    } else {
     if ((rc = capture(e, &e->g_density, [&]() -> int {
            int r = phase_start(e);
            for (int k = 0; k < reruns && !r; k++) {
@@ -2804,10 +2865,12 @@ static int pass_graph_locked(swsph_engine *e, swsph_pass_stats *stats) {
       return rc;
     if ((rc = capture(e, &e->g_finish, [&]() -> int { return phase_finish(e); })))
       return rc;
+    }
     e->graph_gen = e->gen;
     e->graph_reruns = reruns;
   }
   HIPCHK(hipGraphLaunch(e->g_density, e->st));
+  if (iterates(e)) return finish_iterated(e, stats, l0);
   HIPCHK(hipMemcpyAsync(e->h_hist, e->d_hist,
                         (reruns + 1) * sizeof(unsigned long long),
                         hipMemcpyDeviceToHost, e->st));

@@ -93,6 +93,24 @@ constexpr int kMasks = 2;
 // FP16 (two rows per instruction) when a chunk has an even number of rows.
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
+// The pre-test of the tiles of 16 runs on the matrix cores: one
+// v_mfma_f32_16x16x4_f32 forms 16 candidates x 16 i-particles as
+// |x_j|^2 - 2 x_i . x_j + (|x_i|^2 - R_i) in the tile frame (positions
+// relative to the centre of the i-box in units of the tile's largest search
+// radius).  Lane g + 16 s holds the results of particle g against candidates
+// 4 s .. 4 s + 3 of the product; the candidates enter permuted so that these
+// are the candidates of stream s (s, s + 4, s + 8, s + 12 of the 16).
+typedef float float4v __attribute__((ext_vector_type(4)));
+// Relative slack of the squares in the matrix pre-test: products, squares
+// and the accumulation each round a few times by 2^-24 of |x_i|^2 + |x_j|^2.
+constexpr float kSqLo = 1.f - 0x1p-18f;
+constexpr float kRadUp = 1.f + 0x1p-20f;
+// Rows of the staged candidates in LDS, 80 floats apart so that the four
+// components of 16 candidates lie in 64 different banks.
+constexpr int kTpRow = 80;
+constexpr int kTpRowJ = 4 * kTpRow + 48;
+constexpr int kTpLen = kTpRowJ + 64;
+
 // One wave per block in the batched kernels: each wave works on its own
 // chunk or tile with its own LDS (several waves per block measured slower on
 // the 128^3 box).
@@ -144,15 +162,29 @@ __host__ __device__ inline int xcd_blocks(int n) {
 // CI: i-particles per wave (S = 64 / CI candidate streams each); CJ:
 // particles per candidate chunk (CJ >= S: a row of S candidates lies in one
 // chunk).
+// Staging of the pre-test: candidate records, or paired FP16 positions.
+template <int CI>
+struct PretestLds {
+  PosRec lpos[64];
+  // FP16 pre-test: staged candidates in the tile frame, rows paired
+  _Float16 hx[64], hy[64], hz[64];
+};
+// Matrix pre-test: staged candidates in the tile frame, rows x, y, z,
+// |x|^2 and (force loop) |x|^2 - H_j^2, and the i side of the products (the
+// lanes' elements of B; |x_i|^2 - R_i and |x_i|^2 of the particles), read
+// back for every 64 candidates so that no register holds them over a walk.
+template <>
+struct PretestLds<16> {
+  float tp[kTpLen];
+  float mb[64], mc[16], msq[16];
+};
+
 template <int CI, int CJ>
-struct GatherLds {
+struct GatherLds : PretestLds<CI> {
   static constexpr int S = 64 / CI;
   static_assert(CJ >= S && CJ <= 64, "a row must lie in one chunk");
   static constexpr int RPC = CJ / S;        // rows per chunk
   static constexpr int SLOTS = 64 * kMasks / RPC;  // chunks per phase
-  PosRec lpos[64];
-  // FP16 pre-test: staged candidates in the tile frame, rows paired
-  _Float16 hx[64], hy[64], hz[64];
   float qoffc[27 * 3];  // neighbour image corners relative to the tile centre
   double ttab[27 * 3];
   double qorg[27 * 3];  // corner of each neighbour's image
@@ -173,8 +205,9 @@ __device__ __forceinline__ void interact_rows(
     const typename L::Rec *__restrict__ rec, const GatherLds<CI, CJ> &sh,
     const typename L::I &st, int s, unsigned long long m0,
     unsigned long long m1, typename L::Acc &acc, const NbrList &nl, int i,
-    float rt2, int &ncnt, unsigned int selfm) {
+    float rt2, int &ncnt, unsigned int selfm, int ic) {
   constexpr int S = GatherLds<CI, CJ>::S, RPC = GatherLds<CI, CJ>::RPC;
+  constexpr bool kMfma = CI == 16;
   // next row of this lane (ascending), taken out of the masks
   auto pop = [&]() -> int {
     const bool lo = m0 != 0ull;
@@ -234,6 +267,8 @@ __device__ __forceinline__ void interact_rows(
   while (any()) {
     int q;
     const int j = locate(pop(), q);
+    // the matrix pre-test passes the particle itself
+    if (kMfma && j == ic) continue;
     eval(j, q, rec[j]);
   }
 }
@@ -398,7 +433,8 @@ __device__ __forceinline__ void run_chunk(
   // rejects a neighbour of the pair contract.
   // (the force loop's symmetric test needs a widened radius per candidate
   // as well, which costs more than the packed rows save: it stays FP32)
-  constexpr bool kF16 = (RPC % 2 == 0) && !L::kSymmetric;
+  constexpr bool kMfma = CI == 16;
+  constexpr bool kF16 = !kMfma && (RPC % 2 == 0) && !L::kSymmetric;
   constexpr float kU16 = 1.f / 2048.f;
   float invR = 0.f, eps16 = 0.f;
   _Float16 ixh = 0, iyh = 0, izh = 0, rt2h = -1;
@@ -424,6 +460,38 @@ __device__ __forceinline__ void run_chunk(
     const float r = sqrtf(rt2 * invR * invR) + 2.f * eps16;
     const float b = r * r * (1.f + 8.f * kU16) * (1.f + 1.f / 1024.f);
     rt2h = act ? (_Float16)fminf(b, 65504.f) : (_Float16)(-1.f);
+  }
+  // Matrix pre-test frame: the i side of the products.  With the positions
+  // rounded to float in this frame as real numbers, the computed value lies
+  // within a few 2^-24 (|x_i| + |x_j|)^2 of r^2 - R; the squares are taken
+  // 2^-18 low and the radii 2^-20 high, so that r^2 < R always gives a
+  // negative value (rt2m carries the error of the positions themselves).
+  float invR2 = 0.f;
+  if constexpr (kMfma) {
+    const double cx = 0.5 * (ilx + ihx), cy = 0.5 * (ily + ihy),
+                 cz = 0.5 * (ilz + ihz);
+    invR = hg2i > 0.f ? 1.f / sqrtf(hg2i) : 1.f;
+    invR2 = invR * invR * kRadUp;
+    if (lane < nq) {
+      sh.qoffc[3 * lane] = (float)(sh.qorg[3 * lane] - cx);
+      sh.qoffc[3 * lane + 1] = (float)(sh.qorg[3 * lane + 1] - cy);
+      sh.qoffc[3 * lane + 2] = (float)(sh.qorg[3 * lane + 2] - cz);
+    }
+    float mb = 0.f, ci = 1.f, sq = 1.f;
+    if (act) {
+      const float fx = (float)(st.x - cx) * invR;
+      const float fy = (float)(st.y - cy) * invR;
+      const float fz = (float)(st.z - cz) * invR;
+      sq = fmaf(fz, fz, fmaf(fy, fy, fx * fx)) * kSqLo;
+      mb = s == 0 ? fx : (s == 1 ? fy : fz);
+      mb = s == 3 ? 1.f : -2.f * mb;
+      ci = fmaf(-rt2m * kRadUp, invR2, sq);
+    }
+    sh.mb[lane] = mb;
+    if (s == 0) {
+      sh.mc[g] = ci;
+      sh.msq[g] = sq;
+    }
   }
   wave_sync();
   // pair-contract frames of the neighbours (from the table in LDS)
@@ -481,101 +549,168 @@ __device__ __forceinline__ void run_chunk(
     if (pass) sh.plist[__popcll(pm & ((1ull << lane) - 1ull))] = pe;
     wave_sync();
     for (int pb = 0; pb < np; pb += G) {
-      // Stage the candidates of up to G surviving chunks.
-      {
+      if constexpr (kMfma) {
+        // Stage up to G surviving chunks: 64 candidates, 16 rows.
         const int c = lane / CJ;
+        float vx = 1e15f, vy = 0.f, vz = 0.f, sq = 1e30f, sqj = 1e30f;
         if (pb + c < np) {
           const unsigned int e = sh.plist[pb + c];
           const int q = (int)(e >> 27);
-          const int j = sh.qj0[q] + (int)(e & kRowMask) * CJ + lane % CJ;
-          PosRec p;
-          if (j < sh.qj1[q]) {
-            p = pos[j];
-          } else {  // past the end of a short chunk: never passes
-            p.x = p.y = p.z = -1e30f;
-            p.hg2m = -1.f;
-          }
-          if (kF16) {
-            // slot of row pair (rr / 2) of stream sp, lane rr % 2 of the pair
-            const int jl = lane % CJ, rr = jl / S, sp = jl % S;
-            const int dst = ((c * (RPC / 2) + (rr >> 1)) * S + sp) * 2 + (rr & 1);
-            sh.hx[dst] = (_Float16)((p.x + sh.qoffc[3 * q]) * invR);
-            sh.hy[dst] = (_Float16)((p.y + sh.qoffc[3 * q + 1]) * invR);
-            sh.hz[dst] = (_Float16)((p.z + sh.qoffc[3 * q + 2]) * invR);
-          } else {
-            sh.lpos[lane] = p;
+          const int js = sh.qj0[q] + (int)(e & kRowMask) * CJ;
+          const int j = js + lane % CJ;
+          if (lane % CJ == 0)
+            sh.cinfo[nrow / RPC + c] = ((unsigned int)q << 27) | (unsigned int)js;
+          if (j < sh.qj1[q]) {  // (past the end of a short chunk: far away)
+            const PosRec p = pos[j];
+            vx = (p.x + sh.qoffc[3 * q]) * invR;
+            vy = (p.y + sh.qoffc[3 * q + 1]) * invR;
+            vz = (p.z + sh.qoffc[3 * q + 2]) * invR;
+            sq = fmaf(vz, vz, fmaf(vy, vy, vx * vx)) * kSqLo;
+            if (L::kSymmetric) sqj = fmaf(-p.hg2m * kRadUp, invR2, sq);
           }
         }
-      }
-      wave_sync();
-      for (int c = 0; c < G; c++) {
-        if (pb + c >= np) break;  // uniform
-        const unsigned int e = (unsigned int)uniform((int)sh.plist[pb + c]);
-        const int q = (int)(e >> 27);
-        const int js = uniform(sh.qj0[q]) + (int)(e & kRowMask) * CJ;
-        const int nj = min(CJ, uniform(sh.qj1[q]) - js);
-        // chunk slot of the lane's own particle (a particle is not its own
-        // neighbour); out of the chunk's range unless the chunk holds it
-        const int selfl = uniform(sh.qcell[q]) == cell_i ? ic - js : -1;
-        // i relative to the neighbour image's corner
-        const float xs = (float)(st.x - sh.qorg[3 * q]);
-        const float ys = (float)(st.y - sh.qorg[3 * q + 1]);
-        const float zs = (float)(st.z - sh.qorg[3 * q + 2]);
-        if (lane == 0)
-          sh.cinfo[nrow / RPC] = ((unsigned int)q << 27) | (unsigned int)js;
-        // hits of this chunk's rows, bit rr for row rr
-        using Nib = typename std::conditional<(RPC > 32), unsigned long long,
-                                              unsigned int>::type;
-        Nib nib = 0;
-        if (kF16) {
-          const half2v ix2 = {ixh, ixh}, iy2 = {iyh, iyh}, iz2 = {izh, izh};
+        sh.tp[lane] = vx;
+        sh.tp[kTpRow + lane] = vy;
+        sh.tp[2 * kTpRow + lane] = vz;
+        sh.tp[3 * kTpRow + lane] = sq;
+        if (L::kSymmetric) sh.tp[kTpRowJ + lane] = sqj;
+        wave_sync();
+        // candidate (row of A) of this lane and its component
+        const int m = (lane & 3) * 4 + ((lane >> 2) & 3);
+        const int t1 = s * kTpRow + m;
+        const int t2 = s == 3 ? kTpRowJ + m : t1;
+        const float mb = sh.mb[lane], ci = sh.mc[g];
+        const float4v mc = {ci, ci, ci, ci};
+        const float cj = L::kSymmetric ? sh.msq[g] : 0.f;
+        const float4v mc2 = {cj, cj, cj, cj};
+        unsigned int w = 0u;  // row 0 in the highest of 16 bits
 #pragma unroll
-          for (int pr = 0; pr < RPC / 2; pr++) {
-            if (2 * pr * S >= nj) break;  // uniform
-            const int idx = 2 * ((c * (RPC / 2) + pr) * S + s);
-            const half2v x2 = *reinterpret_cast<const half2v *>(&sh.hx[idx]);
-            const half2v y2 = *reinterpret_cast<const half2v *>(&sh.hy[idx]);
-            const half2v z2 = *reinterpret_cast<const half2v *>(&sh.hz[idx]);
-            const half2v dx = ix2 - x2, dy = iy2 - y2, dz = iz2 - z2;
-            const half2v r2 = dz * dz + (dy * dy + dx * dx);
-            const bool p0 = r2.x < rt2h, p1 = r2.y < rt2h;
-            const int jl0 = 2 * pr * S + s, jl1 = jl0 + S;
-            nib |= (p0 && jl0 != selfl) ? ((Nib)1 << (2 * pr)) : (Nib)0;
-            nib |= (p1 && jl1 != selfl) ? ((Nib)1 << (2 * pr + 1)) : (Nib)0;
-          }
-        } else {
+        for (int b = 0; b < 4; b++) {
+          float4v dd = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              sh.tp[t1 + 16 * b], mb, mc, 0, 0, 0);
+          if (L::kSymmetric) {
+            const float4v d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                sh.tp[t2 + 16 * b], mb, mc2, 0, 0, 0);
 #pragma unroll
-          for (int rr = 0; rr < RPC; rr++) {
-            if (rr * S >= nj) break;  // uniform
-            const int jl = rr * S + s;
-            const PosRec p = sh.lpos[c * CJ + jl];
-            const float dx = xs - p.x, dy = ys - p.y, dz = zs - p.z;
-            const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-            const bool pass =
-                L::kSymmetric ? (r2 < rt2m || r2 < p.hg2m) : r2 < rt2m;
-            nib |= (pass && jl != selfl) ? ((Nib)1 << rr) : (Nib)0;
+            for (int r = 0; r < 4; r++)
+              dd[r] = __uint_as_float(__float_as_uint(dd[r]) |
+                                      __float_as_uint(d2[r]));
           }
+#pragma unroll
+          for (int r = 0; r < 4; r++)  // append the sign
+            w = __builtin_amdgcn_alignbit(w, __float_as_uint(dd[r]), 31);
         }
+        w = __builtin_bitreverse32(w) >> 16;
         if (nrow < 64)  // uniform
-          m0 |= (unsigned long long)nib << nrow;
+          m0 |= (unsigned long long)w << nrow;
         else
-          m1 |= (unsigned long long)nib << (nrow - 64);
-        nrow += RPC;
+          m1 |= (unsigned long long)w << (nrow - 64);
+        nrow += 16;
         if (nrow == 64 * kMasks) {
           wave_sync();
           interact_rows<L, CI, CJ, BUILD>(rec, sh, st, s, m0, m1, acc, nl, i,
-                                          rt2, ncnt, selfm);
+                                          rt2, ncnt, selfm, ic);
           m0 = m1 = 0ull;
           nrow = 0;
         }
+        wave_sync();
+      } else {
+        // Stage the candidates of up to G surviving chunks.
+        {
+          const int c = lane / CJ;
+          if (pb + c < np) {
+            const unsigned int e = sh.plist[pb + c];
+            const int q = (int)(e >> 27);
+            const int j = sh.qj0[q] + (int)(e & kRowMask) * CJ + lane % CJ;
+            PosRec p;
+            if (j < sh.qj1[q]) {
+              p = pos[j];
+            } else {  // past the end of a short chunk: never passes
+              p.x = p.y = p.z = -1e30f;
+              p.hg2m = -1.f;
+            }
+            if (kF16) {
+              // slot of row pair (rr / 2) of stream sp, lane rr % 2 of the pair
+              const int jl = lane % CJ, rr = jl / S, sp = jl % S;
+              const int dst = ((c * (RPC / 2) + (rr >> 1)) * S + sp) * 2 + (rr & 1);
+              sh.hx[dst] = (_Float16)((p.x + sh.qoffc[3 * q]) * invR);
+              sh.hy[dst] = (_Float16)((p.y + sh.qoffc[3 * q + 1]) * invR);
+              sh.hz[dst] = (_Float16)((p.z + sh.qoffc[3 * q + 2]) * invR);
+            } else {
+              sh.lpos[lane] = p;
+            }
+          }
+        }
+        wave_sync();
+        for (int c = 0; c < G; c++) {
+          if (pb + c >= np) break;  // uniform
+          const unsigned int e = (unsigned int)uniform((int)sh.plist[pb + c]);
+          const int q = (int)(e >> 27);
+          const int js = uniform(sh.qj0[q]) + (int)(e & kRowMask) * CJ;
+          const int nj = min(CJ, uniform(sh.qj1[q]) - js);
+          // chunk slot of the lane's own particle (a particle is not its own
+          // neighbour); out of the chunk's range unless the chunk holds it
+          const int selfl = uniform(sh.qcell[q]) == cell_i ? ic - js : -1;
+          // i relative to the neighbour image's corner
+          const float xs = (float)(st.x - sh.qorg[3 * q]);
+          const float ys = (float)(st.y - sh.qorg[3 * q + 1]);
+          const float zs = (float)(st.z - sh.qorg[3 * q + 2]);
+          if (lane == 0)
+            sh.cinfo[nrow / RPC] = ((unsigned int)q << 27) | (unsigned int)js;
+          // hits of this chunk's rows, bit rr for row rr
+          using Nib = typename std::conditional<(RPC > 32), unsigned long long,
+                                                unsigned int>::type;
+          Nib nib = 0;
+          if (kF16) {
+            const half2v ix2 = {ixh, ixh}, iy2 = {iyh, iyh}, iz2 = {izh, izh};
+  #pragma unroll
+            for (int pr = 0; pr < RPC / 2; pr++) {
+              if (2 * pr * S >= nj) break;  // uniform
+              const int idx = 2 * ((c * (RPC / 2) + pr) * S + s);
+              const half2v x2 = *reinterpret_cast<const half2v *>(&sh.hx[idx]);
+              const half2v y2 = *reinterpret_cast<const half2v *>(&sh.hy[idx]);
+              const half2v z2 = *reinterpret_cast<const half2v *>(&sh.hz[idx]);
+              const half2v dx = ix2 - x2, dy = iy2 - y2, dz = iz2 - z2;
+              const half2v r2 = dz * dz + (dy * dy + dx * dx);
+              const bool p0 = r2.x < rt2h, p1 = r2.y < rt2h;
+              const int jl0 = 2 * pr * S + s, jl1 = jl0 + S;
+              nib |= (p0 && jl0 != selfl) ? ((Nib)1 << (2 * pr)) : (Nib)0;
+              nib |= (p1 && jl1 != selfl) ? ((Nib)1 << (2 * pr + 1)) : (Nib)0;
+            }
+          } else {
+  #pragma unroll
+            for (int rr = 0; rr < RPC; rr++) {
+              if (rr * S >= nj) break;  // uniform
+              const int jl = rr * S + s;
+              const PosRec p = sh.lpos[c * CJ + jl];
+              const float dx = xs - p.x, dy = ys - p.y, dz = zs - p.z;
+              const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+              const bool pass =
+                  L::kSymmetric ? (r2 < rt2m || r2 < p.hg2m) : r2 < rt2m;
+              nib |= (pass && jl != selfl) ? ((Nib)1 << rr) : (Nib)0;
+            }
+          }
+          if (nrow < 64)  // uniform
+            m0 |= (unsigned long long)nib << nrow;
+          else
+            m1 |= (unsigned long long)nib << (nrow - 64);
+          nrow += RPC;
+          if (nrow == 64 * kMasks) {
+            wave_sync();
+            interact_rows<L, CI, CJ, BUILD>(rec, sh, st, s, m0, m1, acc, nl, i,
+                                            rt2, ncnt, selfm, ic);
+            m0 = m1 = 0ull;
+            nrow = 0;
+          }
+        }
+        wave_sync();
       }
-      wave_sync();
     }
   }
   if (nrow > 0) {
     wave_sync();
     interact_rows<L, CI, CJ, BUILD>(rec, sh, st, s, m0, m1, acc, nl, i, rt2,
-                                    ncnt, selfm);
+                                    ncnt, selfm, ic);
   }
   L::template combine<S>(acc);
   if (act && s == 0) L::store_acc(d, i, acc);
@@ -645,11 +780,8 @@ __global__ __launch_bounds__(64) void k_loop_task(
 // its own is exhausted; every queue is visited at most once after it runs
 // dry, so every wave exits.
 constexpr int kGrab = 2;
-template <class L, int CI, int CJ, bool BUILD>
-__global__ __launch_bounds__(64, kOccSparseQueue) void k_loop_queue(
-    DevParts d, LoopArgs la, ChunkArgs ca,
-    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
-    NbrList nl, TileArgs tq) {
+template <class F>
+__device__ __forceinline__ void drain_queue(const TileArgs &tq, F run) {
   const int nt = *tq.ntiles;
   const int per = (nt + 7) >> 3;
   int q = blockIdx.x & 7;
@@ -675,12 +807,20 @@ __global__ __launch_bounds__(64, kOccSparseQueue) void k_loop_queue(
       continue;
     }
     const int end = min(hi, lo + kGrab);
-    for (int t = lo; t < end; t++) {
-      wave_sync();
-      run_chunk<L, CI, CJ, false, BUILD, true>(d, la, ca, rec, pos, 0, true, 0,
-                                               0.0, 0.0, 0.0, nl, &tq, t);
-    }
+    for (int t = lo; t < end; t++) run(t);
   }
+}
+
+template <class L, int CI, int CJ, bool BUILD>
+__global__ __launch_bounds__(64, kOccSparseQueue) void k_loop_queue(
+    DevParts d, LoopArgs la, ChunkArgs ca,
+    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
+    NbrList nl, TileArgs tq) {
+  drain_queue(tq, [&](int t) {
+    wave_sync();
+    run_chunk<L, CI, CJ, false, BUILD, true>(d, la, ca, rec, pos, 0, true, 0,
+                                             0.0, 0.0, 0.0, nl, &tq, t);
+  });
 }
 
 // Grid form of the tile queue: one wave per tile over a grid sized for the

@@ -53,7 +53,7 @@ struct ChunkArgs {
   const float *hg2max;      // [nchunks] max (gamma_K h)^2
   // [2 nchunks] the box of the chunk's pre-test records (PosRec x, y, z
   // relative to the cell corner) with their largest widened radius in the
-  // first .w, or null (tables the sparse tiles do not read)
+  // first .w (read by the tiles of 16 and the sparse tiles)
   const float4 *fbox;
   int nchunks;
   int C;                    // chunk capacity (8, 16, 32 or 64)
@@ -147,9 +147,12 @@ constexpr int kListChunk = 64 / kListStreams;
 // tile tables are sized for it.
 constexpr int kMinTile = 4;
 // Slots of the ghost's density-work counter (launch_ghost): the counter
-// block holds 3 + kGhostWorkSlots 64-bit counters.
+// block holds kGhostCounters 64-bit counters.
 constexpr int kGhostWorkSlots = 32;
-constexpr int kGhostCounters = 3 + kGhostWorkSlots;
+// One more slot holds the largest number of density evaluations of a
+// particle when the density tiles iterate (sph_tile.h).
+constexpr int kGhostRounds = 3 + kGhostWorkSlots;
+constexpr int kGhostCounters = kGhostRounds + 1;
 // Sparse tiles (sph_sparse.h): tiles of kMinTile particles, candidates
 // culled by the chunks of kSparseChunk, then by their sub-chunks of
 // kSparseSub against each particle.
@@ -188,6 +191,10 @@ struct LoopArgs {
   // (L::fresh_acc) and are stored, not loaded (the batched loops; their
   // resets are skipped).
   int fresh;
+  // The grid's cell widths (dim / nc), and floor(2^32 / nc) of its axes
+  // (cell coordinates without an integer division).
+  double w[3];
+  unsigned int magic[3];
 };
 
 // Up to two directed cell interactions (i-cell gathers from j-cell, the
@@ -313,6 +320,16 @@ hipError_t launch_queue(LoopKind kind, bool build_lists, const DevParts &d,
                         const TileArgs &ta, const NbrList &nl, int CI, int CJ,
                         bool persistent, int waves, int max_tiles, bool rest,
                         hipStream_t st);
+// The tiles of 16 particles (sph_tile.h) against chunks of ca.C = 8, 16 or
+// 32; grids as launch_queue.  `iter` (density only): the tiles iterate the
+// smoothing lengths to convergence and finish their particles as the ghost
+// does with ga; counters as launch_ghost's plus [kGhostRounds], all zeroed
+// by the caller.
+hipError_t launch_tile16(LoopKind kind, bool iter, const DevParts &d,
+                         const LoopArgs &la, const ChunkArgs &ca,
+                         const TileArgs &ta, const GhostArgs &ga, int max_iter,
+                         unsigned long long *counters, bool persistent,
+                         int waves, int max_tiles, bool rest, hipStream_t st);
 // The tiles of the table in `ts` that hold a particle with filt[i] != 0,
 // appended to ids (in no fixed order: each tile's sums are its own) with
 // their count in *nids.

@@ -14,8 +14,10 @@
 #include "sph_device.h"
 #include "sph_kernels.h"
 #include "sph_loops.h"
+#include "sph_ghost.h"
 #include "sph_gather.h"
 #include "sph_sparse.h"
+#include "sph_tile.h"
 
 using namespace sph;
 using namespace sphl;
@@ -299,150 +301,38 @@ __global__ void k_init_density(DevParts d, int lo, int hi, int max_active_bin,
     for_runs(lo, hi, d.tb, body);
 }
 
-// hydro_prepare_gradient + hydro_reset_gradient (hydro.h:671-750) on a
-// particle whose density sums are final.
-__device__ void prepare_gradient(const DevParts &d, int i, float h, float rho,
-                                 float rho_dh, float wc, float wc_dh,
-                                 float divv, float rx, float ry, float rz,
-                                 const GhostArgs &ga) {
-  const float curl_v = sqrtf(rx * rx + ry * ry + rz * rz);
-  const float abs_div_v = fabsf(divv);
-  const float u = d.u[i];
-  const float P = kGasGm1 * u * rho;
-  const float c = sqrtf(kGasGamma * P / rho);
-  const float bal = abs_div_v / (abs_div_v + curl_v + 0.0001f * c / h);
-  const float common = h * kDimInv / wc;
-  float fgh;
-  if (h > 0.9999f * ga.h_max) {
-    fgh = 0.f;
-  } else {
-    const float gW = common * wc_dh;
-    fgh = (gW < -0.9999f) ? 0.f : common * rho_dh / (1.f + gW);
-  }
-  d.P[i] = P;
-  d.c[i] = c;
-  d.f[i] = fgh;
-  d.bal[i] = bal;
-  const float alpha = d.alpha[i];
-  // the gradient record, built here from the values at hand
-  if (ga.grad_rec) d.rg[rec_slot(d, i)] = grad_rec_of(d, i, rho, u, c, alpha);
-  if (ga.fresh_grad) return;  // the gradient loop starts from these itself
-  d.vsig[i] = 2.f * c;
-  d.avmax[i] = alpha;
-  d.lapu[i] = 0.f;
-  d.ng[i] = 0;
-}
-
 // One ghost round (runner_do_ghost, runner_ghost.c:1113-1628) for the
-// particles flagged in redo[] within [lo, hi): hydro_end_density, one
-// Newton-Raphson / bisection step on h, and either convergence (prepare the
-// gradient loop) or a re-initialised particle flagged for another density
-// round.  `relist` tells whether the particle's neighbour list no longer
-// covers its new search radius (for another round, or for the gradient
-// loop once converged).
+// particles flagged in redo[] within [lo, hi): ghost_step on the density
+// sums, and either convergence (prepare the gradient loop) or a
+// re-initialised particle flagged for another density round.  `relist`
+// tells whether the particle's neighbour list no longer covers its new
+// search radius (for another round, or for the gradient loop once
+// converged).
 __device__ bool ghost_one(const DevParts &d, const GhostArgs &ga, int i,
                           bool &relist) {
-  const float h_old = d.h[i];
-  const float h_old_dim = h_old * h_old * h_old;
-  const float h_old_dim_m1 = h_old * h_old;
-  float rho = d.rho[i], rho_dh = d.rho_dh[i], wc = d.wc[i], wc_dh = d.wc_dh[i];
-  float divv = d.divv[i], rx = d.rotx[i], ry = d.roty[i], rz = d.rotz[i];
-  float left = d.left[i], right = d.right[i];
-  float h_new;
-  bool no_ngb = false;
-  bool done = false;
-  if ((double)wc < 1.e-5 * (double)kRoot) {
-    no_ngb = true;
-    h_new = 2.f * h_old;
-  } else {
-    // hydro_end_density (hydro.h:613-662), a = 1, H = 0
-    const float h_inv = 1.0f / h_old;
-    const float hid = h_inv * h_inv * h_inv;
-    const float hid1 = hid * h_inv;
-    const float mi = d.m[i];
-    rho = (rho + mi * kRoot) * hid;
-    rho_dh = (rho_dh - kDim * mi * kRoot) * hid1;
-    wc = (wc + kRoot) * hid;
-    wc_dh = (wc_dh - kDim * kRoot) * hid1;
-    const float rho_inv = 1.f / rho;
-    rx *= hid1 * rho_inv;
-    ry *= hid1 * rho_inv;
-    rz *= hid1 * rho_inv;
-    divv *= hid1 * rho_inv;
-    const float n_sum = wc * h_old_dim;
-    const float f = n_sum - ga.eta_dim;
-    const float f_prime = wc_dh * h_old_dim + kDim * wc * h_old_dim_m1;
-    if (n_sum < ga.eta_dim)
-      left = fmaxf(left, h_old);
-    else if (n_sum > ga.eta_dim)
-      right = fminf(right, h_old);
-    if (((h_old >= ga.h_max) && (f < 0.f)) ||
-        ((h_old <= ga.h_min) && (f > 0.f))) {
-      done = true;
-      h_new = h_old;
-    } else {
-      h_new = h_old - f / (f_prime + 1.17549435e-38f);
-      h_new = fminf(h_new, 2.f * h_old);
-      h_new = fmaxf(h_new, 0.5f * h_old);
-      h_new = fmaxf(h_new, left);
-      h_new = fminf(h_new, right);
-    }
+  GhostState g{d.h[i], d.left[i], d.right[i]};
+  DensSums a{d.rho[i], d.rho_dh[i], d.wc[i], d.wc_dh[i],
+             d.divv[i], d.rotx[i], d.roty[i], d.rotz[i]};
+  const bool again = ghost_step(ga, d.m[i], g, a);
+  relist = !ga.lists || !(search_radius2(g.h) <= d.r2b[i]);
+  if (again) {
+    // Not converged: re-initialise (hydro_init_part) and ask for a rerun.
+    d.h[i] = g.h;
+    d.left[i] = g.left;
+    d.right[i] = g.right;
+    d.rho[i] = 0.f;
+    d.rho_dh[i] = 0.f;
+    d.wc[i] = 0.f;
+    d.wc_dh[i] = 0.f;
+    d.divv[i] = 0.f;
+    d.rotx[i] = 0.f;
+    d.roty[i] = 0.f;
+    d.rotz[i] = 0.f;
+    d.nd[i] = 0;
+    return true;
   }
-  float h_fin = h_old;
-  if (!done && fabsf(h_new - h_old) > ga.eps * h_old) {
-    float hn;
-    if ((h_new == left && h_old == right) || (h_old == left && h_new == right))
-      hn = cbrtf(0.5f * (left * left * left + right * right * right));
-    else
-      hn = h_new;
-    if (hn < ga.h_max && hn > ga.h_min) {
-      // Not converged: re-initialise (hydro_init_part) and ask for a rerun.
-      d.h[i] = hn;
-      d.left[i] = left;
-      d.right[i] = right;
-      d.rho[i] = 0.f;
-      d.rho_dh[i] = 0.f;
-      d.wc[i] = 0.f;
-      d.wc_dh[i] = 0.f;
-      d.divv[i] = 0.f;
-      d.rotx[i] = 0.f;
-      d.roty[i] = 0.f;
-      d.rotz[i] = 0.f;
-      d.nd[i] = 0;
-      relist = !ga.lists || !(search_radius2(hn) <= d.r2b[i]);
-      return true;
-    }
-    if (hn <= ga.h_min) {
-      h_fin = ga.h_min;
-    } else {
-      h_fin = ga.h_max;
-      if (no_ngb) {
-        // hydro_part_has_no_neighbours (hydro.h:791-825)
-        const float hinv = 1.0f / h_fin;
-        const float hid = hinv * hinv * hinv;
-        rho = d.m[i] * kRoot * hid;
-        wc = kRoot * hid;
-        rho_dh = 0.f;
-        wc_dh = 0.f;
-        rx = ry = rz = 0.f;
-        divv = 0.f;
-      }
-    }
-  }
-  // Converged.
-  d.h[i] = h_fin;
-  d.redo[i] = 0;
-  relist = !ga.lists || !(search_radius2(h_fin) <= d.r2b[i]);
   if (ga.lists) d.lfb[i] = relist ? 1 : 0;
-  d.rho[i] = rho;
-  d.rho_dh[i] = rho_dh;
-  d.wc[i] = wc;
-  d.wc_dh[i] = wc_dh;
-  d.divv[i] = divv;
-  d.rotx[i] = rx;
-  d.roty[i] = ry;
-  d.rotz[i] = rz;
-  prepare_gradient(d, i, h_fin, rho, rho_dh, wc, wc_dh, divv, rx, ry, rz, ga);
+  ghost_finish(d, ga, i, g.h, a);
   return false;
 }
 
@@ -1113,9 +1003,9 @@ hipError_t queue_c(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
   return hipGetLastError();
 }
 
-// Tile (CI) x chunk (CJ) shapes with kernels: CJ = CI, CJ = CI / 2 for
-// CI = 16, 32 (finer candidate chunks under the same tile), and the narrow
-// tiles (4, 16), (4, 32), (8, 16) for sparse activity (a few active particles
+// Tile (CI) x chunk (CJ) shapes with kernels of the chunk engine: CJ = CI,
+// CJ = CI / 2 for CI = 32 (finer candidate chunks under the same tile; the
+// tiles of 16 have their own kernels, launch_tile16), and the narrow tiles (4, 16), (4, 32), (8, 16) for sparse activity (a few active particles
 // per cell: more candidate streams per particle, fewer idle lanes).
 template <class L>
 hipError_t queue_any(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
@@ -1124,15 +1014,12 @@ hipError_t queue_any(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
                      int waves, int mt, bool rest, hipStream_t st) {
   switch (CI * 100 + CJ) {
     case 808: return queue_c<L, 8, 8, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
-    case 1616: return queue_c<L, 16, 16, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
-    case 1608: return queue_c<L, 16, 8, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
     case 3232: return queue_c<L, 32, 32, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
     case 3216: return queue_c<L, 32, 16, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
     case 6464: return queue_c<L, 64, 64, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
     case 416: return queue_c<L, 4, 16, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
     case 432: return queue_c<L, 4, 32, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
     case 816: return queue_c<L, 8, 16, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
-    case 1632: return queue_c<L, 16, 32, false>(d, la, ca, ta, nl, rec, p, waves, mt, rest, st);
   }
   return hipErrorInvalidValue;
 }
@@ -1161,6 +1048,86 @@ hipError_t launch_queue(LoopKind kind, bool build_lists, const DevParts &d,
       return queue_any<ForceLoop>(d, la, ca, ta, nl, d.rf, CI, CJ,
                                   persistent, waves, max_tiles, rest,
                                     st);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <class L, int CJ, bool ITER>
+static int tile16_resident_blocks() {
+  static std::atomic<int> cached{0};
+  if (cached.load() == 0) {
+    int dev = 0, ncu = 0, per = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount,
+                              dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per, k_tile16_queue<L, CJ, ITER>, 64, 0) != hipSuccess ||
+        per <= 0)
+      return 0;
+    cached.store(ncu * per);
+  }
+  return cached.load();
+}
+
+template <class L, int CJ, bool ITER>
+hipError_t tile16_c(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
+                    const TileArgs &ta, const TileGhost &tg,
+                    const typename L::Rec *rec, bool persistent, int waves,
+                    int max_tiles, bool rest, hipStream_t st) {
+  const PosRec *pos = (const PosRec *)d.pos;
+  if (!persistent) {
+    const int nb = max_tiles > 0 ? xcd_blocks(max_tiles) : 0;
+    if (nb > 0)
+      hipLaunchKernelGGL((k_tile16<L, CJ, ITER>), dim3(nb), dim3(64), 0, st, d,
+                         la, ca, rec, pos, ta, tg);
+    if (rest)
+      hipLaunchKernelGGL((k_tile16_rest<L, CJ, ITER>), dim3(kRestBlocks),
+                         dim3(64), 0, st, d, la, ca, rec, pos, ta, tg, nb);
+    return hipGetLastError();
+  }
+  if (waves <= 0) waves = tile16_resident_blocks<L, CJ, ITER>();
+  if (waves <= 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_tile16_queue<L, CJ, ITER>), dim3(waves), dim3(64), 0,
+                     st, d, la, ca, rec, pos, ta, tg);
+  return hipGetLastError();
+}
+
+template <class L, bool ITER>
+hipError_t tile16_any(const DevParts &d, const LoopArgs &la,
+                      const ChunkArgs &ca, const TileArgs &ta,
+                      const TileGhost &tg, const typename L::Rec *rec, bool p,
+                      int waves, int mt, bool rest, hipStream_t st) {
+  switch (ca.C) {
+    case 8: return tile16_c<L, 8, ITER>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
+    case 16: return tile16_c<L, 16, ITER>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
+    case 32: return tile16_c<L, 32, ITER>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_tile16(LoopKind kind, bool iter, const DevParts &d,
+                         const LoopArgs &la, const ChunkArgs &ca,
+                         const TileArgs &ta, const GhostArgs &ga, int max_iter,
+                         unsigned long long *counters, bool persistent,
+                         int waves, int max_tiles, bool rest, hipStream_t st) {
+  if (!ca.fbox || !la.fresh || ta.ids || ta.filt) return hipErrorInvalidValue;
+  const TileGhost tg{ga, max_iter, counters,
+                     (unsigned int *)(counters + kGhostRounds)};
+  switch (kind) {
+    case LoopKind::Density:
+      return iter ? tile16_any<DensityLoop, true>(d, la, ca, ta, tg, d.rd,
+                                                  persistent, waves, max_tiles,
+                                                  rest, st)
+                  : tile16_any<DensityLoop, false>(d, la, ca, ta, tg, d.rd,
+                                                   persistent, waves,
+                                                   max_tiles, rest, st);
+    case LoopKind::Gradient:
+      return tile16_any<GradientLoop, false>(d, la, ca, ta, tg, d.rg,
+                                             persistent, waves, max_tiles,
+                                             rest, st);
+    case LoopKind::Force:
+      return tile16_any<ForceLoop, false>(d, la, ca, ta, tg, d.rf, persistent,
+                                          waves, max_tiles, rest, st);
   }
   return hipErrorInvalidValue;
 }

@@ -17,6 +17,9 @@ constexpr int kOccForceTiles = 6;
 // The sparse-tile kernels (sph_sparse.h): one tile per wave.
 constexpr int kOccSparse = 6;  // density, gradient (their LDS allows 6)
 constexpr int kOccForceSparse = 5;
+// The tiles of 16 (sph_tile.h).
+constexpr int kOccTile16 = 5;  // density, gradient (their LDS allows 5)
+constexpr int kOccForceTile16 = 4;
 // The persistent forms of both engines: their loop around the tile costs
 // registers (at 7 waves per SIMD the density form spilled 34 VGPRs).
 constexpr int kOccSparseQueue = 5;
@@ -147,6 +150,7 @@ struct DensityLoop {
   static constexpr int kWavesPerSimd = kOccDensity;
   static constexpr int kTileWavesPerSimd = kOccDensity;
   static constexpr int kSparseWavesPerSimd = kOccSparse;
+  static constexpr int kTile16WavesPerSimd = kOccTile16;
   using Rec = DensRec;
   using Acc = DensAcc;
   using I = DensI;
@@ -253,6 +257,7 @@ struct GradientLoop {
   static constexpr int kWavesPerSimd = kOccGradient;
   static constexpr int kTileWavesPerSimd = kOccGradient;
   static constexpr int kSparseWavesPerSimd = kOccSparse;
+  static constexpr int kTile16WavesPerSimd = kOccTile16;
   using Rec = GradRec;
   using Acc = GradAcc;
   using I = GradI;
@@ -346,6 +351,7 @@ struct ForceLoop {
   static constexpr int kWavesPerSimd = kOccForce;
   static constexpr int kTileWavesPerSimd = kOccForceTiles;
   static constexpr int kSparseWavesPerSimd = kOccForceSparse;
+  static constexpr int kTile16WavesPerSimd = kOccForceTile16;
   using Rec = ForceRec;
   using Acc = ForceAcc;
   using I = ForceI;

@@ -421,36 +421,10 @@ __global__ __launch_bounds__(64, kOccSparseQueue) void k_sparse_queue(
     DevParts d, LoopArgs la, ChunkArgs c1, ChunkArgs c2,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq) {
-  const int nt = *tq.ntiles;
-  const int per = (nt + 7) >> 3;
-  int q = blockIdx.x & 7;
-  for (int tries = 0; tries < 8;) {
-    const int hi = min(nt, (q + 1) * per);
-    int base = 0;
-    if ((threadIdx.x & 63) == 0) {
-      // Once its own queue is exhausted, a wave reads the others' heads
-      // before it tries to steal: an exhausted queue then costs no atomic
-      // (the tail of a drain, and every wave of a grid for a nearly empty
-      // queue); its own queue takes the atomic directly.
-      base = tries > 0 ? __hip_atomic_load(&tq.heads[64 * q], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT)
-                       : 0;
-      if (tries == 0 || q * per + base < hi)
-        base = atomicAdd(&tq.heads[64 * q], kGrab);
-    }
-    base = uniform(__shfl(base, 0));
-    const int lo = q * per + base;
-    if (lo >= hi) {  // uniform: this queue is exhausted
-      q = (q + 1) & 7;
-      tries++;
-      continue;
-    }
-    const int end = min(hi, lo + kGrab);
-    for (int t = lo; t < end; t++) {
-      wave_sync();
-      run_sparse<L>(d, la, c1, c2, rec, pos, tq, t);
-    }
-  }
+  drain_queue(tq, [&](int t) {
+    wave_sync();
+    run_sparse<L>(d, la, c1, c2, rec, pos, tq, t);
+  });
 }
 
 }  // namespace sphl

@@ -1,0 +1,510 @@
+// sph_tile.h -- neighbour loops over the work queue's tiles of 16 particles.
+//
+// One wave64 owns a tile of up to 16 particles of one cell: lane g + 16 s is
+// candidate stream s of 4 of particle g, as in the chunk engine
+// (sph_gather.h), and visits the same candidates in the same order, so the
+// sums are those of that engine bit for bit.  The work between is arranged
+// in windows of 1024 candidates (256 rows of 4):
+//
+//   1. cull: the chunks of the 27 neighbour cells, one per lane, box against
+//      the tile's box in FP32 (ChunkArgs::fbox) in the tile frame -- positions
+//      relative to the centre of the tile's box; survivors in LDS;
+//   2. test: 64 candidates at a time are staged in the tile frame and met
+//      with the 16 particles by v_mfma_f32_16x16x4_f32 (see the chunk
+//      engine's matrix pre-test); the signs of the results are the hits;
+//   3. expand: each lane writes the rows of its hits to its list in LDS;
+//   4. walk: each lane takes its hits in turn, the next record's loads in
+//      flight while the current one is evaluated (FP64 pair contract, the
+//      loop's test, the interaction).
+//
+// Bound: VALU issue in the walk, whose wave runs as long as its fullest lane.
+// A window of 256 rows evens the lanes out better than the chunk engine's
+// 128 (modulated 97^3 box: 26 -> 21 iterations per tile for 13.5 hits per
+// lane), the matrix test takes 1 instruction per 64 pairs beside the signs
+// (the FP16 rows took 7), and the pipelined walk has one load latency per
+// hit instead of three.
+//
+// The density form can iterate the smoothing lengths itself (ITER): the wave
+// holds the finished sums of its particles after the walk, takes their
+// Newton step (sph_ghost.h) and goes on with the particles that are not done
+// -- on the same lists while their radius is inside the one the lists were
+// made with, else from step 1 -- until all have converged.  That replaces a
+// ghost launch, a tile build and a density launch per round.
+#pragma once
+
+#include "sph_gather.h"
+#include "sph_ghost.h"
+
+namespace sphl {
+
+constexpr int kTileRows = 256;    // rows of 4 candidates in a window
+constexpr int kTileHits = 44;     // hits of a lane between two walks
+
+// What the iterating density form needs beside the loop's arguments.
+struct TileGhost {
+  GhostArgs ga;
+  int max_iter;
+  unsigned long long *counters;  // launch_ghost's: [0] not converged,
+                                 // [3..] density interactions
+  unsigned int *rounds;          // largest number of density evaluations
+};
+
+template <class L, int CJ>
+struct TileLds {
+  static constexpr int RPC = CJ / 4;               // rows per chunk
+  static constexpr int CHUNKS = kTileRows / RPC;   // chunks of a window
+  double fo[27 * 6];    // pair-contract frame {oi, oj} of each neighbour
+  double xi[16 * 3];    // the particles' positions (own cell: oi = oj = x_i)
+  float qoff[27 * 3];   // neighbour image corners relative to the tile centre
+  int qk0[27], qpre[28], qj0[27], qj1[27];
+  // staged candidates: rows x, y, z, |x|^2 and (force) |x|^2 - H_j^2
+  float tp[L::kSymmetric ? kTpLen : 4 * kTpRow];
+  // surviving chunks: (neighbour << 27) | first record slot
+  unsigned int surv[CHUNKS + 64];
+  unsigned char rows[kTileHits * 64];  // hit k of lane l at 64 k + l
+};
+
+// Maximum over the 16 lanes of a row of lanes (lane % 16 varies).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(
+      0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, dpp_f<0x128>(v));  // row_ror:8, 4, 2, 1
+  v = fmaxf(v, dpp_f<0x124>(v));
+  v = fmaxf(v, dpp_f<0x122>(v));
+  return fmaxf(v, dpp_f<0x121>(v));
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// n / d for 0 <= n < 2^31 by the host's floor(2^32 / d) (d >= 2): the
+// estimate is at most 1 short.
+__device__ __forceinline__ int div_magic(int n, int d, unsigned int magic) {
+  const int q = (int)__umulhi((unsigned int)n, magic);
+  return n - q * d >= d ? q + 1 : q;
+}
+
+// One tile of the work queue.
+template <class L, int CJ, bool ITER>
+__device__ __forceinline__ void run_tile(
+    const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
+    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
+    const TileArgs &tq, int tile, const TileGhost &tg) {
+  using Sh = TileLds<L, CJ>;
+  using Rec = typename L::Rec;
+  constexpr int RPC = Sh::RPC, CHUNKS = Sh::CHUNKS;
+  constexpr int G = 64 / CJ;  // chunks staged together
+  static_assert(!ITER || !L::kSymmetric, "the density loop iterates");
+  __shared__ Sh sh;
+  const int lane = threadIdx.x & 63;
+  const int g = lane & 15, s = lane >> 4;
+  const int ts = uniform(tq.tile_start[tile]);
+  const int cnt_i = uniform(tq.tile_start[tile + 1]) - ts;
+  const int cell_i = uniform(tq.tile_cell[tile]);
+  const bool act = g < cnt_i;
+  const int i = act ? tq.alist[ts + g] : 0;
+  const int ic = act ? rec_slot(d, i) : -1;  // record slot
+  typename L::I st{};
+  st.x = st.y = st.z = kFar;
+  if (act) L::load_i(d, i, st);
+
+  // The tile's box in its cell's frame, rounded to float (monotone), the
+  // tile centre in FP64, and the largest radius.
+  const int cyz = div_magic(cell_i, la.grid.nc[2], la.magic[2]);
+  const int cz = cell_i - cyz * la.grid.nc[2];
+  const int cx = div_magic(cyz, la.grid.nc[1], la.magic[1]);
+  const int cy = cyz - cx * la.grid.nc[1];
+  const int ci3[3] = {cx, cy, cz};
+  double cen[3];
+  float half[3];  // half extents, at least those of the particles
+  float fi[3];    // the particle in the tile frame
+  {
+    const double xi[3] = {st.x, st.y, st.z};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double corner = (double)ci3[k] * la.w[k];
+      const float f = act ? (float)(xi[k] - corner) : -1e30f;
+      const float hi = row16_max(f);
+      const float lo = -row16_max(act ? -f : -1e30f);
+      cen[k] = corner + (double)(0.5f * (lane_value(lo, 0) + lane_value(hi, 0)));
+      fi[k] = act ? (float)(xi[k] - cen[k]) : 0.f;
+      half[k] = lane_value(row16_max(fabsf(fi[k])), 0);
+    }
+  }
+  const float hg2i = lane_value(row16_max(act ? st.hg2 : 0.f), 0);
+  // lengths of the matrix test in units of the largest radius
+  const float invR = lane_value(hg2i > 0.f ? 1.f / sqrtf(hg2i) : 1.f, 0);
+  const float invR2 = lane_value(invR * invR * kRadUp, 0);
+  if (s == 0 && act) {
+    sh.xi[3 * g] = st.x;
+    sh.xi[3 * g + 1] = st.y;
+    sh.xi[3 * g + 2] = st.z;
+  }
+
+  // Neighbour table: lane q < 27 describes neighbour q of kStencilOrder.
+  int nchq = 0;
+  if (lane < 27) {
+    const int o = lane == 0 ? 13 : ((lane & 1) ? lane >> 1 : 27 - (lane >> 1));
+    const int o3[3] = {o / 9 - 1, (o / 3) % 3 - 1, o % 3 - 1};
+    int v[3];
+    double t[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      v[k] = ci3[k] + o3[k];
+      t[k] = 0.0;
+      if (v[k] < 0) {
+        v[k] += la.grid.nc[k];
+        t[k] = -la.grid.dim[k];
+      } else if (v[k] >= la.grid.nc[k]) {
+        v[k] -= la.grid.nc[k];
+        t[k] = la.grid.dim[k];
+      }
+      sh.qoff[3 * lane + k] =
+          (float)(((double)v[k] * la.w[k] + t[k]) - cen[k]);
+    }
+    const int cj = (v[0] * la.grid.nc[1] + v[1]) * la.grid.nc[2] + v[2];
+    const int k0 = ca.cell_chunk[cj], k1 = ca.cell_chunk[cj + 1];
+    sh.qk0[lane] = k0;
+    sh.qj0[lane] = la.cell_start[cj];
+    sh.qj1[lane] = la.cell_start[cj + 1];
+    nchq = k1 - k0;
+    double fo[6];
+    (void)pair_frame(o3, ci3, v, t, la.w, fo);
+    for (int k = 0; k < 6; k++) sh.fo[6 * lane + k] = fo[k];
+  }
+  int incl = nchq;  // inclusive prefix over lanes 0..31
+#pragma unroll
+  for (int off = 1; off < 32; off <<= 1) {
+    const int v = __shfl_up(incl, off);
+    if (lane >= off) incl += v;
+  }
+  if (lane < 27) sh.qpre[lane] = incl - nchq;
+  const int total = __builtin_amdgcn_readlane(incl, 26);
+
+  // i side of the matrix test (see the chunk engine)
+  const float ux = fi[0] * invR, uy = fi[1] * invR, uz = fi[2] * invR;
+  const float isq = fmaf(uz, uz, fmaf(uy, uy, ux * ux)) * kSqLo;
+  const float mb =
+      s == 3 ? 1.f : (act ? -2.f * (s == 0 ? ux : (s == 1 ? uy : uz)) : 0.f);
+  // candidate (row of A) of this lane and its component
+  const int am = (lane & 3) * 4 + ((lane >> 2) & 3);
+  const int t1 = s * kTpRow + am;
+  const int t2 = s == 3 ? kTpRowJ + am : t1;
+
+  typename L::Acc acc;
+  int cnt = 0;  // hits in this lane's list
+
+  // Step 4: the lists against the exact contract.
+  auto eval = [&](unsigned int info, const Rec &r, int j) {
+    const int q = (int)(info >> 27);
+    // own cell: oi = oj = x_i, which gives 0 - (float)(x_j - x_i)
+    const double *fo = q ? &sh.fo[6 * q] : &sh.xi[3 * g];
+    const double *fj = q ? fo + 3 : fo;
+    const float dx = (float)(st.x - fo[0]) - (float)(r.x - fj[0]);
+    const float dy = (float)(st.y - fo[1]) - (float)(r.y - fj[1]);
+    const float dz = (float)(st.z - fo[2]) - (float)(r.z - fj[2]);
+    const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+    // (the matrix test passes the particle itself)
+    if (L::test(r2, st, &r) && j != ic) L::interact(r2, dx, dy, dz, st, r, acc);
+  };
+  auto walk = [&]() {
+    auto locate = [&](int k, unsigned int &info) -> int {
+      const int row = sh.rows[64 * k + lane];
+      info = sh.surv[row / RPC];
+      return (int)(info & kRowMask) + (row % RPC) * 4 + s;
+    };
+    unsigned int n0 = 0u, n1 = 0u;
+    int j0 = 0, j1 = 0;
+    Rec r0, r1;
+    if (cnt > 0) {
+      j0 = locate(0, n0);
+      r0 = rec[j0];
+    }
+    for (int k = 0; k < cnt; k += 2) {
+      if (k + 1 < cnt) {
+        j1 = locate(k + 1, n1);
+        r1 = rec[j1];
+      }
+      eval(n0, r0, j0);
+      if (k + 1 >= cnt) break;
+      if (k + 2 < cnt) {
+        j0 = locate(k + 2, n0);
+        r0 = rec[j0];
+      }
+      eval(n1, r1, j1);
+    }
+  };
+
+  // The candidates of a sweep, a window at a time.  pre: the lane's squared
+  // pre-test radius (negative: it takes no part); fb: chunks culled so far;
+  // ns: survivors in LDS (the first `done` of them walked already).
+  float pre = -1.f, maxpre = -1.f;
+  int fb = 0, ns = 0, done = 0;
+  // Steps 1 to 3: fills the lists from the next window and returns whether
+  // candidates are left after it.
+  auto window = [&]() -> bool {
+    // the survivors past the last window open this one
+    if (done > 0) {
+      for (int c = done; c < ns; c += 64) {  // uniform
+        const unsigned int e = c + lane < ns ? sh.surv[c + lane] : 0u;
+        wave_sync();
+        if (c + lane < ns) sh.surv[c - done + lane] = e;
+        wave_sync();
+      }
+      ns -= done;
+    }
+    // 1. cull until the window is full
+    while (ns < CHUNKS && fb < total) {
+      const int f = fb + lane;
+      bool pass = false;
+      unsigned int pe = 0u;
+      if (f < total) {
+        int q = 0;
+#pragma unroll
+        for (int b = 16; b > 0; b >>= 1)
+          if (q + b < 27 && sh.qpre[q + b] <= f) q += b;
+        const int kin = f - sh.qpre[q];
+        const int kc = sh.qk0[q] + kin;
+        const float4 lo = ca.fbox[2 * kc], hi = ca.fbox[2 * kc + 1];
+        const float ox = sh.qoff[3 * q], oy = sh.qoff[3 * q + 1],
+                    oz = sh.qoff[3 * q + 2];
+        const float gx =
+            fmaxf(0.f, fmaxf(lo.x + ox - half[0], -half[0] - (hi.x + ox)));
+        const float gy =
+            fmaxf(0.f, fmaxf(lo.y + oy - half[1], -half[1] - (hi.y + oy)));
+        const float gz =
+            fmaxf(0.f, fmaxf(lo.z + oz - half[2], -half[2] - (hi.z + oz)));
+        const float gap2 = fmaf(gz, gz, fmaf(gy, gy, gx * gx));
+        pass = gap2 < (L::kSymmetric ? fmaxf(maxpre, lo.w) : maxpre);
+        pe = ((unsigned int)q << 27) | (unsigned int)(sh.qj0[q] + kin * CJ);
+      }
+      const unsigned long long pm = __ballot(pass);
+      if (pass) sh.surv[ns + (int)__popcll(pm & ((1ull << lane) - 1ull))] = pe;
+      ns += (int)__popcll(pm);
+      fb += 64;
+    }
+    wave_sync();
+    // 2. and 3. test and expand, two groups of 64 candidates at a time
+    const int nw = min(ns, CHUNKS);
+    const int ng = (nw + G - 1) / G;
+    done = nw;
+    cnt = 0;
+    const float ci = pre >= 0.f ? fmaf(-pre * kRadUp, invR2, isq) : 1e30f;
+    const float4v mc = {ci, ci, ci, ci};
+    const float cs = pre >= 0.f ? isq : 1e30f;
+    const float4v mc2 = {cs, cs, cs, cs};
+    // the candidate of this lane in group k: loaded one group ahead
+    auto load = [&](int k, int &q) -> PosRec {
+      const int c = k * G + lane / CJ;
+      PosRec p{0.f, 0.f, 0.f, 0.f};
+      q = -1;
+      if (c < nw) {
+        const unsigned int e = sh.surv[c];
+        const int j = (int)(e & kRowMask) + lane % CJ;
+        if (j < sh.qj1[e >> 27]) {
+          q = (int)(e >> 27);
+          p = pos[j];
+        }
+      }
+      return p;
+    };
+    int q;
+    PosRec p = load(0, q);
+    for (int k0 = 0; k0 < ng; k0 += 2) {
+      unsigned int hits = 0u;
+#pragma unroll
+      for (int kk = 0; kk < 2; kk++) {
+        const int k = k0 + kk;
+        if (k >= ng) break;  // uniform
+        // past the end of a short chunk: far away
+        float vx = 1e15f, vy = 0.f, vz = 0.f, sq = 1e30f, sqj = 1e30f;
+        if (q >= 0) {
+          vx = (p.x + sh.qoff[3 * q]) * invR;
+          vy = (p.y + sh.qoff[3 * q + 1]) * invR;
+          vz = (p.z + sh.qoff[3 * q + 2]) * invR;
+          sq = fmaf(vz, vz, fmaf(vy, vy, vx * vx)) * kSqLo;
+          if (L::kSymmetric) sqj = fmaf(-p.hg2m * kRadUp, invR2, sq);
+        }
+        if (k + 1 < ng) p = load(k + 1, q);
+        sh.tp[lane] = vx;
+        sh.tp[kTpRow + lane] = vy;
+        sh.tp[2 * kTpRow + lane] = vz;
+        sh.tp[3 * kTpRow + lane] = sq;
+        if (L::kSymmetric) sh.tp[kTpRowJ + lane] = sqj;
+        wave_sync();
+        unsigned int w = 0u;  // row 0 in the highest of 16 bits
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+          float4v dd = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              sh.tp[t1 + 16 * b], mb, mc, 0, 0, 0);
+          if (L::kSymmetric) {
+            const float4v d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                sh.tp[t2 + 16 * b], mb, mc2, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              dd[r] = __uint_as_float(__float_as_uint(dd[r]) |
+                                      __float_as_uint(d2[r]));
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++)  // append the sign
+            w = __builtin_amdgcn_alignbit(w, __float_as_uint(dd[r]), 31);
+        }
+        wave_sync();
+        hits |= (__builtin_bitreverse32(w) >> 16) << (16 * kk);
+      }
+      // a list that these rows could overfill ends the window before them
+      // (they always fit an empty list)
+      if (__any(cnt + __popc(hits) > kTileHits)) {  // uniform
+        done = k0 * G;
+        break;
+      }
+      while (hits != 0u) {  // rows of these groups: 16 k0 + bit
+        const int b = __builtin_ctz(hits);
+        hits &= hits - 1u;
+        sh.rows[64 * cnt + lane] = (unsigned char)(16 * k0 + b);
+        cnt++;
+      }
+    }
+    wave_sync();
+    return done < ns || fb < total;
+  };
+  auto sweep = [&](float radius2) {
+    pre = radius2;
+    maxpre = lane_value(row16_max(pre), 0);
+    fb = ns = done = 0;
+  };
+
+  if constexpr (!ITER) {
+    L::identity(acc);
+    if (act && s == 0) L::fresh_acc(st, acc);
+    wave_sync();
+    sweep(act ? pretest_radius2(st.hg2, la.pos_eps) : -1.f);
+    bool more;
+    do {
+      more = window();
+      walk();
+      wave_sync();
+    } while (more);  // uniform
+    L::template combine<4>(acc);
+    if (act && s == 0) L::store_acc(d, i, acc);
+  } else {
+    // The particle's iteration; every lane of a particle holds its whole
+    // sums after the combination and takes the same step.
+    GhostState gs{0.f, 0.f, tg.ga.h_max};
+    if (act) gs.h = d.h[i];
+    bool live = act;
+    float listed = -1.f;  // squared radius that the lists cover
+    // the lists hold every hit of the sweep (one window took it all)
+    bool whole = false, fresh = true;
+    int work = 0, round = 1;
+    L::identity(acc);
+    wave_sync();
+    for (;;) {  // a window, or a walk over lists that still serve
+      bool more = false;
+      if (fresh || !whole) {  // uniform
+        if (fresh) {
+          // room for the next steps' growth: the lists cover 1 % more at
+          // the first evaluation and 2 % more later (radius)
+          listed = st.hg2 * (round == 1 ? 1.0201f : 1.0404f);
+          sweep(live ? pretest_radius2(listed, la.pos_eps) : -1.f);
+        }
+        more = window();
+        whole = fresh && !more;
+        fresh = false;
+      }
+      walk();
+      wave_sync();
+      if (more) continue;  // uniform
+      L::template combine<4>(acc);
+      if (live) {
+        // (an opaque copy: the addresses of the particle's fields are formed
+        // here and not kept in registers across the walks)
+        int iw = i;
+        asm volatile("" : "+v"(iw));
+        work += acc.n;
+        DensSums a{acc.rho, acc.rho_dh, acc.wc, acc.wc_dh,
+                   acc.divv, acc.rx, acc.ry, acc.rz};
+        const bool again = ghost_step(tg.ga, d.m[iw], gs, a);
+        if (again && round < tg.max_iter) {
+          st.h_inv = 1.f / gs.h;
+          st.hg2 = search_radius2(gs.h);
+        } else {
+          live = false;
+          cnt = 0;
+          if (s == 0) {
+            d.nd[iw] = acc.n;
+            if (again) {  // not converged
+              d.h[iw] = gs.h;
+              d.redo[iw] = 1;
+              atomicAdd(&tg.counters[0], 1ull);
+            } else {
+              ghost_finish(d, tg.ga, iw, gs.h, a);
+            }
+          }
+        }
+      }
+      if (!__any(live)) break;  // uniform
+      L::identity(acc);
+      round++;
+      fresh = !whole || __any(live && !(st.hg2 <= listed));
+    }
+    // density interactions of the tile, and its rounds
+    work = s == 0 ? work : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) work += __shfl_xor(work, off);
+    if (lane == 0) {
+      atomicAdd(&tg.counters[3 + tile % kGhostWorkSlots],
+                (unsigned long long)work);
+      // a plain read first: only a wave that raises the maximum pays an
+      // atomic
+      if ((unsigned int)round >
+          __hip_atomic_load(tg.rounds, __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(tg.rounds, (unsigned int)round);
+    }
+  }
+}
+
+// One wave per tile over a grid sized for the tile count (see k_loop_tiles).
+template <class L, int CJ, bool ITER>
+__global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16(
+    DevParts d, LoopArgs la, ChunkArgs ca,
+    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
+    TileArgs tq, TileGhost tg) {
+  const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
+  if (t >= *tq.ntiles) return;  // uniform per wave
+  run_tile<L, CJ, ITER>(d, la, ca, rec, pos, tq, t, tg);
+}
+
+// The tiles beyond a grid of b0 blocks (see k_loop_tiles_rest).
+template <class L, int CJ, bool ITER>
+__global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_rest(
+    DevParts d, LoopArgs la, ChunkArgs ca,
+    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
+    TileArgs tq, TileGhost tg, int b0) {
+  const int n = *tq.ntiles;
+  const int nb = xcd_blocks(n);
+  for (int b = b0 + (int)blockIdx.x; b < nb; b += (int)gridDim.x) {
+    const int t = xcd_item(b, threadIdx.x >> 6, n);
+    if (t >= n) continue;  // uniform per wave
+    wave_sync();
+    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, tq, t, tg);
+  }
+}
+
+// Persistent form (see k_loop_queue).
+template <class L, int CJ, bool ITER>
+__global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_queue(
+    DevParts d, LoopArgs la, ChunkArgs ca,
+    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
+    TileArgs tq, TileGhost tg) {
+  drain_queue(tq, [&](int t) {
+    wave_sync();
+    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, tq, t, tg);
+  });
+}
+
+}  // namespace sphl

@@ -1,0 +1,99 @@
+"""The tiles of 16 of the work queue (swift_amd/csrc/sph_tile.h): their
+windows, hit lists and in-wave smoothing-length iteration against the chunk
+grid with its separate ghost rounds, bit for bit, and against the oracle.
+
+Boxes where the tiling can go wrong: cells that are no multiple of 16, cells
+with few particles, radii that give a lane more hits than its list
+holds and a tile more candidates than a window, partly active and inhibited
+particles, and starts that need many rounds.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from parity import assert_parity
+
+pytestmark = pytest.mark.gpu
+
+
+def _box(name):
+    from swift_amd import HydroProps, ics
+    if name == "ragged":
+        return HydroProps(ncell=(3, 4, 3)), ics.modulated_box(13, seed=2, amp=0.3)
+    if name == "lists":  # 500 neighbours at the start, all cells in reach
+        st = ics.modulated_box(15, seed=3, amp=0.2)
+        st["h"] = np.full_like(st["h"], 0.33 / 1.936492)
+        return HydroProps(ncell=(3, 3, 3)), st
+    if name == "windows":  # 3000 particles in a cell, half of it in reach
+        st = ics.clustered_box(9000, seed=4, n_spheres=3, a_min=0.02,
+                               a_max=0.05)
+        st["h"] = np.minimum(st["h"] * np.float32(1.9),
+                             np.float32(0.24 / 1.936492))
+        return HydroProps(ncell=(4, 4, 4)), st
+    if name == "few":  # 8 particles in a cell
+        st = ics.lattice_box(6, seed=5, jitter=0.3)
+        st["h"] = np.full_like(st["h"], 0.09)
+        return HydroProps(ncell=(3, 3, 3), eta=0.85), st
+    st = ics.modulated_box(14, seed=6, amp=0.4)
+    st["h"] *= np.float32(0.6)
+    if name == "half":
+        ics.set_active_fraction(st, 0.5, seed=7)
+        # the state that inactive neighbours bring along
+        st["rho"] = np.ones_like(st["rho"])
+        st["pressure"] = (st["u"] * np.float32(2 / 3)).astype(np.float32)
+        st["soundspeed"] = np.sqrt(st["pressure"] * np.float32(5 / 3))
+    else:
+        rng = np.random.default_rng(8)
+        st["time_bin"][rng.uniform(size=st["h"].size) < 0.2] = \
+            ics.TIME_BIN_INHIBITED
+    return HydroProps(ncell=(3, 3, 4)), st
+
+
+def _run(props, st, mode, shape, graph=False, waves=0):
+    from swift_amd import Engine
+    with Engine(props) as eng:
+        eng.set_regrid(False)
+        eng.set_schedule(mode, waves)
+        for loop in ("density", "gradient", "force"):
+            eng.set_tile_shape(loop, *shape)
+        eng.set_particles(st)
+        eng.save_state()
+        for _ in range(3 if graph else 1):
+            eng.restore_state()
+            s = eng.pass_graph() if graph else eng.pass_batched()
+        return s, eng.results()
+
+
+@pytest.mark.parametrize("box", ["ragged", "lists", "windows", "few", "half",
+                                 "inhibited"])
+def test_tiles16_match_grid(orc, box):
+    props, st = _box(box)
+    s0, r0 = _run(props, st, 0, (16, 16))
+    act = st["time_bin"] <= props.max_active_bin
+    chk = {k: np.array(v, copy=True) for k, v in st.items()}
+    chk["h"] = r0["h"]
+    assert_parity(r0, orc.pass_fp64(props, chk), act)
+    for kw in (dict(mode=1, shape=(16, 16)), dict(mode=1, shape=(16, 8)),
+               dict(mode=1, shape=(16, 32)),
+               dict(mode=2, shape=(16, 16), waves=5),
+               dict(mode=1, shape=(16, 16), graph=True)):
+        s1, r1 = _run(props, st, **kw)
+        for k in r0:
+            assert np.array_equal(r0[k][act], r1[k][act], equal_nan=True), (kw, k)
+        for k in ("ghost_rounds", "n_density_all", "n_density", "n_force"):
+            assert s0[k] == s1[k], (kw, k)
+    if box == "windows":
+        assert s0["ghost_rounds"] >= 4
+
+
+def test_tiles16_unconverged_is_an_error():
+    """More rounds needed than allowed: status 3 from both forms."""
+    import dataclasses
+    from swift_amd import SwsphError
+    props, st = _box("ragged")
+    props = dataclasses.replace(props, max_iter=2)
+    for kw in (dict(mode=0, shape=(16, 16)), dict(mode=1, shape=(16, 16)),
+               dict(mode=1, shape=(16, 16), graph=True)):
+        with pytest.raises(SwsphError, match="status 3"):
+            _run(props, st, **kw)
