@@ -819,7 +819,8 @@ bool iterates(const swsph_engine *e) {
 // neighbour list), drained by persistent waves; `build` rebuilds the lists
 // of the selected particles while doing their density.
 int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
-               bool build, bool iter = false) {
+               bool build, const GhostArgs *iter = nullptr,
+               bool given = false) {
   int rc = 0;
   const int C = build ? kListChunk : e->loop_c[(int)k];
   const int CJ = build ? kListChunk : e->loop_cj[(int)k];
@@ -898,10 +899,10 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
                                persistent, e->queue_waves, max_tiles, rest,
                                e->st));
   else if ((max_tiles > 0 || rest) && C == 16 && !build)
-    HIPCHK(sphk::launch_tile16(k, iter, e->d, la, chunk_args(t), ta,
-                               batched_ghost_args(e), e->props.max_iter,
-                               e->d_redo, persistent, e->queue_waves, max_tiles,
-                               rest, e->st));
+    HIPCHK(sphk::launch_tile16(k, iter != nullptr, given, e->d, la,
+                               chunk_args(t), ta, iter ? *iter : GhostArgs{},
+                               e->props.max_iter, e->d_redo, persistent,
+                               e->queue_waves, max_tiles, rest, e->st));
   else if (max_tiles > 0 || rest)
     HIPCHK(sphk::launch_queue(k, build, e->d, la, chunk_args(t), ta, e->nl, C,
                               CJ, persistent, e->queue_waves, max_tiles, rest,
@@ -1089,12 +1090,32 @@ int ensure_subset(swsph_engine *e, int count) {
 // finish leaves the cell's gradient records and chunk bounds current.
 int ghost_cell(swsph_engine *e, int ci, int *rounds, int off = 0, int nt = 1) {
   const int lo = e->cell_start[ci], hi = e->cell_start[ci + 1];
-  const GhostArgs ga = ghost_args(e);
-  std::vector<int> nb;
-  all_neighbours(e, ci, nb);
+  GhostArgs ga = ghost_args(e);
   int redo = 0;
   int it = 0;
   int rc = 0;
+  if (chunk_c(e, (int)LoopKind::Density) == 16 && !e->use_lists) {
+    // the cell's waves iterate their particles themselves, the re-runs over
+    // the whole stencil at once (27 launches per round otherwise)
+    const swsph_engine::ChunkTable *t = chunk_table(e, 16, &rc);
+    if (!t) return rc;
+    ga.grad_rec = 1;
+    // the work slots accumulate over the ghosts of a pass
+    HIPCHK(sphk::launch_zero_u64(e->d_redo, 3, e->st));
+    HIPCHK(sphk::launch_zero_u64(e->d_redo + kGhostRounds, 1, e->st));
+    HIPCHK(sphk::launch_ghost_cell(
+        e->d, loop_args(e), chunk_args(t), ga, e->props.max_iter, e->d_redo,
+        ci, t->cell_chunk_h[ci + 1] - t->cell_chunk_h[ci], off, nt, e->st));
+    e->launches += 3;
+    if ((rc = read_redo(e, &redo))) return rc;
+    if (redo > 0)
+      return fail(3, "Smoothing length failed to converge on %d particles",
+                  redo);
+    if (rounds) *rounds = std::max(*rounds, (int)e->h_redo[kGhostRounds]);
+    return refresh_bounds(e, ci, ci + 1);
+  }
+  std::vector<int> nb;
+  all_neighbours(e, ci, nb);
   // with shares, the re-runs take the flags of this share only (the other
   // shares' particles keep the flags hydro_init_part set until their own
   // ghost runs)
@@ -1518,7 +1539,8 @@ int phase_start(swsph_engine *e) {
     HIPCHK(sphk::launch_zero_u64(e->d_redo, kGhostCounters, e->st));
     e->launches++;
     e->tiles_c = 0;  // activity may have changed since the last pass
-    return queue_loop(e, LoopKind::Density, 0, nullptr, false, true);
+    const GhostArgs ga = batched_ghost_args(e);
+    return queue_loop(e, LoopKind::Density, 0, nullptr, false, &ga);
   }
   HIPCHK(sphk::launch_init_density(e->d, 0, (int)e->n, e->props.max_active_bin,
                                    e->props.h_max, e->st, nullptr, nullptr,
@@ -1891,7 +1913,27 @@ int init_cells_locked(swsph_engine *e, const int *cells, int n) {
 int ghost_cells_locked(swsph_engine *e, const int *cells, int n, int *rounds) {
   int rc;
   if ((rc = select_cells(e, cells, n))) return rc;
-  const GhostArgs ga = ghost_args(e);
+  GhostArgs ga = ghost_args(e);
+  if (iterates(e)) {
+    ga.grad_rec = 1;
+    int redo = 0;
+    // the work slots accumulate over the ghosts of a pass
+    hipError_t err = sphk::launch_zero_u64(e->d_redo, 3, e->st);
+    if (err == hipSuccess)
+      err = sphk::launch_zero_u64(e->d_redo + kGhostRounds, 1, e->st);
+    e->launches += 2;
+    if (err != hipSuccess) rc = fail(2, "ghost: %s", hipGetErrorString(err));
+    if (!rc)
+      rc = queue_loop(e, LoopKind::Density, 1, e->d.redo, false, &ga, true);
+    if (!rc) rc = read_redo(e, &redo);
+    if (!rc && redo > 0)
+      rc = fail(3, "Smoothing length failed to converge on %d particles", redo);
+    clear_cells(e);
+    if (!rc) rc = refresh_bounds(e, 0, e->ncells);
+    if (rounds)
+      *rounds = std::max(*rounds, std::max(1, (int)e->h_redo[kGhostRounds]));
+    return rc;
+  }
   const int *list, *cnt;
   int redo = 0, it = 0;
   for (; it < e->props.max_iter; it++) {

@@ -324,12 +324,21 @@ hipError_t launch_queue(LoopKind kind, bool build_lists, const DevParts &d,
 // 32; grids as launch_queue.  `iter` (density only): the tiles iterate the
 // smoothing lengths to convergence and finish their particles as the ghost
 // does with ga; counters as launch_ghost's plus [kGhostRounds], all zeroed
-// by the caller.
-hipError_t launch_tile16(LoopKind kind, bool iter, const DevParts &d,
-                         const LoopArgs &la, const ChunkArgs &ca,
-                         const TileArgs &ta, const GhostArgs &ga, int max_iter,
+// by the caller.  `given`: the sums of the first evaluation are in the
+// particles' fields already.
+hipError_t launch_tile16(LoopKind kind, bool iter, bool given,
+                         const DevParts &d, const LoopArgs &la,
+                         const ChunkArgs &ca, const TileArgs &ta,
+                         const GhostArgs &ga, int max_iter,
                          unsigned long long *counters, bool persistent,
                          int waves, int max_tiles, bool rest, hipStream_t st);
+// The same on the flagged particles of one cell (nchunks chunks of the table
+// of 16) of share off of nt, after their density tasks.
+hipError_t launch_ghost_cell(const DevParts &d, const LoopArgs &la,
+                             const ChunkArgs &ca, const GhostArgs &ga,
+                             int max_iter, unsigned long long *counters,
+                             int cell, int nchunks, int off, int nt,
+                             hipStream_t st);
 // The tiles of the table in `ts` that hold a particle with filt[i] != 0,
 // appended to ids (in no fixed order: each tile's sums are its own) with
 // their count in *nids.

@@ -1105,14 +1105,30 @@ hipError_t tile16_any(const DevParts &d, const LoopArgs &la,
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_tile16(LoopKind kind, bool iter, const DevParts &d,
-                         const LoopArgs &la, const ChunkArgs &ca,
-                         const TileArgs &ta, const GhostArgs &ga, int max_iter,
+hipError_t launch_ghost_cell(const DevParts &d, const LoopArgs &la,
+                             const ChunkArgs &ca, const GhostArgs &ga,
+                             int max_iter, unsigned long long *counters,
+                             int cell, int nchunks, int off, int nt,
+                             hipStream_t st) {
+  if (!ca.fbox || ca.C != 16) return hipErrorInvalidValue;
+  if (nchunks <= 0) return hipSuccess;
+  const TileGhost tg{ga, max_iter, counters,
+                     (unsigned int *)(counters + kGhostRounds), 1};
+  hipLaunchKernelGGL((k_ghost_cell<DensityLoop>), dim3(nchunks), dim3(64), 0,
+                     st, d, la, ca, d.rd, (const PosRec *)d.pos, tg, cell, off,
+                     nt);
+  return hipGetLastError();
+}
+
+hipError_t launch_tile16(LoopKind kind, bool iter, bool given,
+                         const DevParts &d, const LoopArgs &la,
+                         const ChunkArgs &ca, const TileArgs &ta,
+                         const GhostArgs &ga, int max_iter,
                          unsigned long long *counters, bool persistent,
                          int waves, int max_tiles, bool rest, hipStream_t st) {
   if (!ca.fbox || !la.fresh || ta.ids || ta.filt) return hipErrorInvalidValue;
   const TileGhost tg{ga, max_iter, counters,
-                     (unsigned int *)(counters + kGhostRounds)};
+                     (unsigned int *)(counters + kGhostRounds), given ? 1 : 0};
   switch (kind) {
     case LoopKind::Density:
       return iter ? tile16_any<DensityLoop, true>(d, la, ca, ta, tg, d.rd,

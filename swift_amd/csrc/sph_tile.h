@@ -47,7 +47,29 @@ struct TileGhost {
   unsigned long long *counters;  // launch_ghost's: [0] not converged,
                                  // [3..] density interactions
   unsigned int *rounds;          // largest number of density evaluations
+  // 1: the first evaluation is done already, its raw sums are in the fields
+  // (the density tasks or bundles before a ghost task)
+  int given;
 };
+
+// The particles of a tile: lane g + 16 s of the wave holds the field slot
+// and record slot of particle g (act: it takes part).
+struct TileParts {
+  int cell;
+  bool act;
+  int i, ic;
+};
+__device__ __forceinline__ TileParts queue_parts(const DevParts &d,
+                                                 const TileArgs &tq, int tile) {
+  const int g = threadIdx.x & 15;
+  const int ts = uniform(tq.tile_start[tile]);
+  TileParts t;
+  t.act = g < uniform(tq.tile_start[tile + 1]) - ts;
+  t.cell = uniform(tq.tile_cell[tile]);
+  t.i = t.act ? tq.alist[ts + g] : 0;
+  t.ic = t.act ? rec_slot(d, t.i) : -1;
+  return t;
+}
 
 template <class L, int CJ>
 struct TileLds {
@@ -87,12 +109,12 @@ __device__ __forceinline__ int div_magic(int n, int d, unsigned int magic) {
   return n - q * d >= d ? q + 1 : q;
 }
 
-// One tile of the work queue.
+// One tile; slot spreads the density work over the counters.
 template <class L, int CJ, bool ITER>
 __device__ __forceinline__ void run_tile(
     const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
-    const TileArgs &tq, int tile, const TileGhost &tg) {
+    const TileParts &tp, const TileGhost &tg, int slot) {
   using Sh = TileLds<L, CJ>;
   using Rec = typename L::Rec;
   constexpr int RPC = Sh::RPC, CHUNKS = Sh::CHUNKS;
@@ -101,12 +123,9 @@ __device__ __forceinline__ void run_tile(
   __shared__ Sh sh;
   const int lane = threadIdx.x & 63;
   const int g = lane & 15, s = lane >> 4;
-  const int ts = uniform(tq.tile_start[tile]);
-  const int cnt_i = uniform(tq.tile_start[tile + 1]) - ts;
-  const int cell_i = uniform(tq.tile_cell[tile]);
-  const bool act = g < cnt_i;
-  const int i = act ? tq.alist[ts + g] : 0;
-  const int ic = act ? rec_slot(d, i) : -1;  // record slot
+  const int cell_i = tp.cell;
+  const bool act = tp.act;
+  const int i = tp.i, ic = tp.ic;
   typename L::I st{};
   st.x = st.y = st.z = kFar;
   if (act) L::load_i(d, i, st);
@@ -398,13 +417,14 @@ __device__ __forceinline__ void run_tile(
     bool live = act;
     float listed = -1.f;  // squared radius that the lists cover
     // the lists hold every hit of the sweep (one window took it all)
-    bool whole = false, fresh = true;
+    bool whole = false, fresh = true, given = tg.given != 0;
     int work = 0, round = 1;
     L::identity(acc);
+    if (given && act) L::load_acc(d, i, acc);
     wave_sync();
     for (;;) {  // a window, or a walk over lists that still serve
       bool more = false;
-      if (fresh || !whole) {  // uniform
+      if (!given && (fresh || !whole)) {  // uniform
         if (fresh) {
           // room for the next steps' growth: the lists cover 1 % more at
           // the first evaluation and 2 % more later (radius)
@@ -418,7 +438,8 @@ __device__ __forceinline__ void run_tile(
       walk();
       wave_sync();
       if (more) continue;  // uniform
-      L::template combine<4>(acc);
+      if (!given) L::template combine<4>(acc);
+      given = false;
       if (live) {
         // (an opaque copy: the addresses of the particle's fields are formed
         // here and not kept in registers across the walks)
@@ -456,7 +477,7 @@ __device__ __forceinline__ void run_tile(
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) work += __shfl_xor(work, off);
     if (lane == 0) {
-      atomicAdd(&tg.counters[3 + tile % kGhostWorkSlots],
+      atomicAdd(&tg.counters[3 + slot % kGhostWorkSlots],
                 (unsigned long long)work);
       // a plain read first: only a wave that raises the maximum pays an
       // atomic
@@ -476,7 +497,7 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16(
     TileArgs tq, TileGhost tg) {
   const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
   if (t >= *tq.ntiles) return;  // uniform per wave
-  run_tile<L, CJ, ITER>(d, la, ca, rec, pos, tq, t, tg);
+  run_tile<L, CJ, ITER>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
 }
 
 // The tiles beyond a grid of b0 blocks (see k_loop_tiles_rest).
@@ -491,7 +512,7 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_rest(
     const int t = xcd_item(b, threadIdx.x >> 6, n);
     if (t >= n) continue;  // uniform per wave
     wave_sync();
-    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, tq, t, tg);
+    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
   }
 }
 
@@ -503,8 +524,27 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_queue(
     TileArgs tq, TileGhost tg) {
   drain_queue(tq, [&](int t) {
     wave_sync();
-    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, tq, t, tg);
+    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
   });
+}
+
+// runner_do_ghost on one cell after its density tasks: one wave per chunk of
+// 16 of the cell, each taking the chunk's flagged particles of share off of
+// nt (slot counted from the cell's first field slot, as k_ghost).
+template <class L>
+__global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_ghost_cell(
+    DevParts d, LoopArgs la, ChunkArgs ca,
+    const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
+    TileGhost tg, int cell, int off, int nt) {
+  const int lo = la.cell_start[cell], hi = la.cell_start[cell + 1];
+  TileParts t;
+  t.cell = cell;
+  t.ic = lo + 16 * (int)blockIdx.x + (int)(threadIdx.x & 15);
+  t.i = t.ic < hi ? field_slot(d, t.ic) : 0;
+  t.act = t.ic < hi && d.redo[t.i] != 0 && (t.i - lo) % nt == off;
+  if (!__any(t.act)) return;  // uniform
+  if (!t.act) t.ic = -1;
+  run_tile<L, 16, true>(d, la, ca, rec, pos, t, tg, (int)blockIdx.x);
 }
 
 }  // namespace sphl
