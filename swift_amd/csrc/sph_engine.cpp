@@ -356,9 +356,9 @@ void free_dev(swsph_engine *e) {
                   e->d.divv_dt, e->d.ax, e->d.ay, e->d.az, e->d.udt, e->d.hdt,
                   e->d.nf, e->d.mintb, e->d.rd, e->d.rg, e->d.rf, e->d.pos,
                   e->d.r2b, e->d.lfb, e->d.sel, e->d.cell, e->nl.idx,
-                  e->nl.cnt, e->ts.flag, e->ts.scan, e->ts.blk, e->ts.cnt,
-                  e->ts.cscan, e->ts.cblk, e->ts.alist, e->ts.tile_start,
-                  e->ts.tile_cell, e->ts.ntiles, e->ts.heads,
+                  e->nl.cnt, e->ts.cell, e->ts.blk, e->ts.alist, e->ts.nlist,
+                  e->ts.tile_start, e->ts.tile_cell, e->ts.ntiles, e->ts.ids,
+                  e->ts.nids, e->ts.heads,
                   e->d_cell_start, e->d_tiles, e->d.vfx, e->d.vfy, e->d.vfz,
                   e->d.ufull, e->d.perm, e->d_key[0], e->d_key[1],
                   e->d_val[0], e->d_val[1], e->d_sort_tmp, e->d_stage,
@@ -659,19 +659,18 @@ int alloc_dev(swsph_engine *e, size_t n) {
   {
     TileScratch &t = e->ts;
     const size_t nc = (size_t)e->ncells;
-    HIPCHK(dalloc(&t.flag, n));
-    HIPCHK(dalloc(&t.scan, n + 1));
-    HIPCHK(dalloc(&t.blk, n / 1024 + 2));
-    HIPCHK(dalloc(&t.cnt, nc));
-    HIPCHK(dalloc(&t.cscan, nc + 1));
-    HIPCHK(dalloc(&t.cblk, nc / 1024 + 2));
+    HIPCHK(dalloc(&t.cell, nc));
+    HIPCHK(dalloc(&t.blk, nc / kTileCells + 1));
     HIPCHK(dalloc(&t.alist, n));
+    HIPCHK(dalloc(&t.nlist, 1));
     // a cell of k particles makes ceil(k / C) tiles: at most n / C + nc
     // tiles for tiles of C >= kMinTile particles, plus the end marker
     e->tile_cap = n / kMinTile + nc + 1;
     HIPCHK(dalloc(&t.tile_start, e->tile_cap));
     HIPCHK(dalloc(&t.tile_cell, e->tile_cap));
     HIPCHK(dalloc(&t.ntiles, 1));
+    HIPCHK(dalloc(&t.ids, e->tile_cap));
+    HIPCHK(dalloc(&t.nids, 1));
     HIPCHK(dalloc(&t.heads, 8 * 64));
   }
   // binning buffers
@@ -844,10 +843,10 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
   const bool subset = mode == 1 && e->tiles_c == C && C == kMinTile &&
                       !build && !la.cmask;
   if (subset) {
-    ta.ids = e->ts.flag;    // free until the next build (tiles <= particles)
-    ta.ntiles = e->ts.blk;  // the subset's count
+    ta.ids = e->ts.ids;
+    ta.ntiles = e->ts.nids;  // the subset's count
     ta.filt = flag;
-    HIPCHK(sphk::launch_select_tiles(e->ts, flag, e->ts.flag, e->ts.blk,
+    HIPCHK(sphk::launch_select_tiles(e->ts, flag, e->ts.ids, e->ts.nids,
                                      e->st));
     if (e->schedule == 2 || e->capturing)
       HIPCHK(sphk::launch_zero_u32((unsigned int *)e->ts.heads, 8 * 64,
@@ -907,7 +906,7 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
     HIPCHK(sphk::launch_queue(k, build, e->d, la, chunk_args(t), ta, e->nl, C,
                               CJ, persistent, e->queue_waves, max_tiles, rest,
                               e->st));
-  e->launches += 13;
+  e->launches += 4;
   return time_end(e, k, a);
 }
 
@@ -1564,7 +1563,7 @@ const int *queue_list(const swsph_engine *e, const int **cnt) {
     *cnt = nullptr;
     return nullptr;
   }
-  *cnt = e->ts.scan + e->n;
+  *cnt = e->ts.nlist;
   return e->ts.alist;
 }
 
@@ -1883,10 +1882,10 @@ int select_particles(swsph_engine *e, int mode, const int *flag,
                      const int **list, const int **cnt) {
   HIPCHK(sphk::launch_build_tiles(e->d, loop_args(e), (int)e->n, e->ncells,
                                   16, mode, flag, e->ts, e->st));
-  e->launches += 12;
+  e->launches += 3;
   e->tiles_c = 0;
   *list = e->ts.alist;
-  *cnt = e->ts.scan + e->n;
+  *cnt = e->ts.nlist;
   return 0;
 }
 

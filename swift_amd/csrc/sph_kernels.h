@@ -271,17 +271,18 @@ struct StepArgs {
 };
 
 // Scratch of the tile builder, sized for n particles and ncells cells.
+// Cells per block of the builder's per-cell kernels (one wave each).
+constexpr int kTileCells = 16;
 struct TileScratch {
-  int *flag;        // [n]
-  int *scan;        // [n + 1]
-  int *blk;         // [n / 1024 + 2]
-  int *cnt;         // [ncells]
-  int *cscan;       // [ncells + 1]
-  int *cblk;        // [ncells / 1024 + 2]
-  int *alist;       // [n]
+  unsigned long long *cell;  // [ncells] selected particles << 32 | tiles
+  unsigned long long *blk;   // [ncells / kTileCells + 1] their block sums
+  int *alist;       // [n] the selected particles, in cell order
+  int *nlist;       // [1] their number
   int *tile_start;  // [n / C + ncells + 1] for the smallest C in use
   int *tile_cell;
   int *ntiles;      // [1]
+  int *ids;         // [as tile_start] a subset of the tiles
+  int *nids;        // [1]
   int *heads;       // [8 * 64]
 };
 namespace sphk {

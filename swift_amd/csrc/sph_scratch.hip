@@ -1,9 +1,9 @@
 // sph_scratch.hip -- the fixed device scratch of the allocation-free batched
 // pass (swsph_pass_batched_noalloc).
 //
-// The per-pass scratch of the batched pass -- the work queue (particle
-// flags, the scans, the compact particle list, the tile table, its count
-// and the per-XCD queue heads) and the ghost / interaction counters -- is
+// The per-pass scratch of the batched pass -- the work queue (the cells'
+// counts, the compact particle list, the tile table, its count and the
+// per-XCD queue heads) and the ghost / interaction counters -- is
 // carved from one file-scope device array instead of engine allocations.
 // Every process that loads the library holds the array on each GPU it uses
 // until it exits.  The array's name is only a host-side handle: host code
@@ -23,16 +23,12 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // noalloc_scratch carves them.
 constexpr size_t scratch_bytes(size_t n, size_t nc) {
   const size_t tcap = n / kMinTile + nc + 1;
-  return align256(4 * n)                   // flag
-         + align256(4 * (n + 1))           // scan
-         + align256(4 * (n / 1024 + 2))    // blk
-         + align256(4 * nc)                // cnt
-         + align256(4 * (nc + 1))          // cscan
-         + align256(4 * (nc / 1024 + 2))   // cblk
-         + align256(4 * n)                 // alist
-         + 2 * align256(4 * tcap)          // tile_start, tile_cell
-         + align256(4)                     // ntiles
-         + align256(4 * 8 * 64)            // heads
+  return align256(8 * nc)                         // cell
+         + align256(8 * (nc / kTileCells + 1))    // blk
+         + align256(4 * n)                        // alist
+         + 3 * align256(4 * tcap)                 // tile_start, _cell, ids
+         + 3 * align256(4)                        // nlist, ntiles, nids
+         + align256(4 * 8 * 64)                   // heads
          + align256(8 * kGhostCounters)    // ghost counters
          + align256(8 * 3);                // interaction counters
 }
@@ -46,7 +42,7 @@ void *g_ptr[kMaxDevices] = {};
 
 }  // namespace
 
-// The scratch itself (about 30 MB for the limits in sph_kernels.h).
+// The scratch itself (about 16 MB for the limits in sph_kernels.h).
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace sphk {
@@ -90,16 +86,15 @@ hipError_t noalloc_scratch(int device, int64_t n, int ncells, TileScratch *ts,
     off += align256(bytes);
     return p;
   };
-  ts->flag = (int *)take(4 * nn);
-  ts->scan = (int *)take(4 * (nn + 1));
-  ts->blk = (int *)take(4 * (nn / 1024 + 2));
-  ts->cnt = (int *)take(4 * nc);
-  ts->cscan = (int *)take(4 * (nc + 1));
-  ts->cblk = (int *)take(4 * (nc / 1024 + 2));
+  ts->cell = (unsigned long long *)take(8 * nc);
+  ts->blk = (unsigned long long *)take(8 * (nc / kTileCells + 1));
   ts->alist = (int *)take(4 * nn);
   ts->tile_start = (int *)take(4 * tcap);
   ts->tile_cell = (int *)take(4 * tcap);
+  ts->ids = (int *)take(4 * tcap);
+  ts->nlist = (int *)take(4);
   ts->ntiles = (int *)take(4);
+  ts->nids = (int *)take(4);
   ts->heads = (int *)take(4 * 8 * 64);
   *redo = (unsigned long long *)take(8 * kGhostCounters);
   *cnt = (unsigned long long *)take(8 * 3);
