@@ -212,20 +212,21 @@ __device__ __forceinline__ void build_records(const DevParts &d, R *dst,
         for_runs(lo, hi, d.tb, one);
       return;
     }
-    // kRuns runs of the block's width; a run whose 64 particles of a wave
+    // kRuns runs a grid's width apart; a run whose 64 particles of a wave
     // are all active is staged in the wave's LDS and stored as contiguous
     // words, otherwise the active ones store their records one by one
     const int lane = threadIdx.x & 63;
     W *mine = buf + (threadIdx.x >> 6) * 64 * Q;
-    const int base = lo + blockIdx.x * kRecBlock * kRuns + threadIdx.x;
+    const int base = lo + blockIdx.x * kRecBlock + threadIdx.x;
+    const int stride = gridDim.x * kRecBlock;
     int8_t t[kRuns];
 #pragma unroll
     for (int u = 0; u < kRuns; u++) {
-      const int i = base + u * kRecBlock;
+      const int i = base + u * stride;
       t[u] = i < hi ? d.tb[i] : (int8_t)kBinInhibited;
     }
     for (int u = 0; u < kRuns; u++) {
-      const int i = base + u * kRecBlock;
+      const int i = base + u * stride;
       const bool act = i < hi && is_active(t[u], mab);
       if (__ballot(act) == ~0ull) {  // uniform over the wave
         const R r = make(i);
@@ -337,10 +338,10 @@ __device__ bool ghost_one(const DevParts &d, const GhostArgs &ga, int i,
 }
 
 // Counts are reduced over the block first: one atomic per block and
-// counter keeps the same-address traffic small.  A block covers kRuns runs
-// of kGhostBlock particles (their redo flags loaded together); the
-// particles that go again are appended to d.sel in block, wave, run, lane
-// order.
+// counter keeps the same-address traffic small.  A block covers kRuns runs of
+// kGhostBlock particles a grid's width apart (their redo flags loaded
+// together); the particles that go again are appended to d.sel in block,
+// wave, run, lane order.
 constexpr int kGhostBlock = 256;
 __global__ __launch_bounds__(kGhostBlock) void k_ghost(
     DevParts d, GhostArgs ga, int lo, int hi, int off, int nt,
@@ -349,20 +350,21 @@ __global__ __launch_bounds__(kGhostBlock) void k_ghost(
   __shared__ int wcnt[3][W];
   __shared__ unsigned long long wwork[W];
   __shared__ int base;
-  // run u of this thread: particle slot i0 + u * kGhostBlock, or with a
-  // compact list the particle of list entry k0 + u * kGhostBlock
-  const int i0 = lo + blockIdx.x * kGhostBlock * kRuns + threadIdx.x;
-  const int k0 = blockIdx.x * kGhostBlock * kRuns + threadIdx.x;
+  // run u of this thread: particle slot i0 + u * stride, or with a compact
+  // list the particle of list entry k0 + u * stride
+  const int i0 = lo + blockIdx.x * kGhostBlock + threadIdx.x;
+  const int k0 = blockIdx.x * kGhostBlock + threadIdx.x;
+  const int stride = gridDim.x * kGhostBlock;
   const int nl = list ? *cnt : 0;
   int idx[kRuns], redo[kRuns];
 #pragma unroll
   for (int u = 0; u < kRuns; u++) {
     if (list) {
-      const int k = k0 + u * kGhostBlock;
+      const int k = k0 + u * stride;
       idx[u] = k < nl ? list[k] : -1;
     } else {
       // share off of nt of the slots (runner_do_ghost's offset / ntasks)
-      const int i = i0 + u * kGhostBlock;
+      const int i = i0 + u * stride;
       idx[u] = (i < hi && (nt == 1 || (i - lo) % nt == off)) ? i : -1;
     }
   }
@@ -606,18 +608,18 @@ __global__ void k_count(DevParts d, int n, int max_active_bin,
   __shared__ unsigned long long part[3][4];
   unsigned long long a = 0, b = 0, c = 0;
   // kRuns time bins in flight per thread and sweep
-  const int stride = gridDim.x * blockDim.x * kRuns;
-  for (int i0 = blockIdx.x * blockDim.x * kRuns + threadIdx.x; i0 < n;
-       i0 += stride) {
+  const int stride = gridDim.x * blockDim.x;
+  for (int i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < n;
+       i0 += stride * kRuns) {
     int8_t t[kRuns];
 #pragma unroll
     for (int u = 0; u < kRuns; u++) {
-      const int i = i0 + u * (int)blockDim.x;
+      const int i = i0 + u * stride;
       t[u] = i < n ? d.tb[i] : kBinInhibited;
     }
 #pragma unroll
     for (int u = 0; u < kRuns; u++) {
-      const int i = i0 + u * (int)blockDim.x;
+      const int i = i0 + u * stride;
       if (i < n && is_active(t[u], max_active_bin)) {
         a += (unsigned)d.nd[i];
         b += (unsigned)d.ng[i];
@@ -663,13 +665,13 @@ __global__ void k_count_active(const int8_t *__restrict__ tb, int n,
                                int max_active_bin, unsigned int *out) {
   __shared__ unsigned int part[4];
   unsigned int c = 0;
-  const int stride = gridDim.x * blockDim.x * kRuns;
-  for (int i0 = blockIdx.x * blockDim.x * kRuns + threadIdx.x; i0 < n;
-       i0 += stride) {
+  const int stride = gridDim.x * blockDim.x;
+  for (int i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < n;
+       i0 += stride * kRuns) {
     int8_t t[kRuns];
 #pragma unroll
     for (int u = 0; u < kRuns; u++) {
-      const int i = i0 + u * (int)blockDim.x;
+      const int i = i0 + u * stride;
       t[u] = i < n ? tb[i] : kBinInhibited;
     }
 #pragma unroll

@@ -43,8 +43,8 @@ namespace {
 
 constexpr int kBlock = 256;
 // Grid cap of the kernels that reduce into one counter: a grid-stride loop
-// over the particles, one atomic per block.
-constexpr int kReduceBlocks = 4096;
+// over the particles, one atomic per block (1024 blocks fill the chip).
+constexpr int kReduceBlocks = 1024;
 constexpr long long kMaxNrTimesteps = 1LL << (kNumTimeBins + 1);
 constexpr int kNeighbourMaxDeltaBin = 2;  // time_bin_neighbour_max_delta_bin
 
@@ -455,7 +455,12 @@ __global__ __launch_bounds__(kBlock) void k_timestep(DevParts d, StepArgs a,
   if (threadIdx.x == 0) {
     long long m = red[0];
     for (int k = 1; k < kBlock / 64; k++) m = red[k] < m ? red[k] : m;
-    atomicMin(ti_end_min, (unsigned long long)m);
+    // a plain read first: only a block that lowers the minimum pays an
+    // atomic
+    if ((unsigned long long)m <
+        __hip_atomic_load(ti_end_min, __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(ti_end_min, (unsigned long long)m);
     if (nact) atomicAdd(err + 1, (unsigned int)nact);
   }
 }
