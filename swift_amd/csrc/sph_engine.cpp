@@ -806,19 +806,27 @@ TileArgs tile_args(const swsph_engine *e) {
   return ta;
 }
 
-// The density tiles iterate the smoothing lengths themselves (sph_tile.h):
-// one launch instead of a round of ghost, tile build and density each.
-bool iterates(const swsph_engine *e) {
-  return e->schedule >= 1 && !e->use_lists &&
-         e->loop_c[(int)LoopKind::Density] == 16;
+// Loop k of a batched pass runs in tiles of 16, which finish their particles
+// themselves (sph_tile.h).
+bool finishes(const swsph_engine *e, LoopKind k) {
+  return e->schedule >= 1 && !e->use_lists && e->loop_c[(int)k] == 16;
 }
+// The density tiles iterate the smoothing lengths: one launch instead of a
+// round of ghost, tile build and density each.
+bool iterates(const swsph_engine *e) {
+  return finishes(e, LoopKind::Density);
+}
+
+// Waves of a captured grid that may find no tile (each exits at once: a few
+// thousand cost under 2 us).
+constexpr int kSpareTiles = 4096;
 
 // A batched loop through the work queue: tiles of the particles selected by
 // `mode` (0 active, 1 active and flagged, 2 flagged without a usable
 // neighbour list), drained by persistent waves; `build` rebuilds the lists
 // of the selected particles while doing their density.
 int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
-               bool build, const GhostArgs *iter = nullptr,
+               bool build, const GhostArgs *fin = nullptr,
                bool given = false) {
   int rc = 0;
   const int C = build ? kListChunk : e->loop_c[(int)k];
@@ -882,10 +890,14 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
     // tiles, whose re-runs of a dense box hold most tiles again, they take
     // the same grid (surplus waves exit at once); narrow tiles' re-runs,
     // often a few tiles, are drained by the persistent grid.
+    // A grid for the largest possible count that has few waves to spare
+    // needs no grid behind it (4-12 us each on a small box).
     const auto it = e->cap_tiles.find(C);
     if (it != e->cap_tiles.end() && (mode == 0 || C > kMinTile)) {
-      max_tiles = std::min(max_tiles, it->second);
-      rest = true;
+      if (max_tiles - it->second > kSpareTiles) {
+        max_tiles = std::min(max_tiles, it->second);
+        rest = true;
+      }
     } else if (mode != 0) {
       persistent = true;
     }
@@ -898,8 +910,8 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
                                persistent, e->queue_waves, max_tiles, rest,
                                e->st));
   else if ((max_tiles > 0 || rest) && C == 16 && !build)
-    HIPCHK(sphk::launch_tile16(k, iter != nullptr, given, e->d, la,
-                               chunk_args(t), ta, iter ? *iter : GhostArgs{},
+    HIPCHK(sphk::launch_tile16(k, fin != nullptr, given, e->d, la,
+                               chunk_args(t), ta, fin ? *fin : GhostArgs{},
                                e->props.max_iter, e->d_redo, persistent,
                                e->queue_waves, max_tiles, rest, e->st));
   else if (max_tiles > 0 || rest)
@@ -1609,41 +1621,50 @@ int phase_finish(swsph_engine *e) {
   // the active ones' gradient records were written by the ghost as each
   // particle converged
   if ((rc = refresh_bounds(e, 0, e->ncells))) return rc;
+  // The extra ghost resets no force sums (the force loop starts its own).
+  // With tiles of 16 it ends the gradient tiles and writes the force records;
+  // with the narrow tiles of sparse activity its own sweep writes them;
+  // otherwise (most particles active) the builder's wave-staged contiguous
+  // stores are faster than one scattered 96-byte record per thread.
+  GhostArgs gx = ghost_args(e);
+  gx.fresh_force = 1;
+  const bool fin_g = finishes(e, LoopKind::Gradient);
+  const bool narrow =
+      e->schedule >= 1 && e->loop_c[(int)LoopKind::Force] == kMinTile;
+  gx.force_rec = fin_g || narrow ? 1 : 0;
   if (e->use_lists) {
     if ((rc = list_loop(e, LoopKind::Gradient, false, 0))) return rc;
     if (e->list_fallback > 0 &&
         (rc = queue ? queue_loop(e, LoopKind::Gradient, 1, e->d.lfb, false)
                     : stencil(e, LoopKind::Gradient, true, e->d.lfb)))
       return rc;
-  } else if ((rc = queue ? queue_loop(e, LoopKind::Gradient, 0, nullptr, false)
+  } else if ((rc = queue ? queue_loop(e, LoopKind::Gradient, 0, nullptr, false,
+                                      fin_g ? &gx : nullptr)
                          : stencil(e, LoopKind::Gradient, false))) {
     return rc;
   }
   // after the gradient loop the queue's list holds all active particles
   const int *cnt;
   const int *list = queue_list(e, &cnt);
-  GhostArgs gx = ghost_args(e);
-  gx.fresh_force = 1;
-  // With the narrow tiles of sparse activity the extra ghost writes the
-  // active force records as it goes; otherwise (most particles active) the
-  // builder's wave-staged contiguous stores are faster than one scattered
-  // 96-byte record per thread.
-  const bool narrow = e->schedule >= 1 &&
-                      e->loop_c[(int)LoopKind::Force] == kMinTile;
-  gx.force_rec = narrow ? 1 : 0;
-  HIPCHK(sphk::launch_extra_ghost(e->d, gx, 0, n, e->st, list, cnt));
-  e->launches++;
-  if (!narrow) {
-    HIPCHK(sphk::launch_build_records(LoopKind::Force, e->d, 0, n, e->st,
-                                      e->props.max_active_bin, list, cnt));
+  if (!fin_g) {
+    HIPCHK(sphk::launch_extra_ghost(e->d, gx, 0, n, e->st, list, cnt));
     e->launches++;
+    if (!gx.force_rec) {
+      HIPCHK(sphk::launch_build_records(LoopKind::Force, e->d, 0, n, e->st,
+                                        e->props.max_active_bin, list, cnt));
+      e->launches++;
+    }
   }
-  if ((rc = queue ? queue_loop(e, LoopKind::Force, 0, nullptr, false)
+  const bool fin_f = finishes(e, LoopKind::Force);
+  if ((rc = queue ? queue_loop(e, LoopKind::Force, 0, nullptr, false,
+                               fin_f ? &gx : nullptr)
                   : stencil(e, LoopKind::Force, false)))
     return rc;
-  HIPCHK(sphk::launch_end_force(e->d, 0, n, e->props.max_active_bin, e->st,
-                                list, cnt));
-  e->launches++;
+  if (!fin_f) {
+    HIPCHK(sphk::launch_end_force(e->d, 0, n, e->props.max_active_bin, e->st,
+                                  list, cnt));
+    e->launches++;
+  }
   return 0;
 }
 

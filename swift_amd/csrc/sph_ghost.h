@@ -1,5 +1,5 @@
-// sph_ghost.h -- the per-particle arithmetic of the ghost, shared by the
-// ghost kernel and by the density tiles that iterate the smoothing lengths
+// sph_ghost.h -- the per-particle arithmetic of the ghosts and of the end of
+// the force loop, shared by their kernels and by the tiles that do it
 // themselves (sph_tile.h).  Contraction is off, so that both round alike.
 #pragma once
 
@@ -143,6 +143,77 @@ __device__ __forceinline__ void ghost_finish(const DevParts &d,
   d.avmax[i] = alpha;
   d.lapu[i] = 0.f;
   d.ng[i] = 0;
+}
+
+// runner_do_extra_ghost (runner_ghost.c:1016-1111) on one active particle
+// whose gradient sums the caller holds: hydro_end_gradient,
+// hydro_prepare_force (hydro.h:840-954, a = 1), hydro_reset_acceleration and
+// timestep_limiter_prepare_force.
+__device__ __forceinline__ void extra_ghost_one(const DevParts &d,
+                                                const GhostArgs &ga, int i,
+                                                int8_t tb, float vsig,
+                                                float lapu_sum, float avmax) {
+#pragma clang fp contract(off)
+  const float h = d.h[i];
+  const float h_inv = 1.0f / h;
+  const float hid1 = h_inv * h_inv * h_inv * h_inv;
+  const float lapu = lapu_sum * (2.f * hid1);
+  d.lapu[i] = lapu;
+  const float dt_alpha =
+      tb <= 0 ? 0.f : (float)((double)(1LL << (tb + 1)) * ga.time_base);
+  const float ksp = h * kGamma;
+  const float ksp_inv = 1.f / ksp;
+  const float rho = d.rho[i];
+  const float u = d.u[i];
+  const float P = kGasGm1 * u * rho;
+  const float c = sqrtf(kGasGamma * P / rho);
+  const float sct_inv = c * ksp_inv;
+  const float divv = d.divv[i];
+  const float div_v_dt =
+      dt_alpha == 0.f ? 0.f : (divv - d.divv_prev[i]) / dt_alpha;
+  const float S = divv < 0.f ? ksp * ksp * fmaxf(0.f, -div_v_dt) : 0.f;
+  const float alpha_loc = ga.alpha_max * S / (c * c + S);
+  float alpha = d.alpha[i];
+  if (alpha_loc > alpha) {
+    alpha = alpha_loc;
+  } else {
+    const float tr = dt_alpha * sct_inv * ga.visc_length;
+    alpha += alpha_loc * tr;
+    alpha /= (1.f + tr);
+  }
+  alpha = fmaxf(alpha, ga.alpha_min);
+  d.alpha[i] = alpha;
+  d.divv_prev[i] = divv;
+  d.divv_dt[i] = div_v_dt;
+  const float dtpi = vsig * ksp_inv;
+  const float sqrt_u_inv = 1.f / sqrtf(u);
+  float adt = ga.diff_beta * ksp * lapu * sqrt_u_inv;
+  const float ad0 = d.adiff[i];
+  adt -= (ad0 - ga.diff_alpha_min) * dtpi;
+  float na = ad0 + adt * dt_alpha;
+  na = fmaxf(na, ga.diff_alpha_min);
+  const float lim = ga.diff_alpha_max * (1.f - avmax / ga.alpha_max);
+  const float adiff = fminf(na, lim);
+  d.adiff[i] = adiff;
+  // the force record, built here from the values at hand
+  if (ga.force_rec)
+    d.rf[rec_slot(d, i)] =
+        force_rec_of(d, i, tb, h, rho, P, c, alpha, adiff, u);
+  if (ga.fresh_force) return;
+  d.ax[i] = 0.f;
+  d.ay[i] = 0.f;
+  d.az[i] = 0.f;
+  d.udt[i] = 0.f;
+  d.hdt[i] = 0.f;
+  d.nf[i] = 0;
+  d.mintb[i] = (int8_t)(kNumTimeBins + 1);
+}
+
+// runner_do_end_hydro_force (runner_others.c:815-870) -> hydro_end_force on
+// the h_dt sum of one particle.
+__device__ __forceinline__ float end_force_hdt(float hdt, float h) {
+#pragma clang fp contract(off)
+  return hdt * (h * kDimInv);
 }
 
 }  // namespace sphl

@@ -322,12 +322,13 @@ hipError_t launch_queue(LoopKind kind, bool build_lists, const DevParts &d,
                         bool persistent, int waves, int max_tiles, bool rest,
                         hipStream_t st);
 // The tiles of 16 particles (sph_tile.h) against chunks of ca.C = 8, 16 or
-// 32; grids as launch_queue.  `iter` (density only): the tiles iterate the
-// smoothing lengths to convergence and finish their particles as the ghost
-// does with ga; counters as launch_ghost's plus [kGhostRounds], all zeroed
-// by the caller.  `given`: the sums of the first evaluation are in the
-// particles' fields already.
-hipError_t launch_tile16(LoopKind kind, bool iter, bool given,
+// 32; grids as launch_queue.  `fin`: the tiles also finish their particles
+// with ga -- density: they iterate the smoothing lengths to convergence and
+// end as the ghost does (counters as launch_ghost's plus [kGhostRounds], all
+// zeroed by the caller; `given`: the sums of the first evaluation are in the
+// particles' fields already); gradient: the extra ghost; force: the end of
+// the force loop.
+hipError_t launch_tile16(LoopKind kind, bool fin, bool given,
                          const DevParts &d, const LoopArgs &la,
                          const ChunkArgs &ca, const TileArgs &ta,
                          const GhostArgs &ga, int max_iter,

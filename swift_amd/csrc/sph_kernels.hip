@@ -433,65 +433,12 @@ __global__ void k_fill_f32(float *p, float v, int n) {
   if (i < n) p[i] = v;
 }
 
-// runner_do_extra_ghost (runner_ghost.c:1016-1111): hydro_end_gradient,
-// hydro_prepare_force (hydro.h:840-954, a = 1), hydro_reset_acceleration and
-// timestep_limiter_prepare_force for active particles in [lo, hi).
+// runner_do_extra_ghost for the active particles in [lo, hi) or of the list.
 __global__ void k_extra_ghost(DevParts d, GhostArgs ga, int lo, int hi,
                               const int *list, const int *cnt) {
   auto body = [&](int i, int8_t tb) {
     if (!is_active(tb, ga.max_active_bin)) return;
-    const float h = d.h[i];
-    const float h_inv = 1.0f / h;
-    const float hid1 = h_inv * h_inv * h_inv * h_inv;
-    const float lapu = d.lapu[i] * (2.f * hid1);
-    d.lapu[i] = lapu;
-    const float dt_alpha =
-        tb <= 0 ? 0.f : (float)((double)(1LL << (tb + 1)) * ga.time_base);
-    const float ksp = h * kGamma;
-    const float ksp_inv = 1.f / ksp;
-    const float vsig = d.vsig[i];
-    const float rho = d.rho[i];
-    const float P = kGasGm1 * d.u[i] * rho;
-    const float c = sqrtf(kGasGamma * P / rho);
-    const float sct_inv = c * ksp_inv;
-    const float divv = d.divv[i];
-    const float div_v_dt =
-        dt_alpha == 0.f ? 0.f : (divv - d.divv_prev[i]) / dt_alpha;
-    const float S = divv < 0.f ? ksp * ksp * fmaxf(0.f, -div_v_dt) : 0.f;
-    const float alpha_loc = ga.alpha_max * S / (c * c + S);
-    float alpha = d.alpha[i];
-    if (alpha_loc > alpha) {
-      alpha = alpha_loc;
-    } else {
-      const float tr = dt_alpha * sct_inv * ga.visc_length;
-      alpha += alpha_loc * tr;
-      alpha /= (1.f + tr);
-    }
-    alpha = fmaxf(alpha, ga.alpha_min);
-    d.alpha[i] = alpha;
-    d.divv_prev[i] = divv;
-    d.divv_dt[i] = div_v_dt;
-    const float dtpi = vsig * ksp_inv;
-    const float sqrt_u_inv = 1.f / sqrtf(d.u[i]);
-    float adt = ga.diff_beta * ksp * lapu * sqrt_u_inv;
-    const float ad0 = d.adiff[i];
-    adt -= (ad0 - ga.diff_alpha_min) * dtpi;
-    float na = ad0 + adt * dt_alpha;
-    na = fmaxf(na, ga.diff_alpha_min);
-    const float lim = ga.diff_alpha_max * (1.f - d.avmax[i] / ga.alpha_max);
-    d.adiff[i] = fminf(na, lim);
-    // the force record, built here from the values at hand
-    if (ga.force_rec)
-      d.rf[rec_slot(d, i)] = force_rec_of(d, i, tb, h, rho, P, c, alpha,
-                                          fminf(na, lim), d.u[i]);
-    if (ga.fresh_force) return;
-    d.ax[i] = 0.f;
-    d.ay[i] = 0.f;
-    d.az[i] = 0.f;
-    d.udt[i] = 0.f;
-    d.hdt[i] = 0.f;
-    d.nf[i] = 0;
-    d.mintb[i] = (int8_t)(kNumTimeBins + 1);
+    extra_ghost_one(d, ga, i, tb, d.vsig[i], d.lapu[i], d.avmax[i]);
   };
   if (list)
     for_runs_list(list, cnt, d.tb, body);
@@ -499,11 +446,12 @@ __global__ void k_extra_ghost(DevParts d, GhostArgs ga, int lo, int hi,
     for_runs(lo, hi, d.tb, body);
 }
 
-// runner_do_end_hydro_force (runner_others.c:815-870) -> hydro_end_force.
+// runner_do_end_hydro_force for the active particles.
 __global__ void k_end_force(DevParts d, int lo, int hi, int max_active_bin,
                             const int *list, const int *cnt) {
   auto body = [&](int i, int8_t tb) {
-    if (is_active(tb, max_active_bin)) d.hdt[i] *= d.h[i] * kDimInv;
+    if (is_active(tb, max_active_bin))
+      d.hdt[i] = end_force_hdt(d.hdt[i], d.h[i]);
   };
   if (list)
     for_runs_list(list, cnt, d.tb, body);
@@ -1044,7 +992,7 @@ hipError_t launch_queue(LoopKind kind, bool build_lists, const DevParts &d,
   return hipErrorInvalidValue;
 }
 
-template <class L, int CJ, bool ITER>
+template <class L, int CJ, bool FIN>
 static int tile16_resident_blocks() {
   static std::atomic<int> cached{0};
   if (cached.load() == 0) {
@@ -1053,7 +1001,7 @@ static int tile16_resident_blocks() {
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount,
                               dev) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, k_tile16_queue<L, CJ, ITER>, 64, 0) != hipSuccess ||
+            &per, k_tile16_queue<L, CJ, FIN>, 64, 0) != hipSuccess ||
         per <= 0)
       return 0;
     cached.store(ncu * per);
@@ -1061,7 +1009,7 @@ static int tile16_resident_blocks() {
   return cached.load();
 }
 
-template <class L, int CJ, bool ITER>
+template <class L, int CJ, bool FIN>
 hipError_t tile16_c(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
                     const TileArgs &ta, const TileGhost &tg,
                     const typename L::Rec *rec, bool persistent, int waves,
@@ -1070,29 +1018,29 @@ hipError_t tile16_c(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
   if (!persistent) {
     const int nb = max_tiles > 0 ? xcd_blocks(max_tiles) : 0;
     if (nb > 0)
-      hipLaunchKernelGGL((k_tile16<L, CJ, ITER>), dim3(nb), dim3(64), 0, st, d,
+      hipLaunchKernelGGL((k_tile16<L, CJ, FIN>), dim3(nb), dim3(64), 0, st, d,
                          la, ca, rec, pos, ta, tg);
     if (rest)
-      hipLaunchKernelGGL((k_tile16_rest<L, CJ, ITER>), dim3(kRestBlocks),
+      hipLaunchKernelGGL((k_tile16_rest<L, CJ, FIN>), dim3(kRestBlocks),
                          dim3(64), 0, st, d, la, ca, rec, pos, ta, tg, nb);
     return hipGetLastError();
   }
-  if (waves <= 0) waves = tile16_resident_blocks<L, CJ, ITER>();
+  if (waves <= 0) waves = tile16_resident_blocks<L, CJ, FIN>();
   if (waves <= 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_tile16_queue<L, CJ, ITER>), dim3(waves), dim3(64), 0,
+  hipLaunchKernelGGL((k_tile16_queue<L, CJ, FIN>), dim3(waves), dim3(64), 0,
                      st, d, la, ca, rec, pos, ta, tg);
   return hipGetLastError();
 }
 
-template <class L, bool ITER>
+template <class L, bool FIN>
 hipError_t tile16_any(const DevParts &d, const LoopArgs &la,
                       const ChunkArgs &ca, const TileArgs &ta,
                       const TileGhost &tg, const typename L::Rec *rec, bool p,
                       int waves, int mt, bool rest, hipStream_t st) {
   switch (ca.C) {
-    case 8: return tile16_c<L, 8, ITER>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
-    case 16: return tile16_c<L, 16, ITER>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
-    case 32: return tile16_c<L, 32, ITER>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
+    case 8: return tile16_c<L, 8, FIN>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
+    case 16: return tile16_c<L, 16, FIN>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
+    case 32: return tile16_c<L, 32, FIN>(d, la, ca, ta, tg, rec, p, waves, mt, rest, st);
   }
   return hipErrorInvalidValue;
 }
@@ -1112,7 +1060,7 @@ hipError_t launch_ghost_cell(const DevParts &d, const LoopArgs &la,
   return hipGetLastError();
 }
 
-hipError_t launch_tile16(LoopKind kind, bool iter, bool given,
+hipError_t launch_tile16(LoopKind kind, bool fin, bool given,
                          const DevParts &d, const LoopArgs &la,
                          const ChunkArgs &ca, const TileArgs &ta,
                          const GhostArgs &ga, int max_iter,
@@ -1121,21 +1069,17 @@ hipError_t launch_tile16(LoopKind kind, bool iter, bool given,
   if (!ca.fbox || !la.fresh || ta.ids || ta.filt) return hipErrorInvalidValue;
   const TileGhost tg{ga, max_iter, counters,
                      (unsigned int *)(counters + kGhostRounds), given ? 1 : 0};
+  auto run = [&](auto loop, const auto *rec) {
+    using L = decltype(loop);
+    return fin ? tile16_any<L, true>(d, la, ca, ta, tg, rec, persistent, waves,
+                                     max_tiles, rest, st)
+               : tile16_any<L, false>(d, la, ca, ta, tg, rec, persistent,
+                                      waves, max_tiles, rest, st);
+  };
   switch (kind) {
-    case LoopKind::Density:
-      return iter ? tile16_any<DensityLoop, true>(d, la, ca, ta, tg, d.rd,
-                                                  persistent, waves, max_tiles,
-                                                  rest, st)
-                  : tile16_any<DensityLoop, false>(d, la, ca, ta, tg, d.rd,
-                                                   persistent, waves,
-                                                   max_tiles, rest, st);
-    case LoopKind::Gradient:
-      return tile16_any<GradientLoop, false>(d, la, ca, ta, tg, d.rg,
-                                             persistent, waves, max_tiles,
-                                             rest, st);
-    case LoopKind::Force:
-      return tile16_any<ForceLoop, false>(d, la, ca, ta, tg, d.rf, persistent,
-                                          waves, max_tiles, rest, st);
+    case LoopKind::Density: return run(DensityLoop{}, d.rd);
+    case LoopKind::Gradient: return run(GradientLoop{}, d.rg);
+    case LoopKind::Force: return run(ForceLoop{}, d.rf);
   }
   return hipErrorInvalidValue;
 }

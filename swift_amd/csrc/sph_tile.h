@@ -24,7 +24,11 @@
 // (the FP16 rows took 7), and the pipelined walk has one load latency per
 // hit instead of three.
 //
-// The density form can iterate the smoothing lengths itself (ITER): the wave
+// With FIN the tiles also finish their particles, which saves the sweeps over
+// them that would follow (a launch each and their fields read back): the
+// gradient form ends with the extra ghost and the force record, the force
+// form with the end of the force loop.
+// The density form then iterates the smoothing lengths itself: the wave
 // holds the finished sums of its particles after the walk, takes their
 // Newton step (sph_ghost.h) and goes on with the particles that are not done
 // -- on the same lists while their radius is inside the one the lists were
@@ -40,7 +44,7 @@ namespace sphl {
 constexpr int kTileRows = 256;    // rows of 4 candidates in a window
 constexpr int kTileHits = 44;     // hits of a lane between two walks
 
-// What the iterating density form needs beside the loop's arguments.
+// What the finishing forms need beside the loop's arguments.
 struct TileGhost {
   GhostArgs ga;
   int max_iter;
@@ -110,7 +114,7 @@ __device__ __forceinline__ int div_magic(int n, int d, unsigned int magic) {
 }
 
 // One tile; slot spreads the density work over the counters.
-template <class L, int CJ, bool ITER>
+template <class L, int CJ, bool FIN>
 __device__ __forceinline__ void run_tile(
     const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
@@ -119,7 +123,7 @@ __device__ __forceinline__ void run_tile(
   using Rec = typename L::Rec;
   constexpr int RPC = Sh::RPC, CHUNKS = Sh::CHUNKS;
   constexpr int G = 64 / CJ;  // chunks staged together
-  static_assert(!ITER || !L::kSymmetric, "the density loop iterates");
+  constexpr bool ITER = FIN && std::is_same<L, DensityLoop>::value;
   __shared__ Sh sh;
   const int lane = threadIdx.x & 63;
   const int g = lane & 15, s = lane >> 4;
@@ -408,7 +412,22 @@ __device__ __forceinline__ void run_tile(
       wave_sync();
     } while (more);  // uniform
     L::template combine<4>(acc);
-    if (act && s == 0) L::store_acc(d, i, acc);
+    if (act && s == 0) {
+      // (an opaque copy: the addresses of the particle's fields are formed
+      // here and not kept in registers across the walks)
+      int iw = i;
+      asm volatile("" : "+v"(iw));
+      if constexpr (FIN && std::is_same<L, GradientLoop>::value) {
+        d.vsig[iw] = acc.vsig;
+        d.avmax[iw] = acc.avmax;
+        d.ng[iw] = acc.n;
+        extra_ghost_one(d, tg.ga, iw, d.tb[iw], acc.vsig, acc.lapu, acc.avmax);
+      } else {
+        if constexpr (FIN && std::is_same<L, ForceLoop>::value)
+          acc.hdt = end_force_hdt(acc.hdt, d.h[iw]);
+        L::store_acc(d, iw, acc);
+      }
+    }
   } else {
     // The particle's iteration; every lane of a particle holds its whole
     // sums after the combination and takes the same step.
@@ -490,18 +509,18 @@ __device__ __forceinline__ void run_tile(
 }
 
 // One wave per tile over a grid sized for the tile count (see k_loop_tiles).
-template <class L, int CJ, bool ITER>
+template <class L, int CJ, bool FIN>
 __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, TileGhost tg) {
   const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
   if (t >= *tq.ntiles) return;  // uniform per wave
-  run_tile<L, CJ, ITER>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
+  run_tile<L, CJ, FIN>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
 }
 
 // The tiles beyond a grid of b0 blocks (see k_loop_tiles_rest).
-template <class L, int CJ, bool ITER>
+template <class L, int CJ, bool FIN>
 __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_rest(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
@@ -512,19 +531,19 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_rest(
     const int t = xcd_item(b, threadIdx.x >> 6, n);
     if (t >= n) continue;  // uniform per wave
     wave_sync();
-    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
+    run_tile<L, CJ, FIN>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
   }
 }
 
 // Persistent form (see k_loop_queue).
-template <class L, int CJ, bool ITER>
+template <class L, int CJ, bool FIN>
 __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_queue(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, TileGhost tg) {
   drain_queue(tq, [&](int t) {
     wave_sync();
-    run_tile<L, CJ, ITER>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
+    run_tile<L, CJ, FIN>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
   });
 }
 
