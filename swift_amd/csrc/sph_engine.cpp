@@ -216,6 +216,9 @@ struct swsph_engine {
   // the uploaded cell list, and whether the mask is in force; the cells
   // holding active particles (swsph_sched_pass).
   unsigned char *d_cmask = nullptr, *d_cact = nullptr;
+  unsigned int *d_images = nullptr;  // image masks of a bundle's cells
+  int *d_tasks = nullptr;            // its tasks
+  size_t cap_tasks = 0;
   int *d_clist = nullptr;
   int cmask_cap = 0;
   bool cmask_on = false;
@@ -363,7 +366,7 @@ void free_dev(swsph_engine *e) {
                   e->d.ufull, e->d.perm, e->d_key[0], e->d_key[1],
                   e->d_val[0], e->d_val[1], e->d_sort_tmp, e->d_stage,
                   e->d_subflag, e->d_inv, e->d_subind, e->d_suberr,
-                  e->d_cmask, e->d_cact, e->d_clist, e->d_cand_buf,
+                  e->d_cmask, e->d_cact, e->d_clist, e->d_images, e->d_cand_buf,
                   e->d_soa_buf, e->d_moved};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -375,6 +378,7 @@ void free_dev(swsph_engine *e) {
   e->inv_gen = 0;
   e->d_cmask = e->d_cact = nullptr;
   e->d_clist = nullptr;
+  e->d_images = nullptr;
   e->cmask_cap = 0;
   e->cmask_on = false;
   e->d = DevParts{};
@@ -803,6 +807,7 @@ TileArgs tile_args(const swsph_engine *e) {
   ta.heads = e->ts.heads;
   ta.ids = nullptr;
   ta.filt = nullptr;
+  ta.images = nullptr;
   return ta;
 }
 
@@ -872,8 +877,11 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
   if (!e->capturing && e->schedule == 1) {
     // Eager: one wave per tile of the device-side count (a grid for the
     // largest possible count would mostly be waves that exit at once), read
-    // once per table.
-    if (subset || e->tiles_n < 0) {
+    // once per table; a small grid takes the largest possible count (the
+    // read and its wait cost 15-20 us).
+    if (!subset && max_tiles <= kSpareTiles) {
+      e->tiles_n = max_tiles;
+    } else if (subset || e->tiles_n < 0) {
       HIPCHK(hipMemcpyAsync(e->h_ntiles, ta.ntiles, sizeof(int),
                             hipMemcpyDeviceToHost, e->st));
       HIPCHK(hipStreamSynchronize(e->st));
@@ -1861,6 +1869,24 @@ bool field_view(const DevParts &d, int field, FieldView &v) {
   }
 }
 // ---- bundles of cell tasks (ghost, extra ghost, end force, init) --------
+// The per-cell masks of a bundle.
+int ensure_cell_masks(swsph_engine *e) {
+  if (e->d_cmask && e->cmask_cap >= e->ncells) return 0;
+  for (void *p : {(void *)e->d_cmask, (void *)e->d_cact, (void *)e->d_clist,
+                  (void *)e->d_images})
+    if (p) (void)hipFree(p);
+  e->d_cmask = e->d_cact = nullptr;
+  e->d_clist = nullptr;
+  e->d_images = nullptr;
+  e->cmask_cap = 0;
+  HIPCHK(dalloc(&e->d_cmask, (size_t)e->ncells));
+  HIPCHK(dalloc(&e->d_cact, (size_t)e->ncells));
+  HIPCHK(dalloc(&e->d_clist, (size_t)e->ncells));
+  HIPCHK(dalloc(&e->d_images, (size_t)e->ncells + 1));
+  e->cmask_cap = e->ncells;
+  return 0;
+}
+
 // The cells of a bundle as the device mask that the work-queue selections
 // read, until clear_cells.
 int select_cells(swsph_engine *e, const int *cells, int n) {
@@ -1868,17 +1894,7 @@ int select_cells(swsph_engine *e, const int *cells, int n) {
   if (n > e->ncells) return fail(1, "%d cells listed, %d exist", n, e->ncells);
   for (int k = 0; k < n; k++)
     if (int rc = cell_ok(e, cells[k])) return rc;
-  if (!e->d_cmask || e->cmask_cap < e->ncells) {
-    for (void *p : {(void *)e->d_cmask, (void *)e->d_cact, (void *)e->d_clist})
-      if (p) (void)hipFree(p);
-    e->d_cmask = e->d_cact = nullptr;
-    e->d_clist = nullptr;
-    e->cmask_cap = 0;
-    HIPCHK(dalloc(&e->d_cmask, (size_t)e->ncells));
-    HIPCHK(dalloc(&e->d_cact, (size_t)e->ncells));
-    HIPCHK(dalloc(&e->d_clist, (size_t)e->ncells));
-    e->cmask_cap = e->ncells;
-  }
+  if (int rc = ensure_cell_masks(e)) return rc;
   if (n > 0)
     HIPCHK(hipMemcpyAsync(e->d_clist, cells, sizeof(int) * (size_t)n,
                           hipMemcpyHostToDevice, e->st));
@@ -2010,6 +2026,67 @@ int cell_op_locked(swsph_engine *e, const int *cells, int n, bool extra) {
   return rc;
 }
 
+// A large bundle through the work queue: its tasks become a mask of stencil
+// images per cell on the device, and tiles of 16 of the active particles of
+// the cells they touch meet those images.  *done = false (and nothing done)
+// if a task is not valid: the caller says which.
+int run_tasks_tiles(swsph_engine *e, int loop, const swsph_task *tasks,
+                    int ntasks, bool *done) {
+  static_assert(sizeof(swsph_task) == 3 * sizeof(int) &&
+                    SWSPH_TASK_SELF == kTaskSelf &&
+                    SWSPH_TASK_PAIR == kTaskPair,
+                "tasks are {type, ci, cj}");
+  int rc = 0;
+  *done = false;
+  if ((rc = ensure_cell_masks(e))) return rc;
+  if ((size_t)ntasks > e->cap_tasks) {
+    if (e->d_tasks) (void)hipFree(e->d_tasks);
+    e->d_tasks = nullptr;
+    e->cap_tasks = 0;
+    HIPCHK(dalloc(&e->d_tasks, 3 * (size_t)ntasks));
+    e->cap_tasks = ntasks;
+  }
+  HIPCHK(hipMemcpyAsync(e->d_tasks, tasks, sizeof(swsph_task) * (size_t)ntasks,
+                        hipMemcpyHostToDevice, e->st));
+  HIPCHK(sphk::launch_task_images(e->d_tasks, ntasks, e->grid, e->ncells,
+                                  e->d_images, e->d_cmask, e->st));
+  HIPCHK(hipMemcpyAsync(e->h_small, e->d_images + e->ncells,
+                        sizeof(unsigned int), hipMemcpyDeviceToHost, e->st));
+  HIPCHK(hipStreamSynchronize(e->st));
+  e->launches += 2;
+  if (e->h_small[0]) return 0;
+  if ((rc = ensure_records(e))) return rc;
+  const swsph_engine::ChunkTable *t = chunk_table(e, e->loop_cj[loop], &rc);
+  if (!t) return rc;
+  LoopArgs la = loop_args(e);  // the sums go on from the particles' fields
+  la.cmask = e->d_cmask;
+  TileArgs ta = tile_args(e);
+  ta.images = e->d_images;
+  e->tiles_c = 0;
+  HIPCHK(sphk::launch_build_tiles(e->d, la, (int)e->n, e->ncells, 16, 0,
+                                  nullptr, e->ts, e->st));
+  int max_tiles = (int)(e->n / 16) + e->ncells + 1;
+  if (max_tiles > kSpareTiles) {
+    HIPCHK(hipMemcpyAsync(e->h_ntiles, ta.ntiles, sizeof(int),
+                          hipMemcpyDeviceToHost, e->st));
+    HIPCHK(hipStreamSynchronize(e->st));
+    max_tiles = *e->h_ntiles;
+  }
+  HIPCHK(sphk::launch_tile16((LoopKind)loop, false, false, e->d, la,
+                             chunk_args(t), ta, GhostArgs{}, 0, e->d_redo,
+                             false, 0, max_tiles, false, e->st));
+  e->launches += 4;
+  *done = true;
+  return 0;
+}
+
+// From this many tasks on a bundle of a loop with tiles of 16 goes through
+// the work queue.  The host merges a task in about 37 ns, the device path
+// costs some 25 us more in launches and waits, whatever the size: even at
+// about 700 tasks.  (All 14000 tasks of a loop on 10^3 cells of 64 particles:
+// merging on the host took 500 us for a kernel of 50.)
+constexpr int kTileBundle = 1024;
+
 // A bundle of released self / pair tasks of one loop (swsph_run_tasks).
 int run_tasks_locked(swsph_engine *e, int loop, const swsph_task *tasks,
                      int ntasks) {
@@ -2019,6 +2096,11 @@ int run_tasks_locked(swsph_engine *e, int loop, const swsph_task *tasks,
   if (ntasks == 0) return 0;
   if (e->need_particles) return fail(1, "no particles for the current grid");
   const LoopKind k = (LoopKind)loop;
+  if (ntasks >= kTileBundle && e->n > 0 && e->loop_c[loop] == 16) {
+    bool done = false;
+    const int rc = run_tasks_tiles(e, loop, tasks, ntasks, &done);
+    if (rc || done) return rc;
+  }
   // Per i-cell, bit o of the stencil images it meets (o = 9 (ox + 1) +
   // 3 (oy + 1) + (oz + 1) for the offset of the image's cell), and the
   // i-cells in the order the tasks first touch them.
@@ -2075,7 +2157,9 @@ int run_tasks_locked(swsph_engine *e, int loop, const swsph_task *tasks,
     if (!whole) {
       int a[3];
       coords(c, a);
-      for (int o = 0; o < 27; o++) {
+      for (int p = 0; p < 27; p++) {
+        // (in the order of the 27-cell stencil, as the work queue's tiles)
+        const int o = p == 0 ? 13 : ((p & 1) ? p >> 1 : 27 - (p >> 1));
         if (!(mask[c] >> o & 1u)) continue;
         const int d[3] = {o / 9 - 1, (o / 3) % 3 - 1, o % 3 - 1};
         BundleNbr bn{};
@@ -2283,6 +2367,7 @@ int swsph_engine_destroy(swsph_engine *e) {
   if (e->d_tiend) (void)hipFree(e->d_tiend);
   if (e->d_err) (void)hipFree(e->d_err);
   if (e->d_bitems) (void)hipFree(e->d_bitems);
+  if (e->d_tasks) (void)hipFree(e->d_tasks);
   if (e->d_bnbrs) (void)hipFree(e->d_bnbrs);
   if (e->h_small) (void)hipHostFree(e->h_small);
   if (e->h_tiend) (void)hipHostFree(e->h_tiend);

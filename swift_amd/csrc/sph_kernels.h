@@ -76,6 +76,10 @@ struct TileArgs {
   // particles with filt[i] != 0 take part (null: every tile, particle).
   const int *ids;
   const int *filt;
+  // Stencil images that the particles of each cell meet (bit o: the cell at
+  // offset code o = 9 (ox + 1) + 3 (oy + 1) + (oz + 1)); null: all 27.
+  // Tiles of 16 only.
+  const unsigned int *images;
 };
 
 // Structure-of-arrays particle store in HBM, sorted by top-level cell.
@@ -223,6 +227,7 @@ struct BundleArgs {
   int nitems;
 };
 
+constexpr int kTaskSelf = 0, kTaskPair = 1;
 struct GhostArgs {
   float eta_dim, eps, h_max, h_min;
   int max_active_bin;
@@ -431,6 +436,12 @@ hipError_t launch_ghost(const DevParts &d, const GhostArgs &ga, int lo, int hi,
                         unsigned long long *counters, hipStream_t st,
                         const int *list = nullptr, const int *cnt = nullptr,
                         int off = 0, int nt = 1);
+// The tasks of a bundle as image masks (TileArgs::images) and the mask of
+// the cells they touch; images has ncells + 1 words, the last one != 0 after
+// the launch if a task is not valid or meets a cell pair twice.
+hipError_t launch_task_images(const int *tasks, int ntasks, GridDesc grid,
+                              int ncells, unsigned int *images,
+                              unsigned char *cmask, hipStream_t st);
 // The per-particle kernels below take either the particle range [lo, hi)
 // or (list != nullptr) the particles list[0 .. *cnt) of a compact list whose
 // capacity is hi - lo.

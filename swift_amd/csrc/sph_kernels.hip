@@ -433,6 +433,50 @@ __global__ void k_fill_f32(float *p, float v, int n) {
   if (i < n) p[i] = v;
 }
 
+// Clears the image masks, their error word and the cell mask.
+__global__ void k_task_clear(unsigned int *images, unsigned char *cmask,
+                             int ncells) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c <= ncells) images[c] = 0u;
+  if (c < ncells) cmask[c] = 0;
+}
+
+// One thread per task {type, ci, cj}: sets the image bits of its directed
+// interactions.  A task that swsph_run_tasks refuses sets the error word.
+__global__ void k_task_images(const int *__restrict__ tasks, int ntasks,
+                              GridDesc grid, int ncells, unsigned int *images,
+                              unsigned char *cmask) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= ntasks) return;
+  const int type = tasks[3 * n], ci = tasks[3 * n + 1];
+  const int cj = type == kTaskSelf ? ci : tasks[3 * n + 2];
+  bool ok = ci >= 0 && ci < ncells && cj >= 0 && cj < ncells &&
+            (type == kTaskSelf ||
+             (type == kTaskPair && ci != cj));
+  int o = 0;
+  if (ok) {
+    int a[3], b[3];
+    cell_coords(ci, grid, a[0], a[1], a[2]);
+    cell_coords(cj, grid, b[0], b[1], b[2]);
+    for (int k = 0; k < 3; k++) {
+      int dd = b[k] - a[k];
+      dd = dd > 1 ? dd - grid.nc[k] : (dd < -1 ? dd + grid.nc[k] : dd);
+      ok = ok && dd >= -1 && dd <= 1;
+      o = 3 * o + dd + 1;
+    }
+  }
+  if (ok) {
+    const unsigned int bi = 1u << o, bj = 1u << (26 - o);
+    ok = !(atomicOr(&images[ci], bi) & bi);
+    cmask[ci] = 1;
+    if (type == kTaskPair) {
+      ok = !(atomicOr(&images[cj], bj) & bj) && ok;
+      cmask[cj] = 1;
+    }
+  }
+  if (!ok) atomicOr(&images[ncells], 1u);
+}
+
 // runner_do_extra_ghost for the active particles in [lo, hi) or of the list.
 __global__ void k_extra_ghost(DevParts d, GhostArgs ga, int lo, int hi,
                               const int *list, const int *cnt) {
@@ -1066,7 +1110,8 @@ hipError_t launch_tile16(LoopKind kind, bool fin, bool given,
                          const GhostArgs &ga, int max_iter,
                          unsigned long long *counters, bool persistent,
                          int waves, int max_tiles, bool rest, hipStream_t st) {
-  if (!ca.fbox || !la.fresh || ta.ids || ta.filt) return hipErrorInvalidValue;
+  if (!ca.fbox || (fin && !la.fresh) || ta.ids || ta.filt)
+    return hipErrorInvalidValue;
   const TileGhost tg{ga, max_iter, counters,
                      (unsigned int *)(counters + kGhostRounds), given ? 1 : 0};
   auto run = [&](auto loop, const auto *rec) {
@@ -1417,6 +1462,16 @@ hipError_t launch_ghost(const DevParts &d, const GhostArgs &ga, int lo, int hi,
     hipLaunchKernelGGL(k_ghost, dim3(run_blocks(hi - lo, kGhostBlock)),
                        dim3(kGhostBlock), 0, st, d, ga, lo, hi, off, nt,
                        counters, list, cnt);
+  return hipGetLastError();
+}
+
+hipError_t launch_task_images(const int *tasks, int ntasks, GridDesc grid,
+                              int ncells, unsigned int *images,
+                              unsigned char *cmask, hipStream_t st) {
+  hipLaunchKernelGGL(k_task_clear, dim3(nblk(ncells + 1, 256)), dim3(256), 0,
+                     st, images, cmask, ncells);
+  hipLaunchKernelGGL(k_task_images, dim3(nblk(ntasks, 256)), dim3(256), 0, st,
+                     tasks, ntasks, grid, ncells, images, cmask);
   return hipGetLastError();
 }
 

@@ -57,9 +57,12 @@ struct TileGhost {
 };
 
 // The particles of a tile: lane g + 16 s of the wave holds the field slot
-// and record slot of particle g (act: it takes part).
+// and record slot of particle g (act: it takes part); images: the stencil
+// images they meet (TileArgs::images).
+constexpr unsigned int kAllImages = (1u << 27) - 1u;
 struct TileParts {
   int cell;
+  unsigned int images;
   bool act;
   int i, ic;
 };
@@ -70,6 +73,7 @@ __device__ __forceinline__ TileParts queue_parts(const DevParts &d,
   TileParts t;
   t.act = g < uniform(tq.tile_start[tile + 1]) - ts;
   t.cell = uniform(tq.tile_cell[tile]);
+  t.images = tq.images ? tq.images[t.cell] : kAllImages;
   t.i = t.act ? tq.alist[ts + g] : 0;
   t.ic = t.act ? rec_slot(d, t.i) : -1;
   return t;
@@ -193,7 +197,7 @@ __device__ __forceinline__ void run_tile(
     sh.qk0[lane] = k0;
     sh.qj0[lane] = la.cell_start[cj];
     sh.qj1[lane] = la.cell_start[cj + 1];
-    nchq = k1 - k0;
+    nchq = tp.images >> o & 1u ? k1 - k0 : 0;
     double fo[6];
     (void)pair_frame(o3, ci3, v, t, la.w, fo);
     for (int k = 0; k < 6; k++) sh.fo[6 * lane + k] = fo[k];
@@ -402,7 +406,12 @@ __device__ __forceinline__ void run_tile(
 
   if constexpr (!ITER) {
     L::identity(acc);
-    if (act && s == 0) L::fresh_acc(st, acc);
+    if (act && s == 0) {
+      if (la.fresh)
+        L::fresh_acc(st, acc);
+      else
+        L::load_acc(d, i, acc);
+    }
     wave_sync();
     sweep(act ? pretest_radius2(st.hg2, la.pos_eps) : -1.f);
     bool more;
@@ -558,6 +567,7 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_ghost_cell(
   const int lo = la.cell_start[cell], hi = la.cell_start[cell + 1];
   TileParts t;
   t.cell = cell;
+  t.images = kAllImages;
   t.ic = lo + 16 * (int)blockIdx.x + (int)(threadIdx.x & 15);
   t.i = t.ic < hi ? field_slot(d, t.ic) : 0;
   t.act = t.ic < hi && d.redo[t.i] != 0 && (t.i - lo) % nt == off;
