@@ -477,12 +477,14 @@ hipError_t launch_build_records(LoopKind kind, const DevParts &d, int lo,
 // ---- binning and time integration (sph_step.hip) ----
 // Keys (cell << 30 | in-cell Morton code) of n positions, component k of
 // particle i at p_k[stride * i]; val[i] = i.  With tb (the particles' time
-// bins, same index), (cell << 30 + kBinBits) | (bin << 30) | Morton.
+// bins, same index), (cell << 30 + kBinBits) | (bin << 30) | Morton; *mixed
+// (zeroed by the caller) = 1 if the bins differ.
 constexpr int kBinBits = 6;
 hipError_t launch_bin_keys(const double *px, const double *py, const double *pz,
                            int stride, const GridDesc &g, const double inv_w[3],
                            int n, unsigned long long *key, int *val,
-                           hipStream_t st, const int8_t *tb = nullptr);
+                           hipStream_t st, const int8_t *tb = nullptr,
+                           unsigned int *mixed = nullptr);
 // Stable radix sort of (key, value) pairs on the low `bits` key bits; with
 // temp == nullptr only sets `bytes` (rocprim::radix_sort_pairs).
 hipError_t sort_pairs(void *temp, size_t &bytes, const unsigned long long *kin,
@@ -500,9 +502,34 @@ template <class T>
 hipError_t launch_gather(T *dst, const T *src, int stride, int comp,
                          const int *idx, int n, hipStream_t st);
 // dst[stride * idx[k] + comp] = src[k]
-template <class T>
-hipError_t launch_scatter(T *dst, const T *src, int stride, int comp,
-                          const int *idx, int n, hipStream_t st);
+// The caller's arrays of a new particle set (device copies, caller's order):
+// positions and velocities, the scalars in LoadArgs order (null: the
+// default), the time bins.
+struct LoadArgs {
+  enum { M, U, H, RHO, P, C, F, BAL, ALPHA, ADIFF, DIVV_PREV, N };
+  const double *x;
+  const float *v;
+  const float *src[N];
+  const int8_t *tb;
+  unsigned int *dmax;  // zeroed
+};
+// Every field of the particle slots 0..n-1 from them, slot k being particle
+// d.perm[k]; all other fields zero, no neighbour lists.
+hipError_t launch_load_parts(const DevParts &d, const LoadArgs &a, int n,
+                             hipStream_t st);
+// Words of up to kScatterWords field components to the caller's order:
+// dst[stride * idx[k] + comp] = src[k], size 1, 4 or 8 bytes.
+constexpr int kScatterWords = 24;
+struct ScatterSet {
+  struct W {
+    const void *src;
+    void *dst;
+    unsigned char size, stride, comp;
+  } w[kScatterWords];
+  int n;
+};
+hipError_t launch_scatter(const ScatterSet &s, const int *idx, int n,
+                          hipStream_t st);
 hipError_t launch_fill_i8(int8_t *p, int8_t v, int n, hipStream_t st);
 hipError_t launch_drift(const DevParts &d, const DriftArgs &a,
                         unsigned int *dmax, hipStream_t st);

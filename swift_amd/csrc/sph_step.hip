@@ -69,7 +69,8 @@ __global__ void k_bin_keys(const double *px, const double *py,
                            const double *pz, int stride, GridDesc g,
                            double iw0, double iw1, double iw2, int n,
                            unsigned long long *key, int *val,
-                           const int8_t *tb, int bin_bits) {
+                           const int8_t *tb, int bin_bits,
+                           unsigned int *mixed) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -93,6 +94,7 @@ __global__ void k_bin_keys(const double *px, const double *py,
   unsigned long long b = 0ull;
   if (bin_bits) {  // inhibited particles (and any bin past the field) last
     const int t = tb[i];
+    if (mixed && t != tb[0]) *mixed = 1u;
     b = (unsigned long long)(t < 0 ? 0 : (t > 63 ? 63 : t));
   }
   key[i] = (cid << (30 + bin_bits)) | (b << 30) | m;
@@ -150,11 +152,79 @@ __global__ void k_gather(T *dst, const T *src, int stride, int comp,
 }
 
 // dst[stride * idx[k] + comp] = src[k]: back to the caller's order.
-template <class T>
-__global__ void k_scatter(T *dst, const T *src, int stride, int comp,
-                          const int *idx, int n) {
+// One thread per particle takes all its words (a launch and a read of the
+// index per word before); the stores of a vector's components lie side by
+// side.  kScatterLoads words are loaded before the first is stored: a store
+// behind every load made the sweep latency-bound (a 2 % active pass over
+// 128^3 particles and its read-back 1867 -> 1917 us).
+constexpr int kScatterLoads = 6;
+__global__ void k_scatter(sphk::ScatterSet s, const int *idx, int n) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) dst[(size_t)stride * idx[k] + comp] = src[k];
+  if (k >= n) return;
+  const size_t i = (size_t)idx[k];
+  for (int q0 = 0; q0 < s.n; q0 += kScatterLoads) {
+    unsigned long long v[kScatterLoads];
+#pragma unroll
+    for (int u = 0; u < kScatterLoads; u++) {
+      if (q0 + u >= s.n) break;  // uniform, as the sizes
+      const sphk::ScatterSet::W &w = s.w[q0 + u];
+      v[u] = w.size == 4   ? ((const unsigned int *)w.src)[k]
+             : w.size == 8 ? ((const unsigned long long *)w.src)[k]
+                           : ((const unsigned char *)w.src)[k];
+    }
+#pragma unroll
+    for (int u = 0; u < kScatterLoads; u++) {
+      if (q0 + u >= s.n) break;
+      const sphk::ScatterSet::W &w = s.w[q0 + u];
+      const size_t o = i * w.stride + w.comp;
+      if (w.size == 4)
+        ((unsigned int *)w.dst)[o] = (unsigned int)v[u];
+      else if (w.size == 8)
+        ((unsigned long long *)w.dst)[o] = v[u];
+      else
+        ((unsigned char *)w.dst)[o] = (unsigned char)v[u];
+    }
+  }
+}
+
+// A new particle set: one sweep writes every field of a slot (46 clears and
+// 19 gathers, a launch each, were most of a small box's upload).
+__global__ void k_load_parts(DevParts d, sphk::LoadArgs a, int n) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0) *a.dmax = 0u;
+  if (k >= n) return;
+  const size_t i = (size_t)d.perm[k];
+  d.px[k] = a.x[3 * i];
+  d.py[k] = a.x[3 * i + 1];
+  d.pz[k] = a.x[3 * i + 2];
+  const float vx = a.v[3 * i], vy = a.v[3 * i + 1], vz = a.v[3 * i + 2];
+  d.vx[k] = d.vfx[k] = vx;
+  d.vy[k] = d.vfy[k] = vy;
+  d.vz[k] = d.vfz[k] = vz;
+  auto get = [&](int q, float dflt) {
+    return a.src[q] ? a.src[q][i] : dflt;  // uniform
+  };
+  d.m[k] = get(sphk::LoadArgs::M, 0.f);
+  d.u[k] = d.ufull[k] = get(sphk::LoadArgs::U, 0.f);
+  d.h[k] = get(sphk::LoadArgs::H, 0.f);
+  d.rho[k] = get(sphk::LoadArgs::RHO, 0.f);
+  d.P[k] = get(sphk::LoadArgs::P, 0.f);
+  d.c[k] = get(sphk::LoadArgs::C, 0.f);
+  d.f[k] = get(sphk::LoadArgs::F, 0.f);
+  d.bal[k] = get(sphk::LoadArgs::BAL, 0.f);
+  d.alpha[k] = get(sphk::LoadArgs::ALPHA, 0.1f);
+  d.adiff[k] = get(sphk::LoadArgs::ADIFF, 0.f);
+  d.divv_prev[k] = get(sphk::LoadArgs::DIVV_PREV, 0.f);
+  d.tb[k] = a.tb[i];
+  // fields never written for inactive particles read as zero
+  d.rho_dh[k] = d.wc[k] = d.wc_dh[k] = d.divv[k] = 0.f;
+  d.rotx[k] = d.roty[k] = d.rotz[k] = 0.f;
+  d.left[k] = d.right[k] = 0.f;
+  d.vsig[k] = d.lapu[k] = d.avmax[k] = d.divv_dt[k] = 0.f;
+  d.ax[k] = d.ay[k] = d.az[k] = d.udt[k] = d.hdt[k] = 0.f;
+  d.nd[k] = d.redo[k] = d.ng[k] = d.nf[k] = d.lfb[k] = d.sel[k] = 0;
+  d.mintb[k] = 0;
+  d.r2b[k] = -1.f;
 }
 
 template <class T>
@@ -472,11 +542,12 @@ namespace sphk {
 hipError_t launch_bin_keys(const double *px, const double *py, const double *pz,
                            int stride, const GridDesc &g, const double inv_w[3],
                            int n, unsigned long long *key, int *val,
-                           hipStream_t st, const int8_t *tb) {
+                           hipStream_t st, const int8_t *tb,
+                           unsigned int *mixed) {
   if (n <= 0) return hipSuccess;
   k_bin_keys<<<blocks(n), kBlock, 0, st>>>(px, py, pz, stride, g, inv_w[0],
                                            inv_w[1], inv_w[2], n, key, val, tb,
-                                           tb ? kBinBits : 0);
+                                           tb ? kBinBits : 0, mixed);
   return hipGetLastError();
 }
 
@@ -520,21 +591,19 @@ template hipError_t launch_gather<int>(int *, const int *, int, int,
 template hipError_t launch_gather<int8_t>(int8_t *, const int8_t *, int, int,
                                           const int *, int, hipStream_t);
 
-template <class T>
-hipError_t launch_scatter(T *dst, const T *src, int stride, int comp,
-                          const int *idx, int n, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  k_scatter<T><<<blocks(n), kBlock, 0, st>>>(dst, src, stride, comp, idx, n);
+hipError_t launch_scatter(const ScatterSet &s, const int *idx, int n,
+                          hipStream_t st) {
+  if (n <= 0 || s.n <= 0) return hipSuccess;
+  k_scatter<<<blocks(n), kBlock, 0, st>>>(s, idx, n);
   return hipGetLastError();
 }
-template hipError_t launch_scatter<double>(double *, const double *, int, int,
-                                           const int *, int, hipStream_t);
-template hipError_t launch_scatter<float>(float *, const float *, int, int,
-                                          const int *, int, hipStream_t);
-template hipError_t launch_scatter<int>(int *, const int *, int, int,
-                                        const int *, int, hipStream_t);
-template hipError_t launch_scatter<int8_t>(int8_t *, const int8_t *, int, int,
-                                           const int *, int, hipStream_t);
+
+hipError_t launch_load_parts(const DevParts &d, const LoadArgs &a, int n,
+                             hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  k_load_parts<<<blocks(n), kBlock, 0, st>>>(d, a, n);
+  return hipGetLastError();
+}
 
 hipError_t launch_fill_i8(int8_t *p, int8_t v, int n, hipStream_t st) {
   if (n <= 0) return hipSuccess;

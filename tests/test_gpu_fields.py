@@ -1,0 +1,81 @@
+"""Upload (swsph_set_particles) and read-back (swsph_get_fields): every field
+in one call against one call per field and against what was uploaded, for
+one particle, an odd number (unaligned parts of the staging buffer), and
+more than a million (sweeps and copies overlap on two streams); mixed and
+uniform time bins (the second key sort is left out), and arrays left out
+(defaults)."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _parts(n, mixed, seed):
+    rng = np.random.default_rng(seed)
+    f = lambda lo, hi: rng.uniform(lo, hi, n).astype(np.float32)
+    return dict(x=rng.uniform(0, 1, (n, 3)), v=rng.normal(size=(n, 3)).astype(
+                    np.float32),
+                m=f(1, 2), u=f(1, 2), h=f(0.01, 0.05), rho=f(1, 2),
+                pressure=f(1, 2), soundspeed=f(1, 2), f=f(-1, 1),
+                balsara=f(0, 1), alpha_visc=f(0, 1), alpha_diff=f(0, 1),
+                div_v_prev=f(-1, 1),
+                time_bin=(rng.integers(1, 30, n) if mixed
+                          else np.full(n, 4)).astype(np.int8))
+
+
+def _get_all(eng, n):
+    from swift_amd import FIELDS, lib
+    names = list(FIELDS)
+    outs = [np.empty((n, 3) if FIELDS[k][2] == 3 else (n,), FIELDS[k][1])
+            for k in names]
+    ids = (C.c_int * len(names))(*[FIELDS[k][0] for k in names])
+    ptr = (C.c_void_p * len(names))(*[o.ctypes.data for o in outs])
+    assert lib().swsph_get_fields(eng._h, len(names), ids, ptr) == 0
+    return dict(zip(names, outs))
+
+
+@pytest.mark.parametrize("n,mixed", [(1, False), (999, True), (999, False),
+                                     ((1 << 20) + 77, True),
+                                     ((1 << 20) + 77, False)])
+def test_upload_and_read_back(n, mixed):
+    from swift_amd import Engine, HydroProps
+    p = _parts(n, mixed, seed=n)
+    with Engine(HydroProps(ncell=(5, 5, 5))) as eng:
+        eng.set_particles(_parts(max(1, n // 2), not mixed, seed=1))  # old data
+        eng.set_particles(p)
+        got = _get_all(eng, n)
+        for k, v in got.items():
+            assert np.array_equal(v, eng.get(k)), k
+    up = dict(p, v_full=p["v"], u_full=p["u"])
+    for k, v in got.items():
+        if k in up:
+            assert np.array_equal(v, up[k]), k
+        else:
+            assert not v.any(), k
+
+
+def test_optional_arrays_and_errors():
+    from swift_amd import Engine, HydroProps, lib
+    from swift_amd.engine import _HostParts
+    p = _parts(999, True, seed=5)
+    hp = _HostParts()
+    hp.n = 999
+    for k in ("x", "v", "m", "u", "h", "time_bin"):
+        setattr(hp, k, p[k].ctypes.data)
+    with Engine(HydroProps(ncell=(5, 5, 5))) as eng:
+        assert lib().swsph_set_particles(eng._h, C.byref(hp)) == 0
+        eng.n = 999
+        got = _get_all(eng, 999)
+        out = np.empty(999, np.float32)
+        ids = (C.c_int * 2)(0, 999)
+        ptr = (C.c_void_p * 2)(out.ctypes.data, out.ctypes.data)
+        assert lib().swsph_get_fields(eng._h, 2, ids, ptr) == 1
+    assert np.array_equal(got["x"], p["x"])
+    assert np.all(got["alpha_visc"] == np.float32(0.1))
+    for k in ("rho", "pressure", "soundspeed", "f", "balsara", "alpha_diff",
+              "div_v_prev"):
+        assert not got[k].any(), k
