@@ -69,8 +69,14 @@ struct swsph_engine {
   int *d_cell_start = nullptr;
   int4 *d_tiles = nullptr;
   int ntiles = 0;
-  unsigned long long *d_redo = nullptr;  // ghost counters (launch_ghost)
-  unsigned long long *h_redo = nullptr;  // pinned readback
+  // What a pass reads back, in one block of kStatusWords words: the ghost
+  // counters (launch_ghost), the interaction counts d_cnt[3], then the two
+  // words d_hg2_all, d_dmax; and its pinned copy.  (The allocation-free pass
+  // puts counters and counts elsewhere.)
+  static constexpr int kStatusWords = kGhostCounters + 3 + 1;
+  unsigned long long *d_status = nullptr, *h_status = nullptr;
+  unsigned long long *d_redo = nullptr;
+  unsigned long long *h_redo = nullptr;
   int64_t density_work = 0;  // density interactions over all rounds
   unsigned long long *d_cnt = nullptr;
   unsigned long long *h_cnt = nullptr;
@@ -112,7 +118,6 @@ struct swsph_engine {
   int loop_c[3] = {16, 16, 16};   // tile (i-chunk) capacity CI per loop
   int loop_cj[3] = {16, 16, 16};  // candidate chunk capacity CJ (work queue)
   unsigned int *d_hg2_all = nullptr;  // max (gamma h)^2 over all chunks
-  unsigned int *h_hg2_all = nullptr;
   // Neighbour lists of the batched pass (allocated on first use).
   bool use_lists = false;
   float list_skin = 1.2f;  // list radius / search radius
@@ -195,7 +200,7 @@ struct swsph_engine {
   size_t cap_bitems = 0, cap_bnbrs = 0;
   unsigned int *d_err = nullptr;          // [3] time-step errors, active,
                                           // active count before a step
-  unsigned int *h_small = nullptr;        // pinned readback: dmax, hg2
+  unsigned int *h_small = nullptr;        // of the readback: hg2, dmax
   unsigned long long *h_tiend = nullptr;  // pinned [1]
   unsigned int *h_err = nullptr;          // pinned [3]
   int *h_ntiles = nullptr;                // pinned [1]
@@ -1044,6 +1049,12 @@ void all_neighbours(const swsph_engine *e, int ci, std::vector<int> &out) {
   }
 }
 
+void sum_work(swsph_engine *e) {
+  int64_t work = 0;  // accumulated on the device, over the slots
+  for (int k = 0; k < kGhostWorkSlots; k++) work += (int64_t)e->h_redo[3 + k];
+  e->density_work = work;
+}
+
 // Ghost counters: [0] particles flagged for another round, [1] of those
 // needing a new neighbour list, [2] converged without a usable list.
 int read_redo(swsph_engine *e, int *count, int *relist = nullptr,
@@ -1055,9 +1066,7 @@ int read_redo(swsph_engine *e, int *count, int *relist = nullptr,
   *count = (int)e->h_redo[0];
   if (relist) *relist = (int)e->h_redo[1];
   if (nolist) *nolist = (int)e->h_redo[2];
-  int64_t work = 0;  // accumulated on the device, over the slots
-  for (int k = 0; k < kGhostWorkSlots; k++) work += (int64_t)e->h_redo[3 + k];
-  e->density_work = work;
+  sum_work(e);
   return 0;
 }
 
@@ -1098,30 +1107,40 @@ int ensure_subset(swsph_engine *e, int count) {
 // the subset re-runs of the share's flagged particles over every density
 // interaction of the cell (runner_ghost.c:1548-1580).  The last share to
 // finish leaves the cell's gradient records and chunk bounds current.
-int ghost_cell(swsph_engine *e, int ci, int *rounds, int off = 0, int nt = 1) {
+// later: the caller clears the counters before its cells and reads them
+// after them (cells whose waves iterate).
+bool ghost_iterates(const swsph_engine *e) {
+  return chunk_c(e, (int)LoopKind::Density) == 16 && !e->use_lists;
+}
+int ghost_cell(swsph_engine *e, int ci, int *rounds, int off = 0, int nt = 1,
+               bool later = false) {
   const int lo = e->cell_start[ci], hi = e->cell_start[ci + 1];
   GhostArgs ga = ghost_args(e);
   int redo = 0;
   int it = 0;
   int rc = 0;
-  if (chunk_c(e, (int)LoopKind::Density) == 16 && !e->use_lists) {
+  if (ghost_iterates(e)) {
     // the cell's waves iterate their particles themselves, the re-runs over
     // the whole stencil at once (27 launches per round otherwise)
     const swsph_engine::ChunkTable *t = chunk_table(e, 16, &rc);
     if (!t) return rc;
     ga.grad_rec = 1;
-    // the work slots accumulate over the ghosts of a pass
-    HIPCHK(sphk::launch_zero_u64(e->d_redo, 3, e->st));
-    HIPCHK(sphk::launch_zero_u64(e->d_redo + kGhostRounds, 1, e->st));
+    if (!later) {
+      // the work slots accumulate over the ghosts of a pass
+      HIPCHK(sphk::launch_zero_ghost(e->d_redo, e->st));
+      e->launches++;
+    }
     HIPCHK(sphk::launch_ghost_cell(
         e->d, loop_args(e), chunk_args(t), ga, e->props.max_iter, e->d_redo,
         ci, t->cell_chunk_h[ci + 1] - t->cell_chunk_h[ci], off, nt, e->st));
-    e->launches += 3;
-    if ((rc = read_redo(e, &redo))) return rc;
-    if (redo > 0)
-      return fail(3, "Smoothing length failed to converge on %d particles",
-                  redo);
-    if (rounds) *rounds = std::max(*rounds, (int)e->h_redo[kGhostRounds]);
+    e->launches++;
+    if (!later) {
+      if ((rc = read_redo(e, &redo))) return rc;
+      if (redo > 0)
+        return fail(3, "Smoothing length failed to converge on %d particles",
+                    redo);
+      if (rounds) *rounds = std::max(*rounds, (int)e->h_redo[kGhostRounds]);
+    }
     return refresh_bounds(e, ci, ci + 1);
   }
   std::vector<int> nb;
@@ -1169,31 +1188,17 @@ int extra_ghost_cell(swsph_engine *e, int c) {
   return 0;
 }
 
-int count_into(swsph_engine *e, swsph_pass_stats *s) {
-  HIPCHK(sphk::launch_count(e->d, (int)e->n, e->props.max_active_bin, e->d_cnt,
-                            e->st));
-  HIPCHK(hipMemcpyAsync(e->h_cnt, e->d_cnt, 3 * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, e->st));
-  HIPCHK(hipStreamSynchronize(e->st));
-  if (s) {
-    s->n_density = (int64_t)e->h_cnt[0];
-    s->n_gradient = (int64_t)e->h_cnt[1];
-    s->n_force = (int64_t)e->h_cnt[2];
-  }
-  return 0;
-}
-
 // Kernel support H (largest over the chunk bounds) and drift distance d
 // (largest distance of a particle outside its cell since the last binning)
 // of the current particles.  Every neighbour lies in the 27-cell stencil
 // while H + 2 d <= the cell width (the reference rebuilds its cells when
 // that fails).
-int read_fit(swsph_engine *e, double *H, double *dm) {
-  HIPCHK(hipMemcpyAsync(e->h_small, e->d_hg2_all, sizeof(unsigned int),
-                        hipMemcpyDeviceToHost, e->st));
-  HIPCHK(hipMemcpyAsync(e->h_small + 1, e->d_dmax, sizeof(unsigned int),
-                        hipMemcpyDeviceToHost, e->st));
-  HIPCHK(hipStreamSynchronize(e->st));
+int read_fit(swsph_engine *e, double *H, double *dm, bool wait = true) {
+  if (wait) {
+    HIPCHK(hipMemcpyAsync(e->h_small, e->d_hg2_all, 2 * sizeof(unsigned int),
+                          hipMemcpyDeviceToHost, e->st));
+    HIPCHK(hipStreamSynchronize(e->st));
+  }
   float hg2, d;
   std::memcpy(&hg2, e->h_small, sizeof(float));
   std::memcpy(&d, e->h_small + 1, sizeof(float));
@@ -1209,9 +1214,10 @@ bool fits(const swsph_engine *e, double H, double dm) {
   return true;
 }
 
-int check_fits(swsph_engine *e) {
+// wait = false: the readback holds them already.
+int check_fits(swsph_engine *e, bool wait = true) {
   double H, dm;
-  int rc = read_fit(e, &H, &dm);
+  int rc = read_fit(e, &H, &dm, wait);
   if (rc) return rc;
   if (!fits(e, H, dm))
     return fail(4,
@@ -1221,9 +1227,29 @@ int check_fits(swsph_engine *e) {
   return 0;
 }
 
-// After a pass: the largest kernel support met by the chunk bounds (and the
-// drift since the last binning) must fit the stencil.
-int check_support(swsph_engine *e) { return check_fits(e); }
+// The end of a pass: the interaction counts (enqueued here unless `counted`:
+// by a captured graph), the ghost counters and what check_fits reads, in one
+// copy and one wait (six copies and three waits cost 50 us).
+int read_status(swsph_engine *e, swsph_pass_stats *s, bool counted = false) {
+  if (!counted)
+    HIPCHK(sphk::launch_count(e->d, (int)e->n, e->props.max_active_bin,
+                              e->d_cnt, e->st));
+  const bool own = e->d_redo == e->d_status;
+  const size_t words = swsph_engine::kStatusWords - (own ? 0 : 1);
+  HIPCHK(hipMemcpyAsync(e->h_status, e->d_redo,
+                        words * sizeof(unsigned long long),
+                        hipMemcpyDeviceToHost, e->st));
+  if (!own)
+    HIPCHK(hipMemcpyAsync(e->h_small, e->d_hg2_all, 2 * sizeof(unsigned int),
+                          hipMemcpyDeviceToHost, e->st));
+  HIPCHK(hipStreamSynchronize(e->st));
+  if (s) {
+    s->n_density = (int64_t)e->h_cnt[0];
+    s->n_gradient = (int64_t)e->h_cnt[1];
+    s->n_force = (int64_t)e->h_cnt[2];
+  }
+  return 0;
+}
 
 int rebin(swsph_engine *e);
 
@@ -1671,30 +1697,41 @@ int phase_finish(swsph_engine *e) {
   return 0;
 }
 
+void fill_stats(swsph_engine *e, swsph_pass_stats *stats, int rounds,
+                int64_t l0) {
+  if (!stats) return;
+  stats->ghost_rounds = rounds;
+  stats->launches = e->launches - l0;
+  stats->list_rebuilt = e->list_rebuilt;
+  stats->list_fallback = e->list_fallback;
+  stats->n_density_all = e->density_work;
+}
+
 int finish_stats(swsph_engine *e, swsph_pass_stats *stats, int rounds,
                  int64_t l0) {
   int rc = 0;
-  if (stats) {
-    stats->ghost_rounds = rounds;
-    stats->launches = e->launches - l0;
-    stats->list_rebuilt = e->list_rebuilt;
-    stats->list_fallback = e->list_fallback;
-    stats->n_density_all = e->density_work;
-  }
-  if ((rc = count_into(e, stats))) return rc;
-  if ((rc = check_support(e))) return rc;
+  fill_stats(e, stats, rounds, l0);
+  if ((rc = read_status(e, stats))) return rc;
+  // the largest kernel support met by the chunk bounds (and the drift since
+  // the last binning) must fit the stencil
+  if ((rc = check_fits(e, false))) return rc;
   return collect_timing(e);
 }
 
 // The end of a pass whose density tiles iterated: their counters are read
 // once the whole pass is enqueued.
-int finish_iterated(swsph_engine *e, swsph_pass_stats *stats, int64_t l0) {
-  int redo = 0;
-  if (int rc = read_redo(e, &redo)) return rc;
-  if (redo > 0)
-    return fail(3, "Smoothing length failed to converge on %d particles", redo);
+int finish_iterated(swsph_engine *e, swsph_pass_stats *stats, int64_t l0,
+                    bool counted = false) {
+  int rc = 0;
+  if ((rc = read_status(e, stats, counted))) return rc;
+  sum_work(e);
+  if (e->h_redo[0] > 0)
+    return fail(3, "Smoothing length failed to converge on %d particles",
+                (int)e->h_redo[0]);
   e->last_rounds = std::max(1, (int)e->h_redo[kGhostRounds]);
-  return finish_stats(e, stats, e->last_rounds, l0);
+  fill_stats(e, stats, e->last_rounds, l0);
+  if ((rc = check_fits(e, false))) return rc;
+  return collect_timing(e);
 }
 
 // Captures the launches of fn on the engine stream into an executable graph.
@@ -1949,10 +1986,8 @@ int ghost_cells_locked(swsph_engine *e, const int *cells, int n, int *rounds) {
     ga.grad_rec = 1;
     int redo = 0;
     // the work slots accumulate over the ghosts of a pass
-    hipError_t err = sphk::launch_zero_u64(e->d_redo, 3, e->st);
-    if (err == hipSuccess)
-      err = sphk::launch_zero_u64(e->d_redo + kGhostRounds, 1, e->st);
-    e->launches += 2;
+    const hipError_t err = sphk::launch_zero_ghost(e->d_redo, e->st);
+    e->launches++;
     if (err != hipSuccess) rc = fail(2, "ghost: %s", hipGetErrorString(err));
     if (!rc)
       rc = queue_loop(e, LoopKind::Density, 1, e->d.redo, false, &ga, true);
@@ -2302,30 +2337,19 @@ int swsph_engine_create(const swsph_props *props, swsph_engine **out) {
     delete e;
     return fail(2, "hipStreamCreate failed");
   }
-  if (hipMalloc((void **)&e->d_redo,
-                kGhostCounters * sizeof(unsigned long long)) !=
-          hipSuccess ||
+  constexpr size_t status_bytes =
+      swsph_engine::kStatusWords * sizeof(unsigned long long);
+  if (hipMalloc((void **)&e->d_status, status_bytes) != hipSuccess ||
+      hipHostMalloc((void **)&e->h_status, status_bytes, 0) != hipSuccess ||
       hipMalloc((void **)&e->d_hist, swsph_engine::kHistRounds *
                                          sizeof(unsigned long long)) !=
           hipSuccess ||
       hipHostMalloc((void **)&e->h_hist, swsph_engine::kHistRounds *
                                              sizeof(unsigned long long),
                     0) != hipSuccess ||
-      hipHostMalloc((void **)&e->h_redo,
-                    kGhostCounters * sizeof(unsigned long long), 0) !=
-          hipSuccess ||
-      hipMalloc((void **)&e->d_cnt, 3 * sizeof(unsigned long long)) != hipSuccess ||
-      hipHostMalloc((void **)&e->h_cnt, 3 * sizeof(unsigned long long), 0) !=
-          hipSuccess ||
-      hipMalloc((void **)&e->d_hg2_all, sizeof(unsigned int)) != hipSuccess ||
-      hipHostMalloc((void **)&e->h_hg2_all, sizeof(unsigned int), 0) !=
-          hipSuccess ||
-      hipMalloc((void **)&e->d_dmax, sizeof(unsigned int)) != hipSuccess ||
       hipMalloc((void **)&e->d_tiend, sizeof(unsigned long long)) !=
           hipSuccess ||
       hipMalloc((void **)&e->d_err, 3 * sizeof(unsigned int)) != hipSuccess ||
-      hipHostMalloc((void **)&e->h_small, 2 * sizeof(unsigned int), 0) !=
-          hipSuccess ||
       hipHostMalloc((void **)&e->h_tiend, sizeof(unsigned long long), 0) !=
           hipSuccess ||
       hipHostMalloc((void **)&e->h_err, 3 * sizeof(unsigned int), 0) !=
@@ -2334,6 +2358,13 @@ int swsph_engine_create(const swsph_props *props, swsph_engine **out) {
     delete e;
     return fail(2, "allocation of engine counters failed");
   }
+  e->d_redo = e->d_status;
+  e->h_redo = e->h_status;
+  e->d_cnt = e->d_redo + kGhostCounters;
+  e->h_cnt = e->h_redo + kGhostCounters;
+  e->d_hg2_all = (unsigned int *)(e->d_cnt + 3);
+  e->d_dmax = e->d_hg2_all + 1;
+  e->h_small = (unsigned int *)(e->h_cnt + 3);
   // SPH:max_volume_change default 1.4 (src/hydro_properties.c:42, 122)
   e->integ.log_max_h_change = logf(powf(1.4f, 0.3333333333f));
   // One table per admissible chunk capacity at most: never reallocated, so
@@ -2350,21 +2381,15 @@ int swsph_engine_destroy(swsph_engine *e) {
   for (hipEvent_t ev : e->ev_pool) (void)hipEventDestroy(ev);
   if (e->g_density) (void)hipGraphExecDestroy(e->g_density);
   if (e->g_finish) (void)hipGraphExecDestroy(e->g_finish);
-  if (e->d_redo) (void)hipFree(e->d_redo);
-  if (e->h_redo) (void)hipHostFree(e->h_redo);
   if (e->d_hist) (void)hipFree(e->d_hist);
   if (e->h_hist) (void)hipHostFree(e->h_hist);
-  if (e->d_cnt) (void)hipFree(e->d_cnt);
-  if (e->d_hg2_all) (void)hipFree(e->d_hg2_all);
-  if (e->h_hg2_all) (void)hipHostFree(e->h_hg2_all);
-  if (e->h_cnt) (void)hipHostFree(e->h_cnt);
-  if (e->d_dmax) (void)hipFree(e->d_dmax);
   if (e->d_tiend) (void)hipFree(e->d_tiend);
   if (e->d_err) (void)hipFree(e->d_err);
   if (e->d_bitems) (void)hipFree(e->d_bitems);
   if (e->d_tasks) (void)hipFree(e->d_tasks);
   if (e->d_bnbrs) (void)hipFree(e->d_bnbrs);
-  if (e->h_small) (void)hipHostFree(e->h_small);
+  if (e->d_status) (void)hipFree(e->d_status);
+  if (e->h_status) (void)hipHostFree(e->h_status);
   if (e->h_tiend) (void)hipHostFree(e->h_tiend);
   if (e->h_err) (void)hipHostFree(e->h_err);
   if (e->h_ntiles) (void)hipHostFree(e->h_ntiles);
@@ -2838,8 +2863,22 @@ int swsph_pass_plain(swsph_engine *e, swsph_pass_stats *stats) {
   };
   if ((rc = loop_tasks(LoopKind::Density))) return rc;
   int rounds = 0;
-  for (int c = 0; c < e->ncells; c++)
-    if ((rc = ghost_cell(e, c, &rounds))) return rc;
+  if (ghost_iterates(e)) {
+    // one wait for all cells
+    int redo = 0;
+    HIPCHK(sphk::launch_zero_ghost(e->d_redo, e->st));
+    e->launches++;
+    for (int c = 0; c < e->ncells; c++)
+      if ((rc = ghost_cell(e, c, nullptr, 0, 1, true))) return rc;
+    if ((rc = read_redo(e, &redo))) return rc;
+    if (redo > 0)
+      return fail(3, "Smoothing length failed to converge on %d particles",
+                  redo);
+    rounds = (int)e->h_redo[kGhostRounds];
+  } else {
+    for (int c = 0; c < e->ncells; c++)
+      if ((rc = ghost_cell(e, c, &rounds))) return rc;
+  }
   if ((rc = loop_tasks(LoopKind::Gradient))) return rc;
   for (int c = 0; c < e->ncells; c++)
     if ((rc = extra_ghost_cell(e, c))) return rc;
@@ -2856,8 +2895,8 @@ int swsph_pass_plain(swsph_engine *e, swsph_pass_stats *stats) {
     stats->list_fallback = 0;
     stats->n_density_all = e->density_work;
   }
-  if ((rc = count_into(e, stats))) return rc;
-  return check_support(e);
+  if ((rc = read_status(e, stats))) return rc;
+  return check_fits(e, false);
 }
 
 
@@ -2980,8 +3019,12 @@ static int pass_graph_locked(swsph_engine *e, swsph_pass_stats *stats) {
     if (iterates(e)) {
       // no rounds to count: the pass is one graph
       if ((rc = capture(e, &e->g_density, [&]() -> int {
-             const int r = phase_start(e);
-             return r ? r : phase_finish(e);
+             int r = phase_start(e);
+             if (r || (r = phase_finish(e))) return r;
+             HIPCHK(sphk::launch_count(e->d, (int)e->n,
+                                       e->props.max_active_bin, e->d_cnt,
+                                       e->st));
+             return 0;
            })))
         return rc;
     } else {
@@ -3001,7 +3044,7 @@ static int pass_graph_locked(swsph_engine *e, swsph_pass_stats *stats) {
     e->graph_reruns = reruns;
   }
   HIPCHK(hipGraphLaunch(e->g_density, e->st));
-  if (iterates(e)) return finish_iterated(e, stats, l0);
+  if (iterates(e)) return finish_iterated(e, stats, l0, true);
   HIPCHK(hipMemcpyAsync(e->h_hist, e->d_hist,
                         (reruns + 1) * sizeof(unsigned long long),
                         hipMemcpyDeviceToHost, e->st));
@@ -3203,7 +3246,7 @@ int swsph_count_interactions(swsph_engine *e, int64_t out3[3]) {
   if (!e || !out3) return fail(1, "null argument");
   std::lock_guard<std::mutex> lk(e->mtx);
   swsph_pass_stats s{};
-  int rc = count_into(e, &s);
+  int rc = read_status(e, &s);
   if (rc) return rc;
   out3[0] = s.n_density;
   out3[1] = s.n_gradient;

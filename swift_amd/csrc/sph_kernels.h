@@ -399,6 +399,8 @@ hipError_t launch_mark_subset(int *flag, const int *inv, long long first,
 hipError_t launch_share_flags(int *dst, const int *src, int lo, int hi,
                               int off, int nt, hipStream_t st);
 hipError_t launch_zero_u64(unsigned long long *p, int n, hipStream_t st);
+// Of launch_ghost's counters, [0..2] and [kGhostRounds].
+hipError_t launch_zero_ghost(unsigned long long *counters, hipStream_t st);
 // Bounding boxes and largest search radius of chunks [c0, c1); the largest
 // search radius over them is max-reduced into *hg2_all (float bits).  With
 // fbox, also the boxes of the chunks' pre-test records (grid g, pos_eps as
@@ -539,8 +541,8 @@ hipError_t launch_timestep(const DevParts &d, const StepArgs &a,
                            hipStream_t st);
 // The fixed scratch of the allocation-free pass (sph_scratch.hip): its size,
 // the one-time lookup of its address on `device` (which must be current),
-// and the work queue and counters of a pass over n particles on ncells
-// cells carved from it (hipErrorInvalidValue beyond the limits above,
+// and the work queue and counters (cnt behind redo) of a pass over n
+// particles on ncells cells carved from it (hipErrorInvalidValue beyond the limits above,
 // hipErrorNotInitialized before noalloc_setup on that device).
 size_t noalloc_scratch_bytes();
 hipError_t noalloc_setup(int device);

@@ -508,6 +508,11 @@ __global__ void k_zero_int(int *p, int n) {
   if (i < n) p[i] = 0;
 }
 
+__global__ void k_zero_ghost(unsigned long long *counters) {
+  const int k = threadIdx.x;
+  if (k < 4) counters[k < 3 ? k : kGhostRounds] = 0ull;
+}
+
 __global__ void k_zero_u64(unsigned long long *p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
@@ -1302,6 +1307,11 @@ hipError_t launch_bundle(LoopKind kind, const DevParts &d, const LoopArgs &la,
       return bundle_any<ForceLoop>(d, la, ca, d.rf, ba, st);
   }
   return hipErrorInvalidValue;
+}
+
+hipError_t launch_zero_ghost(unsigned long long *counters, hipStream_t st) {
+  hipLaunchKernelGGL(k_zero_ghost, dim3(1), dim3(64), 0, st, counters);
+  return hipGetLastError();
 }
 
 hipError_t launch_zero_u64(unsigned long long *p, int n, hipStream_t st) {

@@ -29,8 +29,7 @@ constexpr size_t scratch_bytes(size_t n, size_t nc) {
          + 3 * align256(4 * tcap)                 // tile_start, _cell, ids
          + 3 * align256(4)                        // nlist, ntiles, nids
          + align256(4 * 8 * 64)                   // heads
-         + align256(8 * kGhostCounters)    // ghost counters
-         + align256(8 * 3);                // interaction counters
+         + align256(8 * (kGhostCounters + 3));    // ghost counters, counts
 }
 
 constexpr size_t kScratchBytes =
@@ -96,8 +95,8 @@ hipError_t noalloc_scratch(int device, int64_t n, int ncells, TileScratch *ts,
   ts->ntiles = (int *)take(4);
   ts->nids = (int *)take(4);
   ts->heads = (int *)take(4 * 8 * 64);
-  *redo = (unsigned long long *)take(8 * kGhostCounters);
-  *cnt = (unsigned long long *)take(8 * 3);
+  *redo = (unsigned long long *)take(8 * (kGhostCounters + 3));
+  *cnt = *redo + kGhostCounters;
   if (off != scratch_bytes(nn, nc) || off > kScratchBytes)
     return hipErrorInvalidValue;
   *tile_cap = tcap;
