@@ -1007,7 +1007,17 @@ int task(swsph_engine *e, LoopKind k, bool subset, int ci, int cj, bool both,
   ta.icell[0] = ci;
   ta.jcell[0] = cj;
   ta.ntiles[0] = nch(ci);
-  for (int k2 = 0; k2 < 3; k2++) ta.t[k2] = t[k2];
+  const int *nc = e->grid.nc;
+  const int a3[3] = {ci / (nc[1] * nc[2]), (ci / nc[2]) % nc[1], ci % nc[2]};
+  const int b3[3] = {cj / (nc[1] * nc[2]), (cj / nc[2]) % nc[1], cj % nc[2]};
+  int o = 0;  // offset code of the image
+  for (int k2 = 0; k2 < 3; k2++) {
+    ta.t[k2] = t[k2];
+    const int dd = b3[k2] - a3[k2];
+    o = 3 * o + 1 + (dd > 1 ? -1 : dd < -1 ? 1 : dd);
+  }
+  ta.images[0] = 1u << o;
+  ta.images[1] = 1u << (26 - o);
   if (both && ci != cj) {
     ta.icell[1] = cj;
     ta.jcell[1] = ci;

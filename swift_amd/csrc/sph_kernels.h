@@ -208,6 +208,7 @@ struct TaskArgs {
   int jcell[2];
   int ntiles[2];
   double t[6];
+  unsigned int images[2];  // the j-cell as the i-cell's stencil image
 };
 
 // A bundle of released self / pair tasks, merged per i-chunk: item k runs

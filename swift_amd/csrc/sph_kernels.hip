@@ -1238,7 +1238,13 @@ hipError_t task_any(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
   if (nb <= 0) return hipSuccess;
   switch (ca.C) {
     case 8: task_c<L, SUB, 8>(d, la, ca, rec, ta, nb, st); break;
-    case 16: task_c<L, SUB, 16>(d, la, ca, rec, ta, nb, st); break;
+    case 16:
+      if constexpr (SUB)
+        task_c<L, SUB, 16>(d, la, ca, rec, ta, nb, st);
+      else
+        hipLaunchKernelGGL((k_tile16_task<L>), dim3(nb), dim3(64), 0, st, d,
+                           la, ca, rec, (const PosRec *)d.pos, ta);
+      break;
     case 32: task_c<L, SUB, 32>(d, la, ca, rec, ta, nb, st); break;
     case 64: task_c<L, SUB, 64>(d, la, ca, rec, ta, nb, st); break;
     default: return hipErrorInvalidValue;
