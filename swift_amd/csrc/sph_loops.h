@@ -212,25 +212,39 @@ struct DensityLoop {
       a.n += __shfl_xor(a.n, off);
     }
   }
+  // The same of the sums that a step of the smoothing length reads.
+  template <int S>
+  static __device__ __forceinline__ void combine_count(Acc &a) {
+#pragma unroll
+    for (int off = 64 / S; off < 64; off <<= 1) {
+      a.wc += __shfl_xor(a.wc, off);
+      a.wc_dh += __shfl_xor(a.wc_dh, off);
+      a.n += __shfl_xor(a.n, off);
+    }
+  }
   // Candidate test: r < H_i (DOPAIR1 :1386, DOSELF1 :2396).
   template <class R>
   static __device__ __forceinline__ bool test(float r2, const I &s, const R *) {
     return r2 < s.hg2;
   }
-  // runner_iact_nonsym_density (hydro_iact.h:141-193)
+  // runner_iact_nonsym_density (hydro_iact.h:141-193); full = false: only
+  // the sums that a step of the smoothing length reads (wc, wc_dh, n).
   static __device__ __forceinline__ void interact(float r2, float dx, float dy,
                                                   float dz, const I &s,
-                                                  const Rec &j, Acc &a) {
+                                                  const Rec &j, Acc &a,
+                                                  bool full = true) {
     const float r_inv = r2 > 0.f ? fast_rsq(r2) : 0.f;
     const float r = r2 * r_inv;
     const float ui = r * s.h_inv;
     float wi, wi_dx;
     kernel_deval(ui, wi, wi_dx);
     const float t = fmaf(kDim, wi, ui * wi_dx);
-    a.rho = fmaf(j.m, wi, a.rho);
-    a.rho_dh = fmaf(-j.m, t, a.rho_dh);
     a.wc += wi;
     a.wc_dh -= t;
+    a.n += 1;
+    if (!full) return;  // uniform
+    a.rho = fmaf(j.m, wi, a.rho);
+    a.rho_dh = fmaf(-j.m, t, a.rho_dh);
     const float faci = j.m * wi_dx * r_inv;
     const float dvx = s.vx - j.vx, dvy = s.vy - j.vy, dvz = s.vz - j.vz;
     const float dvdr = fmaf(dvz, dz, fmaf(dvy, dy, dvx * dx));
@@ -238,7 +252,6 @@ struct DensityLoop {
     a.rx = fmaf(faci, fmaf(dvy, dz, -dvz * dy), a.rx);
     a.ry = fmaf(faci, fmaf(dvz, dx, -dvx * dz), a.ry);
     a.rz = fmaf(faci, fmaf(dvx, dy, -dvy * dx), a.rz);
-    a.n += 1;
   }
 };
 

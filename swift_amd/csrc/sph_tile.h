@@ -33,7 +33,12 @@
 // Newton step (sph_ghost.h) and goes on with the particles that are not done
 // -- on the same lists while their radius is inside the one the lists were
 // made with, else from step 1 -- until all have converged.  That replaces a
-// ghost launch, a tile build and a density launch per round.
+// ghost launch, a tile build and a density launch per round.  A step reads 2
+// of the 8 sums, and all are needed at the last h only: after the first an
+// evaluation takes the 2 (a third of the walk's arithmetic and 16 of the record's 40 bytes
+// less) until a particle of the tile is expected to converge, its last step
+// (relative: s) making s^2, the order of the next one, pass the tolerance; a
+// particle found to have converged before that is evaluated once more.
 #pragma once
 
 #include "sph_gather.h"
@@ -223,6 +228,7 @@ __device__ __forceinline__ void run_tile(
 
   typename L::Acc acc;
   int cnt = 0;  // hits in this lane's list
+  bool full = true;  // the walk takes all sums (uniform)
 
   // Step 4: the lists against the exact contract.
   auto eval = [&](unsigned int info, const Rec &r, int j) {
@@ -235,7 +241,12 @@ __device__ __forceinline__ void run_tile(
     const float dz = (float)(st.z - fo[2]) - (float)(r.z - fj[2]);
     const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
     // (the matrix test passes the particle itself)
-    if (L::test(r2, st, &r) && j != ic) L::interact(r2, dx, dy, dz, st, r, acc);
+    if (L::test(r2, st, &r) && j != ic) {
+      if constexpr (ITER)
+        L::interact(r2, dx, dy, dz, st, r, acc, full);
+      else
+        L::interact(r2, dx, dy, dz, st, r, acc);
+    }
   };
   auto walk = [&]() {
     auto locate = [&](int k, unsigned int &info) -> int {
@@ -243,23 +254,33 @@ __device__ __forceinline__ void run_tile(
       info = sh.surv[row / RPC];
       return (int)(info & kRowMask) + (row % RPC) * 4 + s;
     };
+    auto fetch = [&](Rec &r, int j) {
+      if (ITER && !full) {  // uniform: the position is enough
+        const Rec *p = rec + j;
+        r.x = p->x;
+        r.y = p->y;
+        r.z = p->z;
+      } else {
+        r = rec[j];
+      }
+    };
     unsigned int n0 = 0u, n1 = 0u;
     int j0 = 0, j1 = 0;
     Rec r0, r1;
     if (cnt > 0) {
       j0 = locate(0, n0);
-      r0 = rec[j0];
+      fetch(r0, j0);
     }
     for (int k = 0; k < cnt; k += 2) {
       if (k + 1 < cnt) {
         j1 = locate(k + 1, n1);
-        r1 = rec[j1];
+        fetch(r1, j1);
       }
       eval(n0, r0, j0);
       if (k + 1 >= cnt) break;
       if (k + 2 < cnt) {
         j0 = locate(k + 2, n0);
-        r0 = rec[j0];
+        fetch(r0, j0);
       }
       eval(n1, r1, j1);
     }
@@ -443,6 +464,9 @@ __device__ __forceinline__ void run_tile(
     GhostState gs{0.f, 0.f, tg.ga.h_max};
     if (act) gs.h = d.h[i];
     bool live = act;
+    // pend: converged in an evaluation of the step's sums only; want: the
+    // next one should take all
+    bool pend = false, want = false;
     float listed = -1.f;  // squared radius that the lists cover
     // the lists hold every hit of the sweep (one window took it all)
     bool whole = false, fresh = true, given = tg.given != 0;
@@ -466,20 +490,32 @@ __device__ __forceinline__ void run_tile(
       walk();
       wave_sync();
       if (more) continue;  // uniform
-      if (!given) L::template combine<4>(acc);
+      if (!given) {
+        if (full)
+          L::template combine<4>(acc);
+        else
+          L::template combine_count<4>(acc);
+      }
       given = false;
       if (live) {
         // (an opaque copy: the addresses of the particle's fields are formed
         // here and not kept in registers across the walks)
         int iw = i;
         asm volatile("" : "+v"(iw));
-        work += acc.n;
+        if (!pend) work += acc.n;
         DensSums a{acc.rho, acc.rho_dh, acc.wc, acc.wc_dh,
                    acc.divv, acc.rx, acc.ry, acc.rz};
+        const GhostState old = gs;
         const bool again = ghost_step(tg.ga, d.m[iw], gs, a);
         if (again && round < tg.max_iter) {
+          const float rel = gs.h / old.h - 1.f;
+          want = rel * rel <= 2.f * tg.ga.eps;
+          pend = false;
           st.h_inv = 1.f / gs.h;
           st.hg2 = search_radius2(gs.h);
+        } else if (!full && !again) {
+          gs = old;
+          pend = want = true;
         } else {
           live = false;
           cnt = 0;
@@ -497,7 +533,8 @@ __device__ __forceinline__ void run_tile(
       }
       if (!__any(live)) break;  // uniform
       L::identity(acc);
-      round++;
+      if (__any(live && !pend)) round++;
+      full = __any(live && want);
       fresh = !whole || __any(live && !(st.hg2 <= listed));
     }
     // density interactions of the tile, and its rounds
