@@ -4,7 +4,7 @@
 // candidate stream s of 4 of particle g, as in the chunk engine
 // (sph_gather.h), and visits the same candidates in the same order, so the
 // sums are those of that engine bit for bit.  The work between is arranged
-// in windows of 1024 candidates (256 rows of 4):
+// in windows of 2048 candidates (512 rows of 4):
 //
 //   1. cull: the chunks of the 27 neighbour cells, one per lane, box against
 //      the tile's box in FP32 (ChunkArgs::fbox) in the tile frame -- positions
@@ -18,9 +18,10 @@
 //      loop's test, the interaction).
 //
 // Bound: VALU issue in the walk, whose wave runs as long as its fullest lane.
-// A window of 256 rows evens the lanes out better than the chunk engine's
-// 128 (modulated 97^3 box: 26 -> 21 iterations per tile for 13.5 hits per
-// lane), the matrix test takes 1 instruction per 64 pairs beside the signs
+// A window of 512 rows evens the lanes out better than the chunk engine's
+// 128 (modulated 97^3 box: 26 -> 21 iterations per tile at 256 for 13.5 hits
+// per lane; 512 rows in lists of 32 against 256 in lists of 44: density -4 %,
+// force -5 %, gradient even; wider ones cost more in LDS), the matrix test takes 1 instruction per 64 pairs beside the signs
 // (the FP16 rows took 7), and the pipelined walk has one load latency per
 // hit instead of three.
 //
@@ -35,10 +36,11 @@
 // made with, else from step 1 -- until all have converged.  That replaces a
 // ghost launch, a tile build and a density launch per round.  A step reads 2
 // of the 8 sums, and all are needed at the last h only: after the first an
-// evaluation takes the 2 (a third of the walk's arithmetic and 16 of the record's 40 bytes
-// less) until a particle of the tile is expected to converge, its last step
-// (relative: s) making s^2, the order of the next one, pass the tolerance; a
-// particle found to have converged before that is evaluated once more.
+// evaluation takes the 2 (a third of the walk's arithmetic and 16 of the
+// record's 40 bytes less) until a particle of the tile is expected to
+// converge, its last step (relative: s) making s^2, the order of the next
+// one, pass the tolerance; a particle found to have converged before that is
+// evaluated once more.
 #pragma once
 
 #include "sph_gather.h"
@@ -46,8 +48,8 @@
 
 namespace sphl {
 
-constexpr int kTileRows = 256;    // rows of 4 candidates in a window
-constexpr int kTileHits = 44;     // hits of a lane between two walks
+constexpr int kTileRows = 512;    // rows of 4 candidates in a window
+constexpr int kTileHits = 32;     // hits of a lane between two walks
 
 // What the finishing forms need beside the loop's arguments.
 struct TileGhost {
@@ -96,7 +98,7 @@ struct TileLds {
   float tp[L::kSymmetric ? kTpLen : 4 * kTpRow];
   // surviving chunks: (neighbour << 27) | first record slot
   unsigned int surv[CHUNKS + 64];
-  unsigned char rows[kTileHits * 64];  // hit k of lane l at 64 k + l
+  unsigned short rows[kTileHits * 64];  // hit k of lane l at 64 k + l
 };
 
 // Maximum over the 16 lanes of a row of lanes (lane % 16 varies).
@@ -412,7 +414,7 @@ __device__ __forceinline__ void run_tile(
       while (hits != 0u) {  // rows of these groups: 16 k0 + bit
         const int b = __builtin_ctz(hits);
         hits &= hits - 1u;
-        sh.rows[64 * cnt + lane] = (unsigned char)(16 * k0 + b);
+        sh.rows[64 * cnt + lane] = (unsigned short)(16 * k0 + b);
         cnt++;
       }
     }
