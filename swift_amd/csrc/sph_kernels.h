@@ -488,6 +488,9 @@ hipError_t launch_bin_keys(const double *px, const double *py, const double *pz,
                            int n, unsigned long long *key, int *val,
                            hipStream_t st, const int8_t *tb = nullptr,
                            unsigned int *mixed = nullptr);
+// *outside = 1 if a position (x[3 i + k]) is not in [0, dim), else 0.
+hipError_t launch_check_box(const double *x, int n, const GridDesc &g,
+                            unsigned int *outside, hipStream_t st);
 // Stable radix sort of (key, value) pairs on the low `bits` key bits; with
 // temp == nullptr only sets `bytes` (rocprim::radix_sort_pairs).
 hipError_t sort_pairs(void *temp, size_t &bytes, const unsigned long long *kin,

@@ -101,6 +101,18 @@ __global__ void k_bin_keys(const double *px, const double *py,
   val[i] = i;
 }
 
+__global__ void k_check_box(const double *x, int n, GridDesc g,
+                            unsigned int *outside) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  bool ok = true;
+  for (int k = 0; k < 3; k++) {
+    const double v = x[3 * (size_t)i + k];
+    ok = ok && v >= 0.0 && v < g.dim[k];
+  }
+  if (!ok) *outside = 1u;
+}
+
 // Periodic wrap of the positions into [0, dim) (box_wrap of space_rebuild;
 // a particle moves by less than a box length between two binnings).
 __global__ void k_wrap(DevParts d, GridDesc g, int n) {
@@ -548,6 +560,13 @@ hipError_t launch_bin_keys(const double *px, const double *py, const double *pz,
   k_bin_keys<<<blocks(n), kBlock, 0, st>>>(px, py, pz, stride, g, inv_w[0],
                                            inv_w[1], inv_w[2], n, key, val, tb,
                                            tb ? kBinBits : 0, mixed);
+  return hipGetLastError();
+}
+
+hipError_t launch_check_box(const double *x, int n, const GridDesc &g,
+                            unsigned int *outside, hipStream_t st) {
+  if (hipError_t err = launch_zero_u32(outside, 1, st)) return err;
+  if (n > 0) k_check_box<<<blocks(n), kBlock, 0, st>>>(x, n, g, outside);
   return hipGetLastError();
 }
 

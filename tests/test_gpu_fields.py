@@ -79,3 +79,26 @@ def test_optional_arrays_and_errors():
     for k in ("rho", "pressure", "soundspeed", "f", "balsara", "alpha_diff",
               "div_v_prev"):
         assert not got[k].any(), k
+
+
+@pytest.mark.parametrize("n", [1, 7, 999, 32767, 32768, 70001])
+def test_positions_outside_the_box(n):
+    """Refused with the index of the first one, on the host and on the device
+    (from 32768 particles on), and the last particles stay."""
+    from swift_amd import Engine, HydroProps
+    from swift_amd._lib import SwsphError
+    good = _parts(n, True, seed=n)
+    with Engine(HydroProps(ncell=(5, 4, 3), dim=(1.0, 1.5, 2.0))) as eng:
+        eng.set_particles(good)
+        for i, k, v in ((0, 0, 1.0), (n // 2, 1, 1.5), (n - 1, 2, 2.0),
+                        (n - 1, 0, -1e-300), (n // 3, 2, np.nan),
+                        (n // 2, 1, np.inf)):
+            bad = _parts(n, True, seed=n)
+            bad["x"][i, k] = v
+            with pytest.raises(SwsphError, match=f"particle {i} lies outside"):
+                eng.set_particles(bad)
+            assert np.array_equal(eng.get("x"), good["x"])
+        edge = _parts(n, True, seed=n)
+        edge["x"][n // 2] = [-0.0, np.nextafter(1.5, 0), np.nextafter(2.0, 0)]
+        eng.set_particles(edge)
+        assert np.array_equal(eng.get("x"), edge["x"])
