@@ -157,6 +157,30 @@ __host__ __device__ inline int xcd_blocks(int n) {
   return 8 * ((per + kWaves - 1) / kWaves);
 }
 
+// The same with runs of up to kXcdRun consecutive items dealt to the XCDs in
+// turn, so that all XCDs sweep the box together: for loops whose items cost
+// about the same, whose neighbour records then come from DRAM once (tiles of
+// 16: gradient and force of 128^3 particles -10 %, of 97^3 -2 %; the density
+// tiles, whose iteration differs from cell to cell, lose 2 % of clustered
+// boxes and keep the ranges).  Short grids take shorter runs, powers of two,
+// so that more items never need fewer blocks.
+constexpr int kXcdRun = 64;
+__host__ __device__ inline int xcd_run(int n) {
+  int r = kXcdRun;
+  while (r > 1 && 256 * r > n) r >>= 1;
+  return r;
+}
+__device__ __forceinline__ int xcd_run_item(int b, int w, int n) {
+  const int r = xcd_run(n);
+  const int k = (b >> 3) * kWaves + w;
+  return min(n, ((k / r) * 8 + (b & 7)) * r + k % r);
+}
+__host__ __device__ inline int xcd_run_blocks(int n) {
+  const int r = xcd_run(n);
+  const int per = (n + 8 * r - 1) / (8 * r) * r;
+  return 8 * ((per + kWaves - 1) / kWaves);
+}
+
 // LDS of one wave: the neighbour table, the compacted surviving chunks, the
 // staged candidate positions and the chunk table of the current 64 rows.
 // CI: i-particles per wave (S = 64 / CI candidate streams each); CJ:

@@ -1065,7 +1065,7 @@ hipError_t tile16_c(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
                     int max_tiles, bool rest, hipStream_t st) {
   const PosRec *pos = (const PosRec *)d.pos;
   if (!persistent) {
-    const int nb = max_tiles > 0 ? xcd_blocks(max_tiles) : 0;
+    const int nb = max_tiles > 0 ? tile16_blocks<L>(max_tiles) : 0;
     if (nb > 0)
       hipLaunchKernelGGL((k_tile16<L, CJ, FIN>), dim3(nb), dim3(64), 0, st, d,
                          la, ca, rec, pos, ta, tg);

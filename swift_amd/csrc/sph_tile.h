@@ -556,13 +556,25 @@ __device__ __forceinline__ void run_tile(
   }
 }
 
+// Block -> tile of the grids below.
+template <class L>
+constexpr bool kTileRuns = !std::is_same<L, DensityLoop>::value;
+template <class L>
+__host__ __device__ inline int tile16_blocks(int n) {
+  return kTileRuns<L> ? xcd_run_blocks(n) : xcd_blocks(n);
+}
+template <class L>
+__device__ __forceinline__ int tile16_item(int b, int w, int n) {
+  return kTileRuns<L> ? xcd_run_item(b, w, n) : xcd_item(b, w, n);
+}
+
 // One wave per tile over a grid sized for the tile count (see k_loop_tiles).
 template <class L, int CJ, bool FIN>
 __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, TileGhost tg) {
-  const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
+  const int t = tile16_item<L>(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
   if (t >= *tq.ntiles) return;  // uniform per wave
   run_tile<L, CJ, FIN>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
 }
@@ -574,9 +586,9 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_rest(
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, TileGhost tg, int b0) {
   const int n = *tq.ntiles;
-  const int nb = xcd_blocks(n);
+  const int nb = tile16_blocks<L>(n);
   for (int b = b0 + (int)blockIdx.x; b < nb; b += (int)gridDim.x) {
-    const int t = xcd_item(b, threadIdx.x >> 6, n);
+    const int t = tile16_item<L>(b, threadIdx.x >> 6, n);
     if (t >= n) continue;  // uniform per wave
     wave_sync();
     run_tile<L, CJ, FIN>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);

@@ -97,3 +97,30 @@ def test_tiles16_unconverged_is_an_error():
                dict(mode=1, shape=(16, 16), graph=True)):
         with pytest.raises(SwsphError, match="status 3"):
             _run(props, st, **kw)
+
+
+@pytest.mark.parametrize("n_side,ncell", [(9, 3), (16, 4), (17, 4), (20, 5),
+                                          (32, 8), (33, 8)])
+def test_tile_order_over_the_xcds(n_side, ncell):
+    """Gradient and force tiles are dealt to the XCDs in runs whose length
+    grows with the number of tiles (256 tiles and a few more, 500, 2048 and
+    more, and fewer than 8 runs): eager, and captured with a grid for more
+    tiles than there are, every tile once -- the grid schedule's sums."""
+    from swift_amd import Engine, HydroProps, ics
+    st = ics.modulated_box(n_side, seed=n_side)
+    out = []
+    for mode in ("grid", "queue", "graph"):
+        with Engine(HydroProps(ncell=(ncell,) * 3)) as eng:
+            eng.set_schedule(0 if mode == "grid" else 1)
+            eng.set_particles(st)
+            if mode == "graph":
+                eng.save_state()
+                for _ in range(2):
+                    eng.restore_state()
+                    eng.pass_graph()
+            else:
+                eng.pass_batched()
+            out.append(eng.results())
+    for r in out[1:]:
+        for k, v in out[0].items():
+            assert np.array_equal(v, r[k]), k
