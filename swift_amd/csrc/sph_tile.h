@@ -113,6 +113,37 @@ __device__ __forceinline__ float row16_max(float v) {
   v = fmaxf(v, dpp_f<0x122>(v));
   return fmaxf(v, dpp_f<0x121>(v));
 }
+// Largest value of the wave (uniform).
+__device__ __forceinline__ int wave_most(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, true));
+  return max(max(__builtin_amdgcn_readlane(v, 0),
+                 __builtin_amdgcn_readlane(v, 16)),
+             max(__builtin_amdgcn_readlane(v, 32),
+                 __builtin_amdgcn_readlane(v, 48)));
+}
+// Marks every field of a loaded record as used here: the wait for its loads
+// stands at this point.
+__device__ __forceinline__ void arrived(const DensRec &r) {
+  asm volatile("" :: "v"(r.x), "v"(r.y), "v"(r.z), "v"(r.vx), "v"(r.vy),
+                    "v"(r.vz), "v"(r.m));
+}
+__device__ __forceinline__ void arrived(const GradRec &r) {
+  asm volatile("" :: "v"(r.x), "v"(r.y), "v"(r.z), "v"(r.vx), "v"(r.vy),
+                    "v"(r.vz), "v"(r.mrho), "v"(r.u), "v"(r.c),
+                    "v"(r.alpha));
+}
+__device__ __forceinline__ void arrived(const ForceRec &r) {
+  asm volatile("" :: "v"(r.x), "v"(r.y), "v"(r.z), "v"(r.hg2), "v"(r.vx),
+                    "v"(r.vy), "v"(r.vz), "v"(r.m), "v"(r.inv_m),
+                    "v"(r.h_inv));
+  asm volatile("" :: "v"(r.rho), "v"(r.inv_rho), "v"(r.pr2), "v"(r.f),
+                    "v"(r.bal), "v"(r.c), "v"(r.alpha), "v"(r.P),
+                    "v"(r.Pad), "v"(r.u));
+  asm volatile("" :: "v"(r.tb));
+}
 __device__ __forceinline__ float lane_value(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
@@ -232,60 +263,76 @@ __device__ __forceinline__ void run_tile(
   int cnt = 0;  // hits in this lane's list
   bool full = true;  // the walk takes all sums (uniform)
 
-  // Step 4: the lists against the exact contract.
-  auto eval = [&](unsigned int info, const Rec &r, int j) {
-    const int q = (int)(info >> 27);
-    // own cell: oi = oj = x_i, which gives 0 - (float)(x_j - x_i)
-    const double *fo = q ? &sh.fo[6 * q] : &sh.xi[3 * g];
-    const double *fj = q ? fo + 3 : fo;
-    const float dx = (float)(st.x - fo[0]) - (float)(r.x - fj[0]);
-    const float dy = (float)(st.y - fo[1]) - (float)(r.y - fj[1]);
-    const float dz = (float)(st.z - fo[2]) - (float)(r.z - fj[2]);
-    const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-    // (the matrix test passes the particle itself)
-    if (L::test(r2, st, &r) && j != ic) {
-      if constexpr (ITER)
-        L::interact(r2, dx, dy, dz, st, r, acc, full);
+  // Step 4: the lists against the exact contract, the next record's loads in
+  // flight while the current one is evaluated.  The loop is uniform (to the
+  // fullest lane's hits) and its loads unconditional, a lane past its hits
+  // reading record 0: with a branch around them, or a register of a record
+  // that an untaken branch has not waited for, the compiler's waits for one
+  // record also wait for the next, and each hit costs a whole load latency.
+  auto walk_as = [&](auto all) {
+    constexpr bool ALL = decltype(all)::value;  // else only the step's sums
+    auto fetch = [&](int k, unsigned int &info, Rec &r) -> int {
+      const bool on = k < cnt;
+      // (read by all lanes: no branch)
+      const int got = sh.rows[64 * min(k, kTileHits - 1) + lane];
+      const int row = on ? got : 0;
+      info = sh.surv[row / RPC];
+      const int at = (int)(info & kRowMask) + (row % RPC) * 4 + s;
+      const int j = on ? at : 0;
+      if constexpr (ALL) {
+        r = rec[j];
+      } else {
+        r.x = rec[j].x;
+        r.y = rec[j].y;
+        r.z = rec[j].z;
+      }
+      return j;
+    };
+    auto eval = [&](int k, unsigned int info, const Rec &r, int j) {
+      // all of the record has arrived from here on
+      if constexpr (ALL)
+        arrived(r);
       else
-        L::interact(r2, dx, dy, dz, st, r, acc);
+        asm volatile("" :: "v"(r.x), "v"(r.y), "v"(r.z));
+      const int q = (int)(info >> 27);
+      // own cell: oi = oj = x_i, which gives 0 - (float)(x_j - x_i)
+      const double *fo = q ? &sh.fo[6 * q] : &sh.xi[3 * g];
+      const double *fj = q ? fo + 3 : fo;
+      const float dx = (float)(st.x - fo[0]) - (float)(r.x - fj[0]);
+      const float dy = (float)(st.y - fo[1]) - (float)(r.y - fj[1]);
+      const float dz = (float)(st.z - fo[2]) - (float)(r.z - fj[2]);
+      const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+      // (the matrix test passes the particle itself)
+      if (L::test(r2, st, &r) && j != ic && k < cnt) {
+        if constexpr (ITER)
+          L::interact(r2, dx, dy, dz, st, r, acc, ALL);
+        else
+          L::interact(r2, dx, dy, dz, st, r, acc);
+      }
+    };
+    const int most = wave_most(cnt);
+    if (most == 0) return;  // uniform
+    unsigned int n0, n1;
+    Rec r0, r1;
+    int j0 = fetch(0, n0, r0), j1 = 0;
+    int k = 0;
+    for (; k + 2 < most; k += 2) {
+      j1 = fetch(k + 1, n1, r1);
+      eval(k, n0, r0, j0);
+      j0 = fetch(k + 2, n0, r0);
+      eval(k + 1, n1, r1, j1);
     }
+    // one or two are left (no load past the last)
+    const bool two = k + 1 < most;
+    if (two) j1 = fetch(k + 1, n1, r1);
+    eval(k, n0, r0, j0);
+    if (two) eval(k + 1, n1, r1, j1);
   };
   auto walk = [&]() {
-    auto locate = [&](int k, unsigned int &info) -> int {
-      const int row = sh.rows[64 * k + lane];
-      info = sh.surv[row / RPC];
-      return (int)(info & kRowMask) + (row % RPC) * 4 + s;
-    };
-    auto fetch = [&](Rec &r, int j) {
-      if (ITER && !full) {  // uniform: the position is enough
-        const Rec *p = rec + j;
-        r.x = p->x;
-        r.y = p->y;
-        r.z = p->z;
-      } else {
-        r = rec[j];
-      }
-    };
-    unsigned int n0 = 0u, n1 = 0u;
-    int j0 = 0, j1 = 0;
-    Rec r0, r1;
-    if (cnt > 0) {
-      j0 = locate(0, n0);
-      fetch(r0, j0);
-    }
-    for (int k = 0; k < cnt; k += 2) {
-      if (k + 1 < cnt) {
-        j1 = locate(k + 1, n1);
-        fetch(r1, j1);
-      }
-      eval(n0, r0, j0);
-      if (k + 1 >= cnt) break;
-      if (k + 2 < cnt) {
-        j0 = locate(k + 2, n0);
-        fetch(r0, j0);
-      }
-      eval(n1, r1, j1);
-    }
+    if (!ITER || full)
+      walk_as(std::true_type{});
+    else
+      walk_as(std::false_type{});
   };
 
   // The candidates of a sweep, a window at a time.  pre: the lane's squared
