@@ -223,13 +223,14 @@ int swsph_cell_write_back(swsph_engine *e, int ci,
  * all cells.  Both leave identical neighbour sets. */
 int swsph_pass_plain(swsph_engine *e, swsph_pass_stats *stats);
 int swsph_pass_batched(swsph_engine *e, swsph_pass_stats *stats);
-/* The batched pass replayed from two captured HIP graphs: hydro_init_part,
- * the first density round and as many ghost / density re-run rounds as the
- * previous pass needed (rounds with nothing left to redo run empty), then
- * gradient -> extra ghost -> force -> end force.  The host reads one
- * convergence counter between the graphs and continues eagerly if more
- * rounds are needed; graphs are re-captured after any change of particles
- * or settings.  Results are identical to swsph_pass_batched.  Needs the
+/* The batched pass replayed from captured HIP graphs: one where the density
+ * loop runs in tiles of 16 of the work queue (the default), whose waves
+ * iterate the smoothing lengths; otherwise two: hydro_init_part, the first
+ * density round and as many ghost / density re-run rounds as the previous
+ * pass needed (rounds with nothing left to redo run empty), then gradient ->
+ * extra ghost -> force -> end force, with one convergence counter read
+ * between them and more rounds run eagerly if needed.  Graphs are re-captured
+ * after any change of particles or settings.  Results are identical to swsph_pass_batched.  Needs the
  * neighbour lists disabled.  No counterpart in the reference. */
 int swsph_pass_graph(swsph_engine *e, swsph_pass_stats *stats);
 /* swsph_pass_batched without any device allocation: the pass's scratch
