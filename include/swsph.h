@@ -388,7 +388,9 @@ int swsph_set_schedule(swsph_engine *e, int mode, int waves);
  * current particles (`repeats` timed passes each, HIP events per loop),
  * keeps the schedule with the smallest summed loop time and, under it, the
  * fastest capacity of each loop; under a work-queue schedule it then tries
- * candidate chunks of half the tile size per loop, and applies the result.
+ * candidate chunks of half the tile size and narrow tiles per loop; where the
+ * loops' picks differ, whole passes of them are timed against passes in tiles
+ * of 16 throughout (shared tables); the fastest is applied.
  * The pass state (h and the (io) fields) is saved before and restored
  * after, so results are those of an untuned engine.  No counterpart in the
  * reference. */
@@ -396,8 +398,10 @@ typedef struct swsph_tune_result {
   int schedule;       /* chosen schedule */
   int chunk[3];       /* chosen chunk capacity of each loop */
   double loop_ms[3];  /* loop times per pass of the choice (ms) */
-  double pass_ms;     /* wall time per pass, chosen schedule, capacity 16 */
-  int trials;         /* configurations timed */
+  double pass_ms;     /* wall time per pass of the choice if whole passes were
+                         compared, else of the schedule with capacity 16 */
+  int trials;         /* shapes timed (the closing comparison of whole passes
+                         of shapes timed before not counted) */
   int chunk_j[3];     /* chosen candidate chunk capacity of each loop */
 } swsph_tune_result;
 int swsph_autotune(swsph_engine *e, int repeats, swsph_tune_result *out);

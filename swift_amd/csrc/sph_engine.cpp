@@ -3342,7 +3342,8 @@ int swsph_autotune(swsph_engine *e, int repeats, swsph_tune_result *out) {
   int trials = 0;
   // Times `repeats` passes of the current settings: per-loop kernel time
   // and wall time per pass (ms).
-  auto time_config = [&](double ms[3], double *wall) -> int {
+  auto time_config = [&](double ms[3], double *wall,
+                         bool trial = true) -> int {
     int r = 0;
     e->gen++;
     // warm-up pass (builds the chunk tables of these capacities)
@@ -3364,7 +3365,7 @@ int swsph_autotune(swsph_engine *e, int repeats, swsph_tune_result *out) {
     *wall = std::chrono::duration<double, std::milli>(t1 - t0).count() / repeats;
     for (int k = 0; k < 3; k++) ms[k] = e->t_ms[k] / repeats;
     e->timing = false;
-    trials++;
+    if (trial) trials++;
     return 0;
   };
   // With lists the density loop builds them in tiles of kListChunk.
@@ -3443,6 +3444,34 @@ int swsph_autotune(swsph_engine *e, int repeats, swsph_tune_result *out) {
         }
     }
     for (int k = 0; k < 3; k++) best_c[k] = best_ci[k];
+    // Loops of different shapes need a chunk table and a tile table each
+    // (256^3 particles, 10 % active: 0.5 ms of 11 for two more), and a density
+    // loop in tiles of 16 needs no ghost rounds (0.4 ms): where the picks
+    // differ, whole passes of them are timed against passes in tiles of 16
+    // against one chunk size.
+    auto same = [&]() {
+      return best_c[0] == best_c[1] && best_c[0] == best_c[2] &&
+             best_cj[0] == best_cj[1] && best_cj[0] == best_cj[2];
+    };
+    if (!rc && !e->use_lists && !same()) {
+      const int mix_c[3] = {best_c[0], best_c[1], best_c[2]};
+      const int mix_cj[3] = {best_cj[0], best_cj[1], best_cj[2]};
+      double best_wall = 1e300;
+      for (int trial = 0; trial < 3 && !rc; trial++) {
+        for (int k = 0; k < 3; k++) {
+          e->loop_c[k] = trial == 0 ? mix_c[k] : 16;
+          e->loop_cj[k] = trial == 0 ? mix_cj[k] : trial == 1 ? 16 : 8;
+        }
+        double ms[3], w = 0;
+        if ((rc = time_config(ms, &w, false)) || w >= best_wall) continue;
+        best_wall = best_pass = w;
+        for (int k = 0; k < 3; k++) {
+          best_c[k] = e->loop_c[k];
+          best_cj[k] = e->loop_cj[k];
+          best_ms[k] = ms[k];
+        }
+      }
+    }
   }
   // apply the choice (or restore the settings after a failure) and the state
   e->schedule = rc ? sched0 : best_s;
