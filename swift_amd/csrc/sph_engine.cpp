@@ -186,6 +186,12 @@ struct swsph_engine {
   static constexpr int kStageWords = 3;
   static constexpr int kStagePad = 2 * sphk::kScatterWords;
   double *d_stage = nullptr;
+  // Read-backs up to kSmallRead bytes leave the device in one copy, into
+  // this pinned block (made for the largest so far, rounded up to a power of
+  // two); d_stage has room for as much.
+  static constexpr size_t kSmallRead = 2 << 20;
+  unsigned char *h_read = nullptr;
+  size_t cap_read = 0;
   // Time integration: parameters, the integer time line, and the largest
   // distance by which a particle lies outside its cell since the last
   // binning (float bits on the device; host copy).
@@ -694,7 +700,10 @@ int alloc_dev(swsph_engine *e, size_t n) {
   HIPCHK(dalloc(&e->d_key[1], n));
   HIPCHK(dalloc(&e->d_val[0], n));
   HIPCHK(dalloc(&e->d_val[1], n));
-  HIPCHK(dalloc(&e->d_stage, swsph_engine::kStageWords * n + swsph_engine::kStagePad));
+  HIPCHK(dalloc(&e->d_stage,
+                std::max(swsph_engine::kStageWords * n,
+                         swsph_engine::kSmallRead / sizeof(double)) +
+                    swsph_engine::kStagePad));
   size_t bytes = 0;
   HIPCHK(sphk::sort_pairs(nullptr, bytes, e->d_key[0], e->d_key[1],
                           e->d_val[0], e->d_val[1], (int)n, 64, e->st));
@@ -2400,6 +2409,7 @@ int swsph_engine_destroy(swsph_engine *e) {
   if (e->d_bnbrs) (void)hipFree(e->d_bnbrs);
   if (e->d_status) (void)hipFree(e->d_status);
   if (e->h_status) (void)hipHostFree(e->h_status);
+  if (e->h_read) (void)hipHostFree(e->h_read);
   if (e->h_tiend) (void)hipHostFree(e->h_tiend);
   if (e->h_err) (void)hipHostFree(e->h_err);
   if (e->h_ntiles) (void)hipHostFree(e->h_ntiles);
@@ -2574,6 +2584,65 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
     if (!outs[q]) return fail(1, "null output for field %d", fields[q]);
   }
   const size_t n = (size_t)e->n;
+  if (n == 0) {
+    HIPCHK(hipStreamSynchronize(e->st));
+    return 0;
+  }
+  // Up to kSmallRead bytes in all: scattered into the staging buffer, one
+  // copy into the engine's pinned block, and from there by the host.
+  // A copy costs about 8 us of launch and gap, a field that the staging
+  // buffer cannot take beside the others a wait of 25 us, the host's copy
+  // 10 us per 100 kB.  Calls on 15^3 particles (0.1 MB, 6 fields) 222 ->
+  // 197 us, 32^3 (1 MB) 274 -> 236, a server request of 24^3 (0.4 MB)
+  // 726 -> 678, 40^3 (2 MB) 911 -> 891: even at the limit, above it the
+  // copies go to the caller's memory themselves.
+  auto padded = [](size_t bytes) { return (bytes + 15) & ~(size_t)15; };
+  size_t total = 0;
+  for (int q = 0; q < nf && total <= swsph_engine::kSmallRead; q++) {
+    FieldView v;
+    (void)field_view(e->d, fields[q], v);
+    total += padded((size_t)v.esize() * v.ncomp * n);
+  }
+  if (total <= swsph_engine::kSmallRead) {
+    if (total > e->cap_read) {
+      if (e->h_read) (void)hipHostFree(e->h_read);
+      e->h_read = nullptr;
+      e->cap_read = 0;
+      size_t cap = 64 << 10;
+      while (cap < total) cap *= 2;
+      HIPCHK(hipHostMalloc((void **)&e->h_read, cap, 0));
+      e->cap_read = cap;
+    }
+    size_t off = 0;
+    for (int q = 0; q < nf;) {
+      sphk::ScatterSet s;
+      s.n = 0;
+      for (; q < nf; q++) {
+        FieldView v;
+        (void)field_view(e->d, fields[q], v);
+        if (s.n + v.ncomp > sphk::kScatterWords) break;
+        for (int k = 0; k < v.ncomp; k++)
+          s.w[s.n++] = {v.c[k], (char *)e->d_stage + off,
+                        (unsigned char)v.esize(), (unsigned char)v.ncomp,
+                        (unsigned char)k};
+        off += padded((size_t)v.esize() * v.ncomp * n);
+      }
+      HIPCHK(sphk::launch_scatter(s, e->d.perm, (int)n, e->st));
+    }
+    if (off > 0)
+      HIPCHK(hipMemcpyAsync(e->h_read, e->d_stage, off, hipMemcpyDeviceToHost,
+                            e->st));
+    HIPCHK(hipStreamSynchronize(e->st));
+    off = 0;
+    for (int q = 0; q < nf; q++) {
+      FieldView v;
+      (void)field_view(e->d, fields[q], v);
+      const size_t bytes = (size_t)v.esize() * v.ncomp * n;
+      std::memcpy(outs[q], e->h_read + off, bytes);
+      off += padded(bytes);
+    }
+    return 0;
+  }
   // As many fields as the staging buffer takes (24 bytes per particle) are
   // scattered into the caller's order, then copied out; the stream keeps the
   // next sweep behind the copies.  One sweep for all of them, or with many
@@ -2611,10 +2680,15 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
         s.w[s.n++] = {v.c[k], (char *)e->d_stage + off, (unsigned char)size,
                       (unsigned char)v.ncomp, (unsigned char)k};
       out[no++] = {outs[q], off, (size_t)size * v.ncomp * n};
-      off += ((size_t)size * v.ncomp * n + 15) & ~(size_t)15;
+      off += padded(out[no - 1].bytes);
     }
-    if (no == 0) {  // the buffer is full: wait for its copies
-      HIPCHK(hipStreamSynchronize(cs));
+    if (no == 0) {
+      // The buffer is full: the next sweep is behind its copies, on their
+      // stream or by an event (the host need not wait).
+      if (overlap) {
+        HIPCHK(hipEventRecord(e->ev_copy, cs));
+        HIPCHK(hipStreamWaitEvent(e->st, e->ev_copy, 0));
+      }
       off = 0;
       per = 0;
       continue;

@@ -102,3 +102,27 @@ def test_positions_outside_the_box(n):
         edge["x"][n // 2] = [-0.0, np.nextafter(1.5, 0), np.nextafter(2.0, 0)]
         eng.set_particles(edge)
         assert np.array_equal(eng.get("x"), edge["x"])
+
+
+@pytest.mark.parametrize("n,names", [
+    (1, ("time_bin",)), (262144, ("h", "rho")), (262145, ("h", "rho")),
+    (65536, ("h", "x", "h")), (9001, ("time_bin", "x", "rho")),
+    (5003, None), (70001, None)])
+def test_read_back_sizes(n, names):
+    """Fields of uploaded particles in one call, to both sides of the 2 MiB
+    that leave the device in one copy, and with the staging buffer filled
+    several times; a field may be asked for twice."""
+    from swift_amd import FIELDS, Engine, HydroProps, lib
+    p = _parts(n, True, seed=n)
+    with Engine(HydroProps(ncell=(5, 5, 5))) as eng:
+        eng.set_particles(p)
+        names = names or [k for k in FIELDS if k in p]
+        outs = [np.full((n, 3) if FIELDS[k][2] == 3 else (n,), -1,
+                        FIELDS[k][1]) for k in names]
+        ids = (C.c_int * len(names))(*[FIELDS[k][0] for k in names])
+        ptr = (C.c_void_p * len(names))(*[o.ctypes.data for o in outs])
+        for _ in range(2):
+            assert lib().swsph_get_fields(eng._h, len(names), ids, ptr) == 0
+            for k, o in zip(names, outs):
+                assert np.array_equal(o, p[k]), k
+                o[...] = -1
