@@ -221,7 +221,9 @@ int swsph_cell_write_back(swsph_engine *e, int ci,
  * Plain: the C task loop of the reference's dependency order (all density
  * tasks, ghosts, gradient tasks, extra ghosts, force tasks, end-force),
  * one launch per task.  Batched: the same pass as a handful of launches over
- * all cells.  Both leave identical neighbour sets. */
+ * all cells.  Both leave identical neighbour sets.  Status 3 if a smoothing
+ * length does not converge: nothing behind the ghost has then changed the
+ * particles, and the pass can be repeated with more iterations. */
 int swsph_pass_plain(swsph_engine *e, swsph_pass_stats *stats);
 int swsph_pass_batched(swsph_engine *e, swsph_pass_stats *stats);
 /* The batched pass replayed from captured HIP graphs: one where the density

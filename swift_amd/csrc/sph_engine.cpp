@@ -356,6 +356,7 @@ GhostArgs ghost_args(const swsph_engine *e) {
   g.lists = e->use_lists ? 1 : 0;
   g.grad_rec = 0;
   g.force_rec = 0;
+  g.stop = nullptr;
   return g;
 }
 
@@ -813,6 +814,7 @@ TileArgs tile_args(const swsph_engine *e) {
   ta.ids = nullptr;
   ta.filt = nullptr;
   ta.images = nullptr;
+  ta.stop = nullptr;
   return ta;
 }
 
@@ -825,6 +827,12 @@ bool finishes(const swsph_engine *e, LoopKind k) {
 // round of ghost, tile build and density each.
 bool iterates(const swsph_engine *e) {
   return finishes(e, LoopKind::Density);
+}
+
+// What the stages behind an iterating density loop look at (TileArgs::stop):
+// its particles that did not converge, which fail the pass.
+const unsigned long long *unconverged(const swsph_engine *e) {
+  return iterates(e) ? e->d_redo : nullptr;
 }
 
 // Waves of a captured grid that may find no tile (each exits at once: a few
@@ -851,6 +859,7 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
   if (sparse && !t1) return rc;
   const LoopArgs la = batched_args(e, k);
   TileArgs ta = tile_args(e);
+  if (k != LoopKind::Density) ta.stop = unconverged(e);
   // The all-active table is kept for the later loops of the pass.  With
   // the narrowest tiles the flagged rounds (mode 1) take the subset of its
   // tiles that hold a flagged particle, with the others masked out, instead
@@ -1660,7 +1669,8 @@ int phase_rerun(swsph_engine *e, int redo, int relist) {
 }
 
 // Gradient records and bounds, gradient loop, extra ghost, force records,
-// force loop, end force.
+// force loop, end force.  After a density loop that iterates none of them
+// changes a particle while particles are left unconverged.
 int phase_finish(swsph_engine *e) {
   int rc = 0;
   const int n = (int)e->n;
@@ -1676,6 +1686,7 @@ int phase_finish(swsph_engine *e) {
   // stores are faster than one scattered 96-byte record per thread.
   GhostArgs gx = ghost_args(e);
   gx.fresh_force = 1;
+  gx.stop = unconverged(e);
   const bool fin_g = finishes(e, LoopKind::Gradient);
   const bool narrow =
       e->schedule >= 1 && e->loop_c[(int)LoopKind::Force] == kMinTile;
@@ -1710,7 +1721,7 @@ int phase_finish(swsph_engine *e) {
     return rc;
   if (!fin_f) {
     HIPCHK(sphk::launch_end_force(e->d, 0, n, e->props.max_active_bin, e->st,
-                                  list, cnt));
+                                  list, cnt, gx.stop));
     e->launches++;
   }
   return 0;

@@ -798,6 +798,12 @@ __global__ __launch_bounds__(64) void k_loop_task(
                                               none);
 }
 
+// The tiles of the queue (uniform).
+__device__ __forceinline__ int tile_count(const TileArgs &tq) {
+  const int n = *tq.ntiles;
+  return tq.stop && *tq.stop != 0ull ? 0 : n;
+}
+
 // Persistent form: a fixed grid of waves drains the tile queue.  A wave
 // starts on the queue of its XCD (blocks are dealt round-robin over the 8
 // XCDs), takes kGrab tiles per atomic, and moves on to the next queue when
@@ -806,7 +812,7 @@ __global__ __launch_bounds__(64) void k_loop_task(
 constexpr int kGrab = 2;
 template <class F>
 __device__ __forceinline__ void drain_queue(const TileArgs &tq, F run) {
-  const int nt = *tq.ntiles;
+  const int nt = tile_count(tq);
   const int per = (nt + 7) >> 3;
   int q = blockIdx.x & 7;
   for (int tries = 0; tries < 8;) {
@@ -854,8 +860,9 @@ __global__ SWSPH_TILE_BOUNDS(L) void k_loop_tiles(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     NbrList nl, TileArgs tq) {
-  const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
-  if (t >= *tq.ntiles) return;  // uniform per wave
+  const int n = tile_count(tq);
+  const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, n);
+  if (t >= n) return;  // uniform per wave
   run_chunk<L, CI, CJ, false, BUILD, true>(d, la, ca, rec, pos, 0, true, 0, 0.0,
                                            0.0, 0.0, nl, &tq, t);
 }
@@ -871,7 +878,7 @@ __global__ __launch_bounds__(64) void k_loop_tiles_rest(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     NbrList nl, TileArgs tq, int b0) {
-  const int n = *tq.ntiles;
+  const int n = tile_count(tq);
   const int nb = xcd_blocks(n);
   for (int b = b0 + (int)blockIdx.x; b < nb; b += (int)gridDim.x) {
     const int t = xcd_item(b, threadIdx.x >> 6, n);

@@ -80,6 +80,12 @@ struct TileArgs {
   // offset code o = 9 (ox + 1) + 3 (oy + 1) + (oz + 1)); null: all 27.
   // Tiles of 16 only.
   const unsigned int *images;
+  // Null, or a counter of the loops before this one: while it is not zero the
+  // queue holds no tiles (tile_count).  Particles whose smoothing length did
+  // not converge make the pass fail, but a density loop that iterates is only
+  // read back at the end of the pass: the loops behind it leave the particles
+  // alone by themselves.
+  const unsigned long long *stop;
 };
 
 // Structure-of-arrays particle store in HBM, sorted by top-level cell.
@@ -246,6 +252,9 @@ struct GhostArgs {
   // 1: the ghost writes the gradient record of each particle it finishes,
   // the extra ghost the force record of each particle (no separate builds).
   int grad_rec, force_rec;
+  // As TileArgs::stop, for the sweeps of the extra ghost and the end of the
+  // force loop.
+  const unsigned long long *stop;
 };
 
 enum class LoopKind { Density, Gradient, Force };
@@ -455,7 +464,8 @@ hipError_t launch_extra_ghost(const DevParts &d, const GhostArgs &ga, int lo,
 hipError_t launch_end_force(const DevParts &d, int lo, int hi,
                             int max_active_bin, hipStream_t st,
                             const int *list = nullptr,
-                            const int *cnt = nullptr);
+                            const int *cnt = nullptr,
+                            const unsigned long long *stop = nullptr);
 hipError_t launch_count(const DevParts &d, int n, int max_active_bin,
                         unsigned long long *out3, hipStream_t st);
 // Copies n floats from each src[k] to dst[k], k < m <= kMaxCopies, in one

@@ -480,6 +480,7 @@ __global__ void k_task_images(const int *__restrict__ tasks, int ntasks,
 // runner_do_extra_ghost for the active particles in [lo, hi) or of the list.
 __global__ void k_extra_ghost(DevParts d, GhostArgs ga, int lo, int hi,
                               const int *list, const int *cnt) {
+  if (ga.stop && *ga.stop != 0ull) return;  // uniform
   auto body = [&](int i, int8_t tb) {
     if (!is_active(tb, ga.max_active_bin)) return;
     extra_ghost_one(d, ga, i, tb, d.vsig[i], d.lapu[i], d.avmax[i]);
@@ -492,7 +493,9 @@ __global__ void k_extra_ghost(DevParts d, GhostArgs ga, int lo, int hi,
 
 // runner_do_end_hydro_force for the active particles.
 __global__ void k_end_force(DevParts d, int lo, int hi, int max_active_bin,
-                            const int *list, const int *cnt) {
+                            const int *list, const int *cnt,
+                            const unsigned long long *stop) {
+  if (stop && *stop != 0ull) return;  // uniform
   auto body = [&](int i, int8_t tb) {
     if (is_active(tb, max_active_bin))
       d.hdt[i] = end_force_hdt(d.hdt[i], d.h[i]);
@@ -1502,10 +1505,10 @@ hipError_t launch_extra_ghost(const DevParts &d, const GhostArgs &ga, int lo,
 
 hipError_t launch_end_force(const DevParts &d, int lo, int hi,
                             int max_active_bin, hipStream_t st, const int *list,
-                            const int *cnt) {
+                            const int *cnt, const unsigned long long *stop) {
   if (hi <= lo) return hipSuccess;
   hipLaunchKernelGGL(k_end_force, dim3(run_blocks(hi - lo, 256)), dim3(256), 0, st, d,
-                     lo, hi, max_active_bin, list, cnt);
+                     lo, hi, max_active_bin, list, cnt, stop);
   return hipGetLastError();
 }
 

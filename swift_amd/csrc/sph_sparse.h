@@ -394,8 +394,9 @@ __global__ __launch_bounds__(64, L::kSparseWavesPerSimd) void k_sparse_tiles(
     DevParts d, LoopArgs la, ChunkArgs c1, ChunkArgs c2,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq) {
-  const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
-  if (t >= *tq.ntiles) return;  // uniform per wave
+  const int n = tile_count(tq);
+  const int t = xcd_item(blockIdx.x, threadIdx.x >> 6, n);
+  if (t >= n) return;  // uniform per wave
   run_sparse<L>(d, la, c1, c2, rec, pos, tq, t);
 }
 
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(64) void k_sparse_tiles_rest(
     DevParts d, LoopArgs la, ChunkArgs c1, ChunkArgs c2,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, int b0) {
-  const int n = *tq.ntiles;
+  const int n = tile_count(tq);
   const int nb = xcd_blocks(n);
   for (int b = b0 + (int)blockIdx.x; b < nb; b += (int)gridDim.x) {
     const int t = xcd_item(b, threadIdx.x >> 6, n);

@@ -621,8 +621,9 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, TileGhost tg) {
-  const int t = tile16_item<L>(blockIdx.x, threadIdx.x >> 6, *tq.ntiles);
-  if (t >= *tq.ntiles) return;  // uniform per wave
+  const int n = tile_count(tq);
+  const int t = tile16_item<L>(blockIdx.x, threadIdx.x >> 6, n);
+  if (t >= n) return;  // uniform per wave
   run_tile<L, CJ, FIN>(d, la, ca, rec, pos, queue_parts(d, tq, t), tg, t);
 }
 
@@ -632,7 +633,7 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_rest(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
     TileArgs tq, TileGhost tg, int b0) {
-  const int n = *tq.ntiles;
+  const int n = tile_count(tq);
   const int nb = tile16_blocks<L>(n);
   for (int b = b0 + (int)blockIdx.x; b < nb; b += (int)gridDim.x) {
     const int t = tile16_item<L>(b, threadIdx.x >> 6, n);
