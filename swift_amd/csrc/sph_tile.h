@@ -512,10 +512,14 @@ __device__ __forceinline__ void run_tile(
     // sums after the combination and takes the same step.
     GhostState gs{0.f, 0.f, tg.ga.h_max};
     if (act) gs.h = d.h[i];
+    if (act && tg.given) {  // as the last ghost or hydro_init_part left it
+      gs.left = d.left[i];
+      gs.right = d.right[i];
+    }
     bool live = act;
-    // pend: converged in an evaluation of the step's sums only; want: the
-    // next one should take all
-    bool pend = false, want = false;
+    // pend: converged in an evaluation of the step's sums only, or (over) out
+    // of iterations; want: the next one should take all
+    bool pend = false, over = false, want = false;
     float listed = -1.f;  // squared radius that the lists cover
     // the lists hold every hit of the sweep (one window took it all)
     bool whole = false, fresh = true, given = tg.given != 0;
@@ -552,29 +556,38 @@ __device__ __forceinline__ void run_tile(
         int iw = i;
         asm volatile("" : "+v"(iw));
         if (!pend) work += acc.n;
-        DensSums a{acc.rho, acc.rho_dh, acc.wc, acc.wc_dh,
-                   acc.divv, acc.rx, acc.ry, acc.rz};
-        const GhostState old = gs;
-        const bool again = ghost_step(tg.ga, d.m[iw], gs, a);
-        if (again && round < tg.max_iter) {
-          const float rel = gs.h / old.h - 1.f;
-          want = rel * rel <= 2.f * tg.ga.eps;
-          pend = false;
-          st.h_inv = 1.f / gs.h;
-          st.hg2 = search_radius2(gs.h);
-        } else if (!full && !again) {
-          gs = old;
-          pend = want = true;
-        } else {
+        if (over) {
+          // Not converged: h, its bracket and the raw sums at it, from which
+          // another ghost goes on.
           live = false;
           cnt = 0;
           if (s == 0) {
-            d.nd[iw] = acc.n;
-            if (again) {  // not converged
-              d.h[iw] = gs.h;
-              d.redo[iw] = 1;
-              atomicAdd(&tg.counters[0], 1ull);
-            } else {
+            d.h[iw] = gs.h;
+            d.left[iw] = gs.left;
+            d.right[iw] = gs.right;
+            d.redo[iw] = 1;
+            L::store_acc(d, iw, acc);
+            atomicAdd(&tg.counters[0], 1ull);
+          }
+        } else {
+          DensSums a{acc.rho, acc.rho_dh, acc.wc, acc.wc_dh,
+                     acc.divv, acc.rx, acc.ry, acc.rz};
+          const GhostState old = gs;
+          const bool again = ghost_step(tg.ga, d.m[iw], gs, a);
+          if (again) {
+            const float rel = gs.h / old.h - 1.f;
+            pend = over = round >= tg.max_iter;
+            want = over || rel * rel <= 2.f * tg.ga.eps;
+            st.h_inv = 1.f / gs.h;
+            st.hg2 = search_radius2(gs.h);
+          } else if (!full) {
+            gs = old;
+            pend = want = true;
+          } else {
+            live = false;
+            cnt = 0;
+            if (s == 0) {
+              d.nd[iw] = acc.n;
               ghost_finish(d, tg.ga, iw, gs.h, a);
             }
           }

@@ -73,3 +73,90 @@ def test_unconverged_pass_ends_at_the_ghost(form):
     assert 0 < count < st["h"].size
     for k in LATER:
         assert np.array_equal(before[k], after[k]), k
+
+
+DENSITY = ("h", "rho", "rho_dh", "wcount", "wcount_dh", "div_v", "rot_v",
+           "pressure", "soundspeed", "f", "balsara", "n_density")
+
+
+def _fail_and_repeat(form):
+    """All fields after status 3, and after the pass repeated from there with
+    enough iterations."""
+    props, st = _start()
+    with _engine(dataclasses.replace(props, max_iter=3), form) as eng:
+        eng.set_particles(st)
+        _fail(eng, form)
+        failed = eng.results()
+        eng.set_props(props)
+        eng.pass_graph() if form[2] else eng.pass_batched()
+        return failed, eng.results()
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_unconverged_pass_can_be_repeated(form):
+    """A particle that did not converge is left with the raw density sums at
+    its last h, a converged one finished, bit for bit as the grid schedule's
+    separate ghost rounds leave them; the repeated pass agrees as well (its
+    gradient and force sums where the tiles add in the grid's order)."""
+    ref = _fail_and_repeat(GRID)
+    got = _fail_and_repeat(form)
+    same = [s[0] == 16 for s in form[1]]
+    for k in ref[0]:
+        assert np.array_equal(ref[0][k], got[0][k]), k
+        if k in DENSITY or all(same):
+            assert np.array_equal(ref[1][k], got[1][k]), k
+
+
+def _ghost_tasks(eng, how):
+    """The ghosts of all cells; how many of the calls ended with status 3."""
+    from swift_amd import SwsphError
+    nc = eng.num_cells()
+    if how == "bundle":
+        calls = [lambda: eng.runner_do_ghost_cells(range(nc))]
+    else:
+        calls = [lambda c=c, o=o: eng.runner_do_ghost(c, o, how)
+                 for c in range(nc) for o in range(how)]
+    failed = 0
+    for call in calls:
+        try:
+            call()
+        except SwsphError as err:
+            assert "status 3" in str(err)
+            failed += 1
+    return failed
+
+
+@pytest.mark.parametrize("how", [1, 2, "bundle"])
+def test_ghost_goes_on_where_it_ended(how):
+    """A ghost task that ran out of iterations, called again, goes on with
+    the bracket and the sums at the h it had reached: the same results as one
+    that had enough iterations."""
+    props, st = _start()
+    out = []
+    for first in (props.max_iter, 3):
+        with _engine(dataclasses.replace(props, max_iter=first),
+                     FORMS[0]) as eng:
+            eng.set_particles(st)
+            nc = eng.num_cells()
+            eng.init_cells(range(nc))
+            nz, ny, nx = props.ncell[2], props.ncell[1], props.ncell[0]
+            pairs = set()
+            for c in range(nc):
+                x, y, z = c // (ny * nz), (c // nz) % ny, c % nz
+                for d in np.ndindex(3, 3, 3):
+                    o = (((x + d[0] - 1) % nx) * ny + (y + d[1] - 1) % ny) \
+                        * nz + (z + d[2] - 1) % nz
+                    if o != c:
+                        pairs.add((min(c, o), max(c, o)))
+            eng.run_tasks("density", [(0, c, c) for c in range(nc)]
+                          + [(1, a, b) for a, b in sorted(pairs)])
+            failed = _ghost_tasks(eng, how)
+            if first == 3:
+                assert failed > 0
+                eng.set_props(props)
+                _ghost_tasks(eng, how)
+            else:
+                assert failed == 0
+            out.append(eng.results(DENSITY))
+    for k in DENSITY:
+        assert np.array_equal(out[0][k], out[1][k]), k
