@@ -350,8 +350,9 @@ hipError_t launch_tile16(LoopKind kind, bool fin, bool given,
                          unsigned long long *counters, bool persistent,
                          int waves, int max_tiles, bool rest, hipStream_t st);
 // The same on the flagged particles of one cell (nchunks chunks of the table
-// of 16) of share off of nt, after their density tasks.
-hipError_t launch_ghost_cell(const DevParts &d, const LoopArgs &la,
+// of 16) of share off of nt, after their density tasks; fin = false: their
+// density sums alone.
+hipError_t launch_ghost_cell(bool fin, const DevParts &d, const LoopArgs &la,
                              const ChunkArgs &ca, const GhostArgs &ga,
                              int max_iter, unsigned long long *counters,
                              int cell, int nchunks, int off, int nt,

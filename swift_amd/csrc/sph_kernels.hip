@@ -1097,18 +1097,25 @@ hipError_t tile16_any(const DevParts &d, const LoopArgs &la,
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_ghost_cell(const DevParts &d, const LoopArgs &la,
+hipError_t launch_ghost_cell(bool fin, const DevParts &d, const LoopArgs &la,
                              const ChunkArgs &ca, const GhostArgs &ga,
                              int max_iter, unsigned long long *counters,
                              int cell, int nchunks, int off, int nt,
                              hipStream_t st) {
-  if (!ca.fbox || ca.C != 16) return hipErrorInvalidValue;
+  if (!ca.fbox || ca.C != 16 || (!fin && !la.fresh))
+    return hipErrorInvalidValue;
   if (nchunks <= 0) return hipSuccess;
   const TileGhost tg{ga, max_iter, counters,
                      (unsigned int *)(counters + kGhostRounds), 1};
-  hipLaunchKernelGGL((k_ghost_cell<DensityLoop>), dim3(nchunks), dim3(64), 0,
-                     st, d, la, ca, d.rd, (const PosRec *)d.pos, tg, cell, off,
-                     nt);
+  const PosRec *pos = (const PosRec *)d.pos;
+  if (fin)
+    hipLaunchKernelGGL((k_ghost_cell<DensityLoop, true>), dim3(nchunks),
+                       dim3(64), 0, st, d, la, ca, d.rd, pos, tg, cell, off,
+                       nt);
+  else
+    hipLaunchKernelGGL((k_ghost_cell<DensityLoop, false>), dim3(nchunks),
+                       dim3(64), 0, st, d, la, ca, d.rd, pos, tg, cell, off,
+                       nt);
   return hipGetLastError();
 }
 

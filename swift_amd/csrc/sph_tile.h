@@ -512,20 +512,20 @@ __device__ __forceinline__ void run_tile(
     // sums after the combination and takes the same step.
     GhostState gs{0.f, 0.f, tg.ga.h_max};
     if (act) gs.h = d.h[i];
-    if (act && tg.given) {  // as the last ghost or hydro_init_part left it
-      gs.left = d.left[i];
-      gs.right = d.right[i];
-    }
     bool live = act;
-    // pend: converged in an evaluation of the step's sums only, or (over) out
-    // of iterations; want: the next one should take all
-    bool pend = false, over = false, want = false;
+    // pend: converged in an evaluation of the step's sums only; want: the
+    // next one should take all
+    bool pend = false, want = false;
     float listed = -1.f;  // squared radius that the lists cover
     // the lists hold every hit of the sweep (one window took it all)
     bool whole = false, fresh = true, given = tg.given != 0;
     int work = 0, round = 1;
     L::identity(acc);
-    if (given && act) L::load_acc(d, i, acc);
+    if (given && act) {
+      L::load_acc(d, i, acc);
+      gs.left = d.left[i];  // as the last ghost or hydro_init_part left them
+      gs.right = d.right[i];
+    }
     wave_sync();
     for (;;) {  // a window, or a walk over lists that still serve
       bool more = false;
@@ -556,38 +556,34 @@ __device__ __forceinline__ void run_tile(
         int iw = i;
         asm volatile("" : "+v"(iw));
         if (!pend) work += acc.n;
-        if (over) {
-          // Not converged: h, its bracket and the raw sums at it, from which
-          // another ghost goes on.
+        DensSums a{acc.rho, acc.rho_dh, acc.wc, acc.wc_dh,
+                   acc.divv, acc.rx, acc.ry, acc.rz};
+        const GhostState old = gs;
+        const bool again = ghost_step(tg.ga, d.m[iw], gs, a);
+        if (again && round < tg.max_iter) {
+          const float rel = gs.h / old.h - 1.f;
+          want = rel * rel <= 2.f * tg.ga.eps;
+          pend = false;
+          st.h_inv = 1.f / gs.h;
+          st.hg2 = search_radius2(gs.h);
+        } else if (!full && !again) {
+          gs = old;
+          pend = want = true;
+        } else {
           live = false;
           cnt = 0;
           if (s == 0) {
-            d.h[iw] = gs.h;
-            d.left[iw] = gs.left;
-            d.right[iw] = gs.right;
-            d.redo[iw] = 1;
-            L::store_acc(d, iw, acc);
-            atomicAdd(&tg.counters[0], 1ull);
-          }
-        } else {
-          DensSums a{acc.rho, acc.rho_dh, acc.wc, acc.wc_dh,
-                     acc.divv, acc.rx, acc.ry, acc.rz};
-          const GhostState old = gs;
-          const bool again = ghost_step(tg.ga, d.m[iw], gs, a);
-          if (again) {
-            const float rel = gs.h / old.h - 1.f;
-            pend = over = round >= tg.max_iter;
-            want = over || rel * rel <= 2.f * tg.ga.eps;
-            st.h_inv = 1.f / gs.h;
-            st.hg2 = search_radius2(gs.h);
-          } else if (!full) {
-            gs = old;
-            pend = want = true;
-          } else {
-            live = false;
-            cnt = 0;
-            if (s == 0) {
-              d.nd[iw] = acc.n;
+            d.nd[iw] = acc.n;
+            if (again) {
+              // Not converged: flagged, with the bracket of its new h; the
+              // host has the sums at that h formed (FIN = false), from which
+              // another ghost goes on.
+              d.h[iw] = gs.h;
+              d.left[iw] = gs.left;
+              d.right[iw] = gs.right;
+              d.redo[iw] = 1;
+              atomicAdd(&tg.counters[0], 1ull);
+            } else {
               ghost_finish(d, tg.ga, iw, gs.h, a);
             }
           }
@@ -670,8 +666,9 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_tile16_queue(
 
 // runner_do_ghost on one cell after its density tasks: one wave per chunk of
 // 16 of the cell, each taking the chunk's flagged particles of share off of
-// nt (slot counted from the cell's first field slot, as k_ghost).
-template <class L>
+// nt (slot counted from the cell's first field slot, as k_ghost).  FIN =
+// false: only their density sums.
+template <class L, bool FIN>
 __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_ghost_cell(
     DevParts d, LoopArgs la, ChunkArgs ca,
     const typename L::Rec *__restrict__ rec, const PosRec *__restrict__ pos,
@@ -685,7 +682,7 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_ghost_cell(
   t.act = t.ic < hi && d.redo[t.i] != 0 && (t.i - lo) % nt == off;
   if (!__any(t.act)) return;  // uniform
   if (!t.act) t.ic = -1;
-  run_tile<L, 16, true>(d, la, ca, rec, pos, t, tg, (int)blockIdx.x);
+  run_tile<L, 16, FIN>(d, la, ca, rec, pos, t, tg, (int)blockIdx.x);
 }
 
 // A self or pair task on cells in chunks of 16: one wave per chunk of either

@@ -15,16 +15,17 @@ pytestmark = pytest.mark.gpu
 LATER = ("v_sig", "laplace_u", "alpha_visc_max_ngb", "alpha_visc",
          "alpha_diff", "div_v_dt", "div_v_prev", "a_hydro", "u_dt", "h_dt",
          "n_gradient", "n_force", "min_ngb_time_bin")
-# (schedule, shapes of the three loops, replayed)
-GRID = (0, ((16, 16),) * 3, False)
+# (schedule, shapes of the three loops, method of the pass)
+GRID = (0, ((16, 16),) * 3, "pass_batched")
 FORMS = [
-    (1, ((16, 16),) * 3, False),
-    (1, ((16, 16),) * 3, True),
-    (2, ((16, 16),) * 3, False),
-    (1, ((16, 8), (32, 16), (8, 8)), False),
-    (1, ((16, 16), (4, 8), (16, 16)), True),
-    (1, ((16, 16), (16, 16), (4, 8)), False),
-    (2, ((16, 16), (32, 32), (4, 8)), False),
+    (1, ((16, 16),) * 3, "pass_batched"),
+    (1, ((16, 16),) * 3, "pass_graph"),
+    (2, ((16, 16),) * 3, "pass_batched"),
+    (1, ((16, 16),) * 3, "pass_batched_noalloc"),
+    (1, ((16, 8), (32, 16), (8, 8)), "pass_batched"),
+    (1, ((16, 16), (4, 8), (16, 16)), "pass_graph"),
+    (1, ((16, 16), (16, 16), (4, 8)), "pass_batched"),
+    (2, ((16, 16), (32, 32), (4, 8)), "pass_batched"),
 ]
 
 
@@ -57,7 +58,7 @@ def _fail(eng, form):
     """One pass that ends with status 3; the number of particles it names."""
     from swift_amd import SwsphError
     with pytest.raises(SwsphError, match="status 3") as err:
-        eng.pass_graph() if form[2] else eng.pass_batched()
+        getattr(eng, form[2])()
     return int(str(err.value).split(" particles")[0].split()[-1])
 
 
@@ -88,7 +89,7 @@ def _fail_and_repeat(form):
         _fail(eng, form)
         failed = eng.results()
         eng.set_props(props)
-        eng.pass_graph() if form[2] else eng.pass_batched()
+        getattr(eng, form[2])()
         return failed, eng.results()
 
 
