@@ -357,6 +357,7 @@ __global__ __launch_bounds__(kGhostBlock) void k_ghost(
   const int stride = gridDim.x * kGhostBlock;
   const int nl = list ? *cnt : 0;
   int idx[kRuns], redo[kRuns];
+  int8_t tb[kRuns];
 #pragma unroll
   for (int u = 0; u < kRuns; u++) {
     if (list) {
@@ -369,13 +370,17 @@ __global__ __launch_bounds__(kGhostBlock) void k_ghost(
     }
   }
 #pragma unroll
-  for (int u = 0; u < kRuns; u++) redo[u] = idx[u] >= 0 ? d.redo[idx[u]] : 0;
+  for (int u = 0; u < kRuns; u++) {
+    redo[u] = idx[u] >= 0 ? d.redo[idx[u]] : 0;
+    tb[u] = idx[u] >= 0 ? d.tb[idx[u]] : (int8_t)kBinInhibited;
+  }
   unsigned int again = 0u, relist = 0u;  // bit u: run u
   // density interactions evaluated for these particles in the last round
   unsigned long long work = 0ull;
 #pragma unroll
   for (int u = 0; u < kRuns; u++) {
-    if (redo[u]) {
+    // (an inactive particle's flag is not cleared by every pass)
+    if (redo[u] && is_active(tb[u], ga.max_active_bin)) {
       const int i = idx[u];
       work += (unsigned long long)d.nd[i];
       bool rl = false;

@@ -679,7 +679,9 @@ __global__ __launch_bounds__(64, L::kTile16WavesPerSimd) void k_ghost_cell(
   t.images = kAllImages;
   t.ic = lo + 16 * (int)blockIdx.x + (int)(threadIdx.x & 15);
   t.i = t.ic < hi ? field_slot(d, t.ic) : 0;
-  t.act = t.ic < hi && d.redo[t.i] != 0 && (t.i - lo) % nt == off;
+  // (an inactive particle's flag is not cleared by every pass)
+  t.act = t.ic < hi && d.redo[t.i] != 0 && (t.i - lo) % nt == off &&
+          is_active(d.tb[t.i], la.max_active_bin);
   if (!__any(t.act)) return;  // uniform
   if (!t.act) t.ic = -1;
   run_tile<L, 16, FIN>(d, la, ca, rec, pos, t, tg, (int)blockIdx.x);

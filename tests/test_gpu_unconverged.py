@@ -161,3 +161,31 @@ def test_ghost_goes_on_where_it_ended(how):
             out.append(eng.results(DENSITY))
     for k in DENSITY:
         assert np.array_equal(out[0][k], out[1][k]), k
+
+
+@pytest.mark.parametrize("shape", [(16, 16), (8, 8)])
+def test_ghost_leaves_inactive_particles(shape):
+    """Particles flagged by a pass that failed, inactive in the next one, are
+    not the business of the ghosts of that step."""
+    props, st = _start()
+    late = np.random.default_rng(6).uniform(size=st["h"].size) < 0.5
+    low = int(st["time_bin"].max())
+    st["time_bin"][late] = low + 4
+    with _engine(dataclasses.replace(props, max_iter=3), FORMS[0]) as eng:
+        eng.set_particles(st)
+        _fail(eng, FORMS[0])
+        eng.set_props(dataclasses.replace(props, max_active_bin=low))
+        eng.pass_batched()
+        before = eng.results(DENSITY)
+        eng.set_tile_shape("density", *shape)
+        nc = eng.num_cells()
+        eng.init_cells(range(nc))
+        for c in range(nc):
+            eng.runner_doself1_branch_density(c)
+        eng.set_props(dataclasses.replace(props, max_active_bin=low,
+                                          h_tolerance=1.0))
+        assert _ghost_tasks(eng, 1) == 0
+        after = eng.results(DENSITY)
+    assert late.any()
+    for k in DENSITY:
+        assert np.array_equal(before[k][late], after[k][late]), k
