@@ -134,3 +134,31 @@ def test_tile_tables_hold_every_shape():
                 tiles = int(((k + C - 1) // C).sum())
                 assert tiles + 1 <= cap, (ncells, n, C, tiles, cap)
                 assert tiles <= max(n, 1)
+
+
+def test_library_is_rebuilt_after_any_source(tmp_path):
+    """make takes an existing library for stale after a change to any of its
+    sources and headers."""
+    import glob
+    import os
+    import shutil
+    import subprocess
+    from swift_amd._lib import HEADER_PATH, LIB_PATH
+    if shutil.which("make") is None:
+        pytest.skip("make not available")
+    csrc = os.path.join(os.path.dirname(LIB_PATH), "csrc")
+    out = tmp_path / "libswsph.so"
+    out.write_bytes(b"")
+    os.utime(out, (2 ** 31, 2 ** 31))  # newer than every source
+
+    def plan(*what):
+        return subprocess.run(["make", "-n", "-C", csrc, f"OUT={out}", *what],
+                              capture_output=True, text=True, check=True).stdout
+
+    assert "-shared" not in plan()
+    files = [f for e in ("h", "hip", "cpp")
+             for f in glob.glob(os.path.join(csrc, "*." + e))]
+    assert len(files) > 10
+    missed = [f for f in files + [HEADER_PATH]
+              if "-shared" not in plan("-W", os.path.abspath(f))]
+    assert not missed, missed
