@@ -875,16 +875,21 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
     ta.filt = flag;
     HIPCHK(sphk::launch_select_tiles(e->ts, flag, e->ts.ids, e->ts.nids,
                                      e->st));
-    if (e->schedule == 2 || e->capturing)
+    e->launches += 2;
+    if (e->schedule == 2 || e->capturing) {
       HIPCHK(sphk::launch_zero_u32((unsigned int *)e->ts.heads, 8 * 64,
                                    e->st));
+      e->launches++;
+    }
   } else if (!(mode == 0 && e->tiles_c == C)) {
     HIPCHK(sphk::launch_build_tiles(e->d, la, (int)e->n, e->ncells, C, mode,
                                     flag, e->ts, e->st));
+    e->launches += 3;
     e->tiles_c = mode == 0 ? C : 0;
     e->tiles_n = -1;
   } else if (e->schedule == 2) {
     HIPCHK(sphk::launch_zero_u32((unsigned int *)e->ts.heads, 8 * 64, e->st));
+    e->launches++;
   }
   int max_tiles = (int)(e->n / C) + e->ncells + 1;
   bool persistent = e->schedule == 2, rest = false;
@@ -940,7 +945,7 @@ int queue_loop(swsph_engine *e, LoopKind k, int mode, const int *flag,
     HIPCHK(sphk::launch_queue(k, build, e->d, la, chunk_args(t), ta, e->nl, C,
                               CJ, persistent, e->queue_waves, max_tiles, rest,
                               e->st));
-  e->launches += 4;
+  e->launches += (max_tiles > 0 ? 1 : 0) + (rest ? 1 : 0);
   return time_end(e, k, a);
 }
 

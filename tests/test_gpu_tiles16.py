@@ -124,3 +124,25 @@ def test_tile_order_over_the_xcds(n_side, ncell):
     for r in out[1:]:
         for k, v in out[0].items():
             assert np.array_equal(v, r[k]), k
+
+
+@pytest.mark.parametrize("mode,shapes,want", [
+    # counters, three for the tile table, density, chunk bounds, gradient,
+    # force
+    (1, ((16, 16),) * 3, 8),
+    # the loops that reuse the table clear its queue heads
+    (2, ((16, 16),) * 3, 10),
+    # a tile table per loop, a second chunk table, and the sweeps of the
+    # extra ghost and the force records
+    (1, ((16, 16), (32, 32), (16, 16)), 17)])
+def test_launches_are_counted_as_issued(mode, shapes, want):
+    from swift_amd import Engine
+    props, st = _box("ragged")
+    with Engine(props) as eng:
+        eng.set_regrid(False)
+        eng.set_schedule(mode)
+        for loop, s in zip(("density", "gradient", "force"), shapes):
+            eng.set_tile_shape(loop, *s)
+        eng.set_particles(st)
+        eng.pass_batched()
+        assert eng.pass_batched()["launches"] == want
