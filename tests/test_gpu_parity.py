@@ -429,6 +429,50 @@ def test_graph_replay_matches_eager(orc, mode):
         assert np.array_equal(eres[k], g2res[k]), k
 
 
+@pytest.mark.parametrize("shape", [(8, 8), (32, 16), (32, 32), (64, 64),
+                                   (4, 32), (4, 8)])
+def test_graph_continues_beyond_the_captured_rounds(shape):
+    """Shapes whose density loop leaves the smoothing lengths to separate
+    ghost rounds, under the work queue: a start that needs more rounds than
+    were captured continues eagerly, the next pass is captured with as many,
+    and one that then needs fewer runs the spare rounds empty -- each with the
+    eager pass's results bit for bit."""
+    from swift_amd import Engine, HydroProps, ics
+    st = ics.modulated_box(16, seed=31, amp=0.5)
+    poor = {k: np.array(v, copy=True) for k, v in st.items()}
+    poor["h"] = (poor["h"] * np.float32(0.55)).astype(np.float32)
+    props = HydroProps(ncell=(4, 4, 4))
+
+    def engine():
+        eng = Engine(props)
+        eng.set_schedule(1)
+        for loop in ("density", "gradient", "force"):
+            eng.set_tile_shape(loop, *shape)
+        return eng
+
+    want = []
+    for s in (poor, st):
+        with engine() as eng:
+            eng.set_particles(s)
+            want.append((eng.pass_batched(), eng.results()))
+    assert want[0][0]["ghost_rounds"] > max(4, want[1][0]["ghost_rounds"])
+    with engine() as eng:
+        for k in (0, 0, 1):
+            eng.set_particles((poor, st)[k])
+            eng.save_state()
+            for rep in range(2):
+                eng.restore_state()
+                g = eng.pass_graph()
+                res = eng.results()
+                for name in ("ghost_rounds", "n_density_all", "n_density",
+                             "n_force"):
+                    if name == "ghost_rounds" and k == 1:
+                        continue  # the captured ones, some of them empty
+                    assert g[name] == want[k][0][name], (k, rep, name)
+                for f in res:
+                    assert np.array_equal(want[k][1][f], res[f]), (k, rep, f)
+
+
 def test_autotune_keeps_state_and_results(orc):
     """The autotuner times every schedule and chunk capacity on the current
     particles (then, under the work queue, half-size candidate chunks and
