@@ -188,8 +188,13 @@ struct swsph_engine {
   double *d_stage = nullptr;
   // Read-backs up to kSmallRead bytes leave the device in one copy, into
   // this pinned block (made for the largest so far, rounded up to a power of
-  // two); d_stage has room for as much.
+  // two); d_stage has room for as much, or for every field once (170 bytes
+  // per particle and their alignment) on fewer particles.  (With 2 MiB for
+  // all, the buffers of 729 particles took 4.4 MiB; 0.6 now.)
   static constexpr size_t kSmallRead = 2 << 20;
+  static size_t small_read(size_t n) {
+    return std::min(kSmallRead, 176 * n + 1024);
+  }
   unsigned char *h_read = nullptr;
   size_t cap_read = 0;
   // Time integration: parameters, the integer time line, and the largest
@@ -703,7 +708,7 @@ int alloc_dev(swsph_engine *e, size_t n) {
   HIPCHK(dalloc(&e->d_val[1], n));
   HIPCHK(dalloc(&e->d_stage,
                 std::max(swsph_engine::kStageWords * n,
-                         swsph_engine::kSmallRead / sizeof(double)) +
+                         swsph_engine::small_read(n) / sizeof(double)) +
                     swsph_engine::kStagePad));
   size_t bytes = 0;
   HIPCHK(sphk::sort_pairs(nullptr, bytes, e->d_key[0], e->d_key[1],
@@ -2626,7 +2631,7 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
     HIPCHK(hipStreamSynchronize(e->st));
     return 0;
   }
-  // Up to kSmallRead bytes in all: scattered into the staging buffer, one
+  // Up to small_read bytes in all: scattered into the staging buffer, one
   // copy into the engine's pinned block, and from there by the host.
   // A copy costs about 8 us of launch and gap, a field that the staging
   // buffer cannot take beside the others a wait of 25 us, the host's copy
@@ -2636,12 +2641,13 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
   // copies go to the caller's memory themselves.
   auto padded = [](size_t bytes) { return (bytes + 15) & ~(size_t)15; };
   size_t total = 0;
-  for (int q = 0; q < nf && total <= swsph_engine::kSmallRead; q++) {
+  const size_t small = swsph_engine::small_read(e->cap_n);
+  for (int q = 0; q < nf && total <= small; q++) {
     FieldView v;
     (void)field_view(e->d, fields[q], v);
     total += padded((size_t)v.esize() * v.ncomp * n);
   }
-  if (total <= swsph_engine::kSmallRead) {
+  if (total <= small) {
     if (total > e->cap_read) {
       if (e->h_read) (void)hipHostFree(e->h_read);
       e->h_read = nullptr;
