@@ -17,8 +17,13 @@ constexpr int kOccForceTiles = 6;
 // The sparse-tile kernels (sph_sparse.h): one tile per wave.
 constexpr int kOccSparse = 6;  // density, gradient (their LDS allows 6)
 constexpr int kOccForceSparse = 5;
-// The tiles of 16 (sph_tile.h).
-constexpr int kOccTile16 = 5;  // density, gradient (their LDS allows 5)
+// The tiles of 16 (sph_tile.h).  Their LDS (density and gradient: 8584 bytes
+// against chunks of 16, 9096 of 8) has room for 19 or 18 waves on a CU, so 4
+// on every SIMD.  A bound of 5, which it allows on two or three of the four,
+// held the density form to 96 registers and made the persistent forms spill
+// up to 18 (clustered 144^3 19.04 ms with 5, 18.53 with 4; stepped 80^3 15.6
+// and 15.3; modulated 97^3 and 128^3 even).
+constexpr int kOccTile16 = 4;
 constexpr int kOccForceTile16 = 4;
 // The persistent forms of both engines: their loop around the tile costs
 // registers (at 7 waves per SIMD the density form spilled 34 VGPRs).
