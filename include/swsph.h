@@ -233,12 +233,13 @@ int swsph_pass_batched(swsph_engine *e, swsph_pass_stats *stats);
  * pass needed (rounds with nothing left to redo run empty), then gradient ->
  * extra ghost -> force -> end force, with one convergence counter read
  * between them and more rounds run eagerly if needed.  Graphs are re-captured
- * after any change of particles or settings.  Results are identical to swsph_pass_batched.  Needs the
- * neighbour lists disabled.  No counterpart in the reference. */
+ * after any change of particles or settings.  Results are identical to
+ * swsph_pass_batched.  Needs the neighbour lists disabled.  No counterpart in
+ * the reference. */
 int swsph_pass_graph(swsph_engine *e, swsph_pass_stats *stats);
 /* swsph_pass_batched without any device allocation: the pass's scratch
- * (the work queue: particle flags, scans, compact particle list, tile
- * table and queue heads; the ghost and interaction counters) lives in one
+ * (the work queue: cell counts, compact particle list, tile table and
+ * queue heads; the ghost and interaction counters) lives in one
  * fixed device array of the library (about 16 MB per GPU, held from the
  * first engine creation on that GPU until the process ends) instead of the
  * engine's buffers.  Same kernels and launches, so the results are
@@ -489,10 +490,10 @@ int swsph_engine_step(swsph_engine *e, swsph_step_info *info);
  * overlaps on the GPU, and a finished request frees its slot for the next
  * at once.  Each slot keeps its engine between requests and reuses its
  * device buffers when the next box fits (the budget counts the admitted
- * requests, not this retained capacity).  A box submitted with keep != 0 stays resident after its step
- * (its id is the request's id) and is stepped again with
- * swsph_server_step without a new upload.  Results stay on the host until
- * swsph_server_release.  Errors: swsph_server_last_error(). */
+ * requests, not this retained capacity).  A box submitted with keep != 0
+ * stays resident after its step (its id is the request's id) and is stepped
+ * again with swsph_server_step without a new upload.  Results stay on the
+ * host until swsph_server_release.  Errors: swsph_server_last_error(). */
 typedef struct swsph_server swsph_server;
 typedef struct swsph_server_opts {
   double hbm_budget_bytes;

@@ -3,9 +3,10 @@
 //
 // The engine keeps the gas particles resident in HBM as a structure of
 // arrays sorted by top-level cell (binned on the device, sph_step.hip) and
-// issues the kernels of sph_kernels.hip and sph_step.hip on one HIP stream.  The per-task entry points are the drop-in for SWIFT's
-// runner task functions; swsph_pass_plain drives them in the reference's
-// dependency order (src/engine_maketasks.c:2546-2573: density -> ghost ->
+// issues the kernels of sph_kernels.hip and sph_step.hip on one HIP stream
+// (large read-backs copy on a second one).  The per-task entry points are the
+// drop-in for SWIFT's runner task functions; swsph_pass_plain drives them in
+// the reference's dependency order (src/engine_maketasks.c:2546-2573: density -> ghost ->
 // gradient -> extra ghost -> force -> end force), swsph_pass_batched runs
 // the same pass as a few launches over all cells, and swsph_engine_step
 // advances the gas in time around it (drift, kicks, time steps).
@@ -2251,7 +2252,7 @@ int run_tasks_locked(swsph_engine *e, int loop, const swsph_task *tasks,
       coords(c, a);
       for (int p = 0; p < 27; p++) {
         // (in the order of the 27-cell stencil, as the work queue's tiles)
-        const int o = p == 0 ? 13 : ((p & 1) ? p >> 1 : 27 - (p >> 1));
+        const int o = stencil_code(p);
         if (!(mask[c] >> o & 1u)) continue;
         const int d[3] = {o / 9 - 1, (o / 3) % 3 - 1, o % 3 - 1};
         BundleNbr bn{};

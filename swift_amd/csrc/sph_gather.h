@@ -17,9 +17,12 @@
 // the largest search radius, then a ballot) and compacts the survivors into
 // LDS.  Survivors are staged 64 particles at a time into LDS and tested in
 // rows of S: stream s tests candidate (row start + s) against its particle
-// g.  The row test is an FP32 pre-test on cell-relative positions whose
-// radius is widened by a proven bound on its difference from the pair
-// contract (pretest_radius2), so it never rejects a neighbour.  A pass sets
+// g.  The row test is a pre-test in lower precision whose radius is widened
+// by a proven bound on its difference from the pair contract
+// (pretest_radius2), so it never rejects a neighbour: with CI = 16 in FP32 on
+// the matrix cores; with an even number of rows per chunk, in density and
+// gradient, in packed FP16; else in FP32 on cell-relative positions.  A pass
+// sets
 // one bit of the lane's row masks (kMasks x 64 bits); a per-chunk table in
 // LDS remembers where each chunk starts and which image it uses.  After
 // 64 x kMasks rows every lane
@@ -43,7 +46,8 @@
 
 namespace sphl {
 
-// Visiting order of the 27 neighbour offsets o = 9(ox+1) + 3(oy+1) + (oz+1).
+// Visiting order of the 27 neighbour offsets o = 9(ox+1) + 3(oy+1) + (oz+1):
+// stencil_code of 0..26.
 __constant__ const int kStencilOrder[27] = {13, 0,  26, 1,  25, 2,  24, 3,  23,
                                             4,  22, 5,  21, 6,  20, 7,  19, 8,
                                             18, 9,  17, 10, 16, 11, 15, 12, 14};
@@ -90,7 +94,8 @@ constexpr unsigned int kRowMask = (1u << 27) - 1u;
 constexpr int kMasks = 2;
 
 // The candidate pre-test of the density and gradient loops runs in packed
-// FP16 (two rows per instruction) when a chunk has an even number of rows.
+// FP16 (two rows per instruction) when a chunk has an even number of rows,
+// the tiles of 16 apart: (32, 32), (32, 16), (64, 64), (4, 32), (8, 16).
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
 // The pre-test of the tiles of 16 runs on the matrix cores: one

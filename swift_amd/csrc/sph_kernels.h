@@ -235,6 +235,13 @@ struct BundleArgs {
 };
 
 constexpr int kTaskSelf = 0, kTaskPair = 1;
+
+// Visiting order of the stencil: the offset code 9 (ox + 1) + 3 (oy + 1) +
+// (oz + 1) of position p of 0..26 -- the own cell, then 0, 26, 1, 25, ...
+// (sph_gather.h has the table).
+__host__ __device__ constexpr int stencil_code(int p) {
+  return p == 0 ? 13 : ((p & 1) ? p >> 1 : 27 - (p >> 1));
+}
 struct GhostArgs {
   float eta_dim, eps, h_max, h_min;
   int max_active_bin;

@@ -1002,8 +1002,9 @@ hipError_t queue_c(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
 
 // Tile (CI) x chunk (CJ) shapes with kernels of the chunk engine: CJ = CI,
 // CJ = CI / 2 for CI = 32 (finer candidate chunks under the same tile; the
-// tiles of 16 have their own kernels, launch_tile16), and the narrow tiles (4, 16), (4, 32), (8, 16) for sparse activity (a few active particles
-// per cell: more candidate streams per particle, fewer idle lanes).
+// tiles of 16 have their own kernels, launch_tile16), and the narrow tiles
+// (4, 16), (4, 32), (8, 16) for sparse activity (a few active particles per
+// cell: more candidate streams per particle, fewer idle lanes).
 template <class L>
 hipError_t queue_any(const DevParts &d, const LoopArgs &la, const ChunkArgs &ca,
                      const TileArgs &ta, const NbrList &nl,

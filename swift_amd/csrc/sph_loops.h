@@ -21,7 +21,7 @@ constexpr int kOccForceSparse = 5;
 // against chunks of 16, 9096 of 8) has room for 19 or 18 waves on a CU, so 4
 // on every SIMD.  A bound of 5, which it allows on two or three of the four,
 // held the density form to 96 registers and made the persistent forms spill
-// up to 18 (clustered 144^3 19.04 ms with 5, 18.53 with 4; stepped 80^3 15.6
+// up to 16 (clustered 144^3 19.04 ms with 5, 18.53 with 4; stepped 80^3 15.6
 // and 15.3; modulated 97^3 and 128^3 even).
 constexpr int kOccTile16 = 4;
 constexpr int kOccForceTile16 = 4;

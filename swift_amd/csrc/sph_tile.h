@@ -17,13 +17,16 @@
 //      flight while the current one is evaluated (FP64 pair contract, the
 //      loop's test, the interaction).
 //
-// Bound: VALU issue in the walk, whose wave runs as long as its fullest lane.
+// Bound: the walk's gathers and VALU issue together, in waves that run as long
+// as their fullest lane (busy share of the cycles, L1 return path / VALU, on
+// modulated 97^3 and clustered 144^3: density 0.92 / 0.81 and 0.89 / 0.95,
+// gradient 0.95 / 0.87 and 0.95 / 0.84, force 0.95 / 0.79 and 0.95 / 0.81).
 // A window of 512 rows evens the lanes out better than the chunk engine's
 // 128 (modulated 97^3 box: 26 -> 21 iterations per tile at 256 for 13.5 hits
 // per lane; 512 rows in lists of 32 against 256 in lists of 44: density -4 %,
-// force -5 %, gradient even; wider ones cost more in LDS), the matrix test takes 1 instruction per 64 pairs beside the signs
-// (the FP16 rows took 7), and the pipelined walk has one load latency per
-// hit instead of three.
+// force -5 %, gradient even; wider ones cost more in LDS), the matrix test
+// takes 1 instruction per 64 pairs beside the signs (the FP16 rows took 7),
+// and the pipelined walk has one load latency per hit instead of three.
 //
 // With FIN the tiles also finish their particles, which saves the sweeps over
 // them that would follow (a launch each and their fields read back): the
@@ -209,10 +212,10 @@ __device__ __forceinline__ void run_tile(
     sh.xi[3 * g + 2] = st.z;
   }
 
-  // Neighbour table: lane q < 27 describes neighbour q of kStencilOrder.
+  // Neighbour table: lane q < 27 describes neighbour q of the stencil.
   int nchq = 0;
   if (lane < 27) {
-    const int o = lane == 0 ? 13 : ((lane & 1) ? lane >> 1 : 27 - (lane >> 1));
+    const int o = stencil_code(lane);
     const int o3[3] = {o / 9 - 1, (o / 3) % 3 - 1, o % 3 - 1};
     int v[3];
     double t[3];
