@@ -121,9 +121,10 @@ int swsph_set_props(swsph_engine *e, const swsph_props *props);
 int swsph_set_particles(swsph_engine *e, const swsph_host_parts *p);
 int swsph_get_field(swsph_engine *e, int field, void *host_out);
 /* nf fields at once (as swsph_get_field each), with one wait at the end:
- * up to 2 MiB in all go through a page-locked block of the engine; above
- * that, with page-locked outputs (hipHostMalloc), the copies are
- * asynchronous DMA behind each other. */
+ * up to 2 MiB in all go through a page-locked block of the engine, with
+ * page-locked outputs (hipHostMalloc) up to 320 KiB per field beyond the
+ * first; above that the copies go to the outputs themselves, with page-locked
+ * ones as asynchronous DMA behind each other. */
 int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
                      void *const *outs);
 int swsph_num_cells(swsph_engine *e, int *ncells);

@@ -2633,16 +2633,33 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
     return 0;
   }
   // Up to small_read bytes in all: scattered into the staging buffer, one
-  // copy into the engine's pinned block, and from there by the host.
-  // A copy costs about 8 us of launch and gap, a field that the staging
-  // buffer cannot take beside the others a wait of 25 us, the host's copy
-  // 10 us per 100 kB.  Calls on 15^3 particles (0.1 MB, 6 fields) 222 ->
-  // 197 us, 32^3 (1 MB) 274 -> 236, a server request of 24^3 (0.4 MB)
-  // 726 -> 678, 40^3 (2 MB) 911 -> 891: even at the limit, above it the
-  // copies go to the caller's memory themselves.
+  // copy into the engine's pinned block, and from there by the host; above
+  // that the copies go to the caller's memory themselves.  The host's copy
+  // costs 36 us per MiB, a copy of its own 8 us and more per field (and for
+  // pageable memory the runtime's staging): with page-locked outputs the
+  // block pays up to kOwnCopy bytes per field beyond the first.  Microseconds
+  // for one field of 0.25 / 1 / 2 MiB to page-locked memory: 26 / 42 / 62 by its
+  // own copy, 33 / 80 / 132 through the block; three fields of 0.6 MiB in
+  // all 51 both ways, six of 2 MiB 118 both ways, 25 of 1.4 MiB 97 through
+  // the block.  Pageable: 34 / 84 / 132 by the runtime, 33 / 86 / 128 through
+  // the block, three fields 107-172 and 34-97.
   auto padded = [](size_t bytes) { return (bytes + 15) & ~(size_t)15; };
   size_t total = 0;
-  const size_t small = swsph_engine::small_read(e->cap_n);
+  size_t small = swsph_engine::small_read(e->cap_n);
+  bool locked = true;  // every output
+  for (int q = 0; q < nf && small > 0; q++) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, outs[q]) != hipSuccess) {
+      (void)hipGetLastError();
+      locked = false;
+    } else if (at.type == hipMemoryTypeUnregistered) {
+      locked = false;
+    } else if (at.type != hipMemoryTypeHost) {
+      small = 0;  // not the host's to write
+    }
+  }
+  constexpr size_t kOwnCopy = 320 << 10;
+  if (locked && nf > 0) small = std::min(small, kOwnCopy * (nf - 1));
   for (int q = 0; q < nf && total <= small; q++) {
     FieldView v;
     (void)field_view(e->d, fields[q], v);

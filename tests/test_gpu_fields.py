@@ -160,3 +160,41 @@ def test_small_boxes_hold_little_memory():
     finally:
         for eng in engines:
             eng.close()
+
+
+@pytest.mark.parametrize("n,names", [
+    (1, ("h",)), (70001, ("h",)), (20479, ("x", "rho")), (20481, ("x", "rho")),
+    (9001, ("h", "rho", "x")), (70001, ("h", "time_bin", "rho", "u")),
+    (87000, ("x",)), (5003, None)])
+@pytest.mark.parametrize("where", ["locked", "device", "mixed"])
+def test_read_back_to_locked_memory(n, names, where):
+    """Outputs in page-locked memory (copied to by the device, or through the
+    engine's block where that is shorter), in device memory, and one of them
+    pageable among page-locked ones."""
+    from swift_amd import FIELDS, Engine, HydroProps, lib
+    p = _parts(n, True, seed=n)
+    names = names or [k for k in FIELDS if k in p]
+    size = [n * FIELDS[k][2] * np.dtype(FIELDS[k][1]).itemsize for k in names]
+    at = np.cumsum([0] + [(s + 255) // 256 * 256 for s in size])
+    L, buf = lib(), C.c_void_p()
+    total = C.c_size_t(int(at[-1]))
+    alloc = ((lambda b: L.hipMalloc(b, total)) if where == "device"
+             else (lambda b: L.hipHostMalloc(b, total, 0)))
+    assert alloc(C.byref(buf)) == 0
+    host = np.empty(int(at[-1]), np.uint8)
+    try:
+        with Engine(HydroProps(ncell=(5, 5, 5))) as eng:
+            eng.set_particles(p)
+            ptrs = [buf.value + int(o) for o in at[:-1]]
+            if where == "mixed":
+                ptrs[0] = host.ctypes.data
+            ids = (C.c_int * len(names))(*[FIELDS[k][0] for k in names])
+            outs = (C.c_void_p * len(names))(*ptrs)
+            assert L.swsph_get_fields(eng._h, len(names), ids, outs) == 0
+            for k, q, s in zip(names, ptrs, size):
+                got = np.empty(p[k].shape, p[k].dtype)
+                assert L.hipMemcpy(got.ctypes.data_as(C.c_void_p),
+                                   C.c_void_p(q), C.c_size_t(s), 4) == 0
+                assert np.array_equal(got, p[k]), k
+    finally:
+        (L.hipFree if where == "device" else L.hipHostFree)(buf)
