@@ -250,3 +250,30 @@ def test_zero_energy_pair(orc):
     errs = compare(res, ref, ok, fields)
     for k, (tol, _) in fields.items():
         assert errs[k] <= tol, (k, errs[k])
+
+
+@pytest.mark.parametrize("n_side,ncell", [(6, 3), (7, 3), (32, 8), (33, 8),
+                                          (65, 16)])
+def test_counts_sum_every_active_particle(n_side, ncell):
+    """The counting sweep at one block, at 128 blocks of one particle per
+    thread and beyond, and with several per thread: the sums of the
+    particles' own counters."""
+    from swift_amd import Engine, HydroProps, ics
+    st = ics.lattice_box(n_side, seed=n_side, jitter=0.2)
+    ics.set_active_fraction(st, 0.6, seed=n_side)
+    st["rho"] = np.ones_like(st["rho"])
+    st["pressure"] = (st["u"] * np.float32(2 / 3)).astype(np.float32)
+    st["soundspeed"] = np.sqrt(st["pressure"] * np.float32(5 / 3))
+    if n_side < 8:
+        st["h"] = np.minimum(st["h"], np.float32(0.15))
+    props = HydroProps(ncell=(ncell,) * 3, eta=0.9 if n_side < 8 else 1.2348)
+    act = st["time_bin"] <= props.max_active_bin
+    with Engine(props) as eng:
+        eng.set_particles(st)
+        s = eng.pass_batched()
+        res = eng.results(["n_density", "n_gradient", "n_force"])
+        assert act.any() and not act.all()
+        want = tuple(int(res[k][act].sum(dtype=np.int64))
+                     for k in ("n_density", "n_gradient", "n_force"))
+        assert want == (s["n_density"], s["n_gradient"], s["n_force"])
+        assert tuple(eng.count_interactions()) == want
