@@ -689,7 +689,7 @@ int alloc_dev(swsph_engine *e, size_t n) {
     TileScratch &t = e->ts;
     const size_t nc = (size_t)e->ncells;
     HIPCHK(dalloc(&t.cell, nc));
-    HIPCHK(dalloc(&t.blk, nc / kTileCells + 1));
+    HIPCHK(dalloc(&t.blk, nc));
     HIPCHK(dalloc(&t.alist, n));
     HIPCHK(dalloc(&t.nlist, 1));
     // a cell of k particles makes ceil(k / C) tiles: at most n / C + nc

@@ -293,11 +293,9 @@ struct StepArgs {
 };
 
 // Scratch of the tile builder, sized for n particles and ncells cells.
-// Cells per block of the builder's per-cell kernels (one wave each).
-constexpr int kTileCells = 16;
 struct TileScratch {
   unsigned long long *cell;  // [ncells] selected particles << 32 | tiles
-  unsigned long long *blk;   // [ncells / kTileCells + 1] their block sums
+  unsigned long long *blk;   // [ncells] their sums by block
   int *alist;       // [n] the selected particles, in cell order
   int *nlist;       // [1] their number
   int *tile_start;  // [n / C + ncells + 1] for the smallest C in use

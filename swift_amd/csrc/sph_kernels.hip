@@ -695,12 +695,20 @@ __global__ void k_count_active(const int8_t *__restrict__ tb, int n,
 // ------------------------------------------------------------ tile builder --
 // The particles a loop processes, compacted in cell order and cut into
 // tiles, in three launches: a wave per cell counts its particles, one block
-// scans the sums of every kTileCells cells, and a wave per cell writes its
-// part of the list and its tiles.  Everything stays on the device.  (A scan
+// scans the sums of every kTileWaves cells, and a wave per cell writes its
+// part of the list and its tiles; a cell that holds most of its block's slots
+// is shared by the block's waves.  Everything stays on the device.  (A scan
 // over the particle slots took ten launches and five passes over 4 bytes
 // per slot: 35 us of launches on a small box, 150-200 us at 16.8 M slots.)
-constexpr int kTileBlock = 64 * kTileCells;
+// Bound by the latency of a wave's dependent loads, 512 slots at a time: with
+// one wave for every cell a bundle on 4096 cells, one of 20000 / 100000 / 300000
+// particles, took 238 / 727 / 1950 us, shared 134 / 204 / 369; a pass over a
+// halo of 69000 in a cell, 1 % active, 2.10 ms, shared 1.74; 27 cells of 16384
+// each 194 us, shared in blocks of a cell each 59.
+constexpr int kTileWaves = 16;  // waves, and cells (or one), per block
+constexpr int kTileBlock = 64 * kTileWaves;
 constexpr int kScanBlock = 1024;
+constexpr int kTileOwn = 1024;  // slots that a wave always takes alone
 
 // Exclusive scan of v over a block of kScanBlock threads; *total receives
 // the block sum.
@@ -741,19 +749,19 @@ __device__ __forceinline__ bool tile_pred(const DevParts &d, const LoopArgs &la,
   return true;
 }
 
-// The particles of cell c that the tiles take, 64 at a time in slot order:
-// f(field slot, taken).  With two slot orders the slots are record slots, so
-// that the particles of a cell that several active time bins hold still form
-// tiles in the cell's Morton order; with one active bin both orders list
-// them alike.  kRuns runs are loaded together.
+// The particles of cell c's slots [lo, hi) that the tiles take, 64 at a time
+// in slot order: f(field slot, taken).  With two slot orders the slots are
+// record slots, so that the particles of a cell that several active time bins
+// hold still form tiles in the cell's Morton order; with one active bin both
+// orders list them alike.  kRuns runs are loaded together.
 template <class F>
 __device__ __forceinline__ void for_cell_tiles(const DevParts &d,
                                                const LoopArgs &la, int mode,
-                                               const int *flag, int c, F f) {
+                                               const int *flag, int c, int lo,
+                                               int hi, F f) {
   if (la.cmask && !la.cmask[c]) return;  // uniform over the wave
   const int lane = threadIdx.x & 63;
-  const int hi = la.cell_start[c + 1];
-  for (int j0 = la.cell_start[c]; j0 < hi; j0 += 64 * kRuns) {
+  for (int j0 = lo; j0 < hi; j0 += 64 * kRuns) {
     int ii[kRuns];
 #pragma unroll
     for (int u = 0; u < kRuns; u++) {
@@ -771,27 +779,64 @@ __device__ __forceinline__ void for_cell_tiles(const DevParts &d,
   }
 }
 
+// Part w of kTileWaves of the slots [lo, hi), whole runs of 64.
+__device__ __forceinline__ int2 cell_part(int lo, int hi, int w) {
+  const int part = (hi - lo + 64 * kTileWaves - 1) / (64 * kTileWaves) * 64;
+  const int a = min(hi, lo + w * part);
+  return make_int2(a, min(hi, a + part));
+}
+// Bit q: cell c0 + q of a block's CPB cells is shared by its waves (the same
+// in every wave): at most 4 cells, those with more than a fifth of the block's
+// slots.  (Shared cells are taken one after the other, so more of a size are
+// done sooner by a wave each: 1000 cells of 1024 particles on average took
+// 107 us with every cell above 1024 shared, 70 like this.)
+template <int CPB>
+__device__ __forceinline__ unsigned long long shared_cells(const LoopArgs &la,
+                                                           int ncells, int c0) {
+  const int q = threadIdx.x & 63;
+  const bool in = q < CPB && c0 + q < ncells;
+  const int len =
+      in ? la.cell_start[c0 + q + 1] - la.cell_start[c0 + q] : 0;
+  int all = len;
+  for (int off = CPB / 2; off > 0; off >>= 1) all += __shfl_xor(all, off);
+  return __ballot(len > max(kTileOwn, all / 5));
+}
+
+template <int CPB>
 __global__ __launch_bounds__(kTileBlock) void k_tile_count(
     DevParts d, LoopArgs la, int mode, const int *flag, int ncells, int C,
     TileScratch ts) {
-  __shared__ unsigned long long sum[kTileCells];
-  const int w = threadIdx.x >> 6;
-  const int c = blockIdx.x * kTileCells + w;
+  __shared__ unsigned int sum[CPB];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c0 = blockIdx.x * CPB;
   if (blockIdx.x == 0 && threadIdx.x < 8 * 64) ts.heads[threadIdx.x] = 0;
-  unsigned long long v = 0ull;
-  if (c < ncells) {
-    unsigned int k = 0u;
-    for_cell_tiles(d, la, mode, flag, c,
-                   [&](int, bool take) { k += __popcll(__ballot(take)); });
-    v = ((unsigned long long)k << 32) | ((k + C - 1) / C);
-    if ((threadIdx.x & 63) == 0) ts.cell[c] = v;
-  }
-  if ((threadIdx.x & 63) == 0) sum[w] = v;
+  if (threadIdx.x < CPB) sum[threadIdx.x] = 0u;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < kTileCells; k++) v += sum[k];
-    ts.blk[blockIdx.x] = v;
+  unsigned long long big = shared_cells<CPB>(la, ncells, c0);
+  auto count = [&](int q, int lo, int hi) {
+    unsigned int k = 0u;
+    for_cell_tiles(d, la, mode, flag, c0 + q, lo, hi,
+                   [&](int, bool take) { k += __popcll(__ballot(take)); });
+    if (lane == 0 && k != 0u) atomicAdd(&sum[q], k);
+  };
+  if (w < CPB && c0 + w < ncells && !(big >> w & 1ull))
+    count(w, la.cell_start[c0 + w], la.cell_start[c0 + w + 1]);
+  for (; big != 0ull; big &= big - 1ull) {
+    const int q = __builtin_ctzll(big);
+    const int2 p =
+        cell_part(la.cell_start[c0 + q], la.cell_start[c0 + q + 1], w);
+    count(q, p.x, p.y);
   }
+  __syncthreads();
+  if (w > 0) return;
+  unsigned long long v = 0ull;  // of cell c0 + lane
+  if (lane < CPB && c0 + lane < ncells) {
+    const unsigned int k = sum[lane];
+    v = ((unsigned long long)k << 32) | ((k + C - 1) / C);
+    ts.cell[c0 + lane] = v;
+  }
+  for (int off = CPB / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  if (lane == 0) ts.blk[blockIdx.x] = v;
 }
 
 // One block: exclusive scan of the nb block sums in place; the totals close
@@ -818,31 +863,68 @@ __global__ __launch_bounds__(kScanBlock) void k_tile_scan(int nb,
   }
 }
 
+template <int CPB>
 __global__ __launch_bounds__(kTileBlock) void k_tile_fill(
     DevParts d, LoopArgs la, int mode, const int *flag, int ncells, int C,
     TileScratch ts) {
-  __shared__ unsigned long long sum[kTileCells];
+  __shared__ unsigned long long cell[CPB];  // as ts.cell
+  __shared__ unsigned long long at0[CPB];   // list and tiles before the cell
+  __shared__ int sum[kTileWaves];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int c = blockIdx.x * kTileCells + w;
-  const unsigned long long v = c < ncells ? ts.cell[c] : 0ull;
-  if (lane == 0) sum[w] = v;
-  __syncthreads();
-  if (v == 0ull) return;
-  unsigned long long base = ts.blk[blockIdx.x];
-  for (int k = 0; k < w; k++) base += sum[k];
-  const int t0 = (int)(unsigned int)base, l0 = (int)(base >> 32);
-  const int nt = (int)(unsigned int)v;
-  for (int t = lane; t < nt; t += 64) {
-    ts.tile_start[t0 + t] = l0 + t * C;
-    ts.tile_cell[t0 + t] = c;
+  const int c0 = blockIdx.x * CPB;
+  if (w == 0) {
+    const unsigned long long v =
+        lane < CPB && c0 + lane < ncells ? ts.cell[c0 + lane] : 0ull;
+    unsigned long long incl = v;
+    for (int off = 1; off < CPB; off <<= 1) {
+      const unsigned long long t = __shfl_up(incl, off);
+      if (lane >= off) incl += t;
+    }
+    if (lane < CPB) {
+      cell[lane] = v;
+      at0[lane] = ts.blk[blockIdx.x] + incl - v;
+    }
   }
-  int at = l0;
+  __syncthreads();
+  unsigned long long big = shared_cells<CPB>(la, ncells, c0);
+  // the cell's tiles, by `step` threads of which this is number `me`
+  auto tiles = [&](int q, int me, int step) {
+    const int t0 = (int)(unsigned int)at0[q], l0 = (int)(at0[q] >> 32);
+    const int nt = (int)(unsigned int)cell[q];
+    for (int t = me; t < nt; t += step) {
+      ts.tile_start[t0 + t] = l0 + t * C;
+      ts.tile_cell[t0 + t] = c0 + q;
+    }
+  };
   const unsigned long long below = (1ull << lane) - 1ull;
-  for_cell_tiles(d, la, mode, flag, c, [&](int i, bool take) {
-    const unsigned long long m = __ballot(take);
-    if (take) ts.alist[at + __popcll(m & below)] = i;
-    at += __popcll(m);
-  });
+  auto list = [&](int q, int lo, int hi, int at) {
+    for_cell_tiles(d, la, mode, flag, c0 + q, lo, hi, [&](int i, bool take) {
+      const unsigned long long m = __ballot(take);
+      if (take) ts.alist[at + __popcll(m & below)] = i;
+      at += __popcll(m);
+    });
+  };
+  if (w < CPB && c0 + w < ncells && !(big >> w & 1ull) && cell[w] != 0ull) {
+    tiles(w, lane, 64);
+    list(w, la.cell_start[c0 + w], la.cell_start[c0 + w + 1],
+         (int)(at0[w] >> 32));
+  }
+  for (; big != 0ull; big &= big - 1ull) {  // the same in every wave
+    const int q = __builtin_ctzll(big);
+    if (cell[q] == 0ull) continue;
+    tiles(q, (int)threadIdx.x, kTileBlock);
+    const int2 p =
+        cell_part(la.cell_start[c0 + q], la.cell_start[c0 + q + 1], w);
+    int k = 0;
+    for_cell_tiles(d, la, mode, flag, c0 + q, p.x, p.y,
+                   [&](int, bool take) { k += __popcll(__ballot(take)); });
+    if (lane == 0) sum[w] = k;
+    __syncthreads();
+    int at = (int)(at0[q] >> 32);
+    for (int j = 0; j < w; j++) at += sum[j];
+    __syncthreads();  // (sum is written again for the next cell)
+    list(q, p.x, p.y, at);
+  }
 }
 
 // Tiles with a particle of filt[i] != 0, appended to ids with one atomic
@@ -945,12 +1027,24 @@ hipError_t launch_build_tiles(const DevParts &d, const LoopArgs &la, int n,
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, ts.nlist, 1);
     return hipGetLastError();
   }
-  const int nb = nblk(ncells, kTileCells);
-  hipLaunchKernelGGL(k_tile_count, dim3(nb), dim3(kTileBlock), 0, st, d, la,
-                     mode, flag, ncells, C, ts);
+  // A block per cell where nearly all cells are shared and their blocks do
+  // not outnumber the work (1000 cells of 1024 particles 70 us by 16 cells in
+  // a block, 77 by one; of 4096 103 and 85; 512 cells of 1024 61 and 58).
+  const bool wide = n / ncells >= max(kTileOwn, 2 * ncells);
+  const int nb = wide ? ncells : nblk(ncells, kTileWaves);
+  if (wide)
+    hipLaunchKernelGGL((k_tile_count<1>), dim3(nb), dim3(kTileBlock), 0, st, d,
+                       la, mode, flag, ncells, C, ts);
+  else
+    hipLaunchKernelGGL((k_tile_count<kTileWaves>), dim3(nb), dim3(kTileBlock),
+                       0, st, d, la, mode, flag, ncells, C, ts);
   hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(kScanBlock), 0, st, nb, ts);
-  hipLaunchKernelGGL(k_tile_fill, dim3(nb), dim3(kTileBlock), 0, st, d, la,
-                     mode, flag, ncells, C, ts);
+  if (wide)
+    hipLaunchKernelGGL((k_tile_fill<1>), dim3(nb), dim3(kTileBlock), 0, st, d,
+                       la, mode, flag, ncells, C, ts);
+  else
+    hipLaunchKernelGGL((k_tile_fill<kTileWaves>), dim3(nb), dim3(kTileBlock),
+                       0, st, d, la, mode, flag, ncells, C, ts);
   return hipGetLastError();
 }
 

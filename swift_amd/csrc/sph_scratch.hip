@@ -24,7 +24,7 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t scratch_bytes(size_t n, size_t nc) {
   const size_t tcap = n / kMinTile + nc + 1;
   return align256(8 * nc)                         // cell
-         + align256(8 * (nc / kTileCells + 1))    // blk
+         + align256(8 * nc)                       // blk
          + align256(4 * n)                        // alist
          + 3 * align256(4 * tcap)                 // tile_start, _cell, ids
          + 3 * align256(4)                        // nlist, ntiles, nids
@@ -86,7 +86,7 @@ hipError_t noalloc_scratch(int device, int64_t n, int ncells, TileScratch *ts,
     return p;
   };
   ts->cell = (unsigned long long *)take(8 * nc);
-  ts->blk = (unsigned long long *)take(8 * (nc / kTileCells + 1));
+  ts->blk = (unsigned long long *)take(8 * nc);
   ts->alist = (int *)take(4 * nn);
   ts->tile_start = (int *)take(4 * tcap);
   ts->tile_cell = (int *)take(4 * tcap);

@@ -210,3 +210,63 @@ def test_tiles16_tasks_over_several_windows(orc, box, how):
         ref = eng.results(["h"])
     # (sums in another order can end the iteration a step apart)
     assert np.allclose(ref["h"], res["h"], rtol=2 * props.h_tolerance)
+
+
+@pytest.mark.parametrize("nc,big", [
+    (3, {}), (3, {0: 1024}), (3, {5: 1025, 26: 1087}), (4, {15: 16385}),
+    (4, {16: 3000, 17: 2900, 18: 2800, 31: 5000}), (4, {0: 1500, 63: 40000}),
+    (3, {c: 1100 + 37 * c for c in range(27)}),
+    (5, {c: 1030 + c for c in range(0, 125, 2)})])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_tile_builder_takes_every_particle(nc, big, mixed):
+    """The builder's list holds the active particles of the selected cells,
+    where a wave takes a cell, where a cell is shared by the waves of its
+    block (more than 1024 slots and a fifth of the block's), and where every
+    cell has a block: seen through init_cells, which clears their density."""
+    from swift_amd import Engine, HydroProps
+    from swift_amd.ics import TIME_BIN_INHIBITED
+    rng = np.random.default_rng(nc + len(big))
+    ncells = nc ** 3
+    counts = rng.integers(0, 40, ncells)
+    for c, k in big.items():
+        counts[c] = k
+    cell = rng.permutation(np.repeat(np.arange(ncells), counts))
+    corner = np.stack([cell // (nc * nc), cell // nc % nc, cell % nc], 1)
+    n = cell.size
+    st = {k: np.ones(n, np.float32) for k in (
+        "m", "u", "rho", "pressure", "soundspeed", "f", "balsara",
+        "alpha_visc", "alpha_diff", "div_v_prev")}
+    st["x"] = (corner + rng.uniform(0.01, 0.99, (n, 3))) / nc
+    st["v"] = np.zeros((n, 3), np.float32)
+    st["h"] = np.full(n, 0.01, np.float32)
+    st["time_bin"] = (rng.choice([1, 2, 3, 5, TIME_BIN_INHIBITED], n) if mixed
+                      else np.full(n, 2)).astype(np.int8)
+    with Engine(HydroProps(ncell=(nc,) * 3, max_active_bin=2)) as eng:
+        eng.set_particles(st)
+        act = st["time_bin"] <= 2
+        left = np.ones(n, bool)
+        for sel in (np.arange(0, ncells, 3), np.arange(ncells - 1, -1, -1)):
+            eng.init_cells(sel)
+            left &= ~(act & np.isin(cell, sel))
+            assert np.array_equal(eng.get("rho"), left.astype(np.float32))
+
+
+@pytest.mark.parametrize("n_side,ncell,frac", [(31, 3, 1.0), (31, 3, 0.1)])
+def test_tiles16_of_large_cells(n_side, ncell, frac):
+    """Every cell has a block of the builder (1100 particles in each of 27):
+    the grid schedule's results, eager and captured."""
+    from swift_amd import HydroProps, ics
+    st = ics.modulated_box(n_side, seed=n_side, amp=0.3)
+    if frac < 1:
+        ics.set_active_fraction(st, frac, seed=1)
+        st["rho"] = np.ones_like(st["rho"])
+        st["pressure"] = (st["u"] * np.float32(2 / 3)).astype(np.float32)
+        st["soundspeed"] = np.sqrt(st["pressure"] * np.float32(5 / 3))
+    props = HydroProps(ncell=(ncell,) * 3)
+    s0, r0 = _run(props, st, 0, (16, 16))
+    for kw in (dict(mode=1, shape=(16, 16)), dict(mode=1, shape=(16, 16),
+                                                  graph=True)):
+        s1, r1 = _run(props, st, **kw)
+        for k in r0:
+            assert np.array_equal(r0[k], r1[k], equal_nan=True), (kw, k)
+        assert s0["n_density_all"] == s1["n_density_all"], kw
