@@ -122,8 +122,8 @@ int swsph_set_particles(swsph_engine *e, const swsph_host_parts *p);
 int swsph_get_field(swsph_engine *e, int field, void *host_out);
 /* nf fields at once (as swsph_get_field each), with one wait at the end:
  * up to 2 MiB in all go through a page-locked block of the engine, with
- * page-locked outputs (hipHostMalloc) up to 320 KiB per field beyond the
- * first; above that the copies go to the outputs themselves, with page-locked
+ * page-locked outputs (hipHostMalloc) and at most 24 bytes per particle up to
+ * 320 KiB per field beyond the first; above that the copies go to the outputs themselves, with page-locked
  * ones as asynchronous DMA behind each other. */
 int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
                      void *const *outs);

@@ -2636,12 +2636,13 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
   // copy into the engine's pinned block, and from there by the host; above
   // that the copies go to the caller's memory themselves.  The host's copy
   // costs 36 us per MiB, a copy of its own 8 us and more per field (and for
-  // pageable memory the runtime's staging): with page-locked outputs the
+  // pageable memory the runtime's staging, for more than the staging buffer
+  // takes at once a wait of 30 us): with page-locked outputs and one sweep the
   // block pays up to kOwnCopy bytes per field beyond the first.  Microseconds
   // for one field of 0.25 / 1 / 2 MiB to page-locked memory: 26 / 42 / 62 by its
-  // own copy, 33 / 80 / 132 through the block; three fields of 0.6 MiB in
-  // all 51 both ways, six of 2 MiB 118 both ways, 25 of 1.4 MiB 97 through
-  // the block.  Pageable: 34 / 84 / 132 by the runtime, 33 / 86 / 128 through
+  // own copy, 33 / 80 / 132 through the block; two, three, four fields even at
+  // 0.35, 0.65, 0.95 MiB in all; six in two sweeps of 1 / 2 MiB 104 / 122 and
+  // 71 / 116.  Pageable: 34 / 84 / 132 by the runtime, 33 / 86 / 128 through
   // the block, three fields 107-172 and 34-97.
   auto padded = [](size_t bytes) { return (bytes + 15) & ~(size_t)15; };
   size_t total = 0;
@@ -2658,13 +2659,18 @@ int swsph_get_fields(swsph_engine *e, int nf, const int *fields,
       small = 0;  // not the host's to write
     }
   }
-  constexpr size_t kOwnCopy = 320 << 10;
-  if (locked && nf > 0) small = std::min(small, kOwnCopy * (nf - 1));
-  for (int q = 0; q < nf && total <= small; q++) {
+  size_t bytes_per = 0;  // of a particle
+  for (int q = 0; q < nf; q++) {
     FieldView v;
     (void)field_view(e->d, fields[q], v);
-    total += padded((size_t)v.esize() * v.ncomp * n);
+    const size_t bytes = (size_t)v.esize() * v.ncomp;
+    bytes_per += bytes;
+    total += padded(bytes * n);
   }
+  constexpr size_t kOwnCopy = 320 << 10;
+  if (locked && nf > 0 &&
+      bytes_per <= swsph_engine::kStageWords * sizeof(double))
+    small = std::min(small, kOwnCopy * (nf - 1));
   if (total <= small) {
     if (total > e->cap_read) {
       if (e->h_read) (void)hipHostFree(e->h_read);
