@@ -241,7 +241,7 @@ int swsph_pass_graph(swsph_engine *e, swsph_pass_stats *stats);
 /* swsph_pass_batched without any device allocation: the pass's scratch
  * (the work queue: cell counts, compact particle list, tile table and
  * queue heads; the ghost and interaction counters) lives in one
- * fixed device array of the library (about 16 MB per GPU, held from the
+ * fixed device array of the library (about 17 MB per GPU, held from the
  * first engine creation on that GPU until the process ends) instead of the
  * engine's buffers.  Same kernels and launches, so the results are
  * bit-identical to swsph_pass_batched.  Limits: at most 2^21 particles on

@@ -384,7 +384,8 @@ void free_dev(swsph_engine *e) {
                   e->d.divv_dt, e->d.ax, e->d.ay, e->d.az, e->d.udt, e->d.hdt,
                   e->d.nf, e->d.mintb, e->d.rd, e->d.rg, e->d.rf, e->d.pos,
                   e->d.r2b, e->d.lfb, e->d.sel, e->d.cell, e->nl.idx,
-                  e->nl.cnt, e->ts.cell, e->ts.blk, e->ts.alist, e->ts.nlist,
+                  e->nl.cnt, e->ts.cell, e->ts.first, e->ts.blk, e->ts.big,
+                  e->ts.part, e->ts.alist, e->ts.nlist,
                   e->ts.tile_start, e->ts.tile_cell, e->ts.ntiles, e->ts.ids,
                   e->ts.nids, e->ts.heads,
                   e->d_cell_start, e->d_tiles, e->d.vfx, e->d.vfy, e->d.vfz,
@@ -689,7 +690,10 @@ int alloc_dev(swsph_engine *e, size_t n) {
     TileScratch &t = e->ts;
     const size_t nc = (size_t)e->ncells;
     HIPCHK(dalloc(&t.cell, nc));
-    HIPCHK(dalloc(&t.blk, nc));
+    HIPCHK(dalloc(&t.first, nc));
+    HIPCHK(dalloc(&t.blk, tile_blocks(n, nc)));
+    HIPCHK(dalloc(&t.big, tile_blocks(n, nc)));
+    HIPCHK(dalloc(&t.part, tile_parts(n)));
     HIPCHK(dalloc(&t.alist, n));
     HIPCHK(dalloc(&t.nlist, 1));
     // a cell of k particles makes ceil(k / C) tiles: at most n / C + nc

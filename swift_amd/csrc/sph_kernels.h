@@ -292,10 +292,27 @@ struct StepArgs {
   int max_active_bin, fixed, lo, hi;
 };
 
+// The tile builder: the waves of a block, the slots that a wave always takes
+// alone, and the mean number of slots per cell from which a block may take a
+// single cell (else as many cells as it has waves).
+constexpr int kTileWaves = 16, kTileOwn = 1024, kTileWide = 1024;
+constexpr size_t tile_blocks(size_t n, size_t ncells) {
+  const size_t wide = n / kTileWide < ncells ? n / kTileWide : ncells;
+  const size_t some = ncells / kTileWaves + 1;
+  return some > wide ? some : wide;
+}
+// Counts of the parts of shared cells: such a cell has more than kTileOwn
+// slots, so its first slot / kTileOwn is no other such cell's.
+constexpr size_t tile_parts(size_t n) {
+  return kTileWaves * (n / kTileOwn + 1);
+}
 // Scratch of the tile builder, sized for n particles and ncells cells.
 struct TileScratch {
   unsigned long long *cell;  // [ncells] selected particles << 32 | tiles
-  unsigned long long *blk;   // [ncells] their sums by block
+  unsigned long long *first; // [ncells] the same before the cell in its block
+  unsigned long long *blk;   // [tile_blocks] their sums by block
+  unsigned int *big;         // [tile_blocks] the cells that its waves share
+  int *part;                 // [tile_parts] the particles of their parts
   int *alist;       // [n] the selected particles, in cell order
   int *nlist;       // [1] their number
   int *tile_start;  // [n / C + ncells + 1] for the smallest C in use

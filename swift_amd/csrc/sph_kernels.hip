@@ -702,13 +702,15 @@ __global__ void k_count_active(const int8_t *__restrict__ tb, int n,
 // per slot: 35 us of launches on a small box, 150-200 us at 16.8 M slots.)
 // Bound by the latency of a wave's dependent loads, 512 slots at a time: with
 // one wave for every cell a bundle on 4096 cells, one of 20000 / 100000 / 300000
-// particles, took 238 / 727 / 1950 us, shared 134 / 204 / 369; a pass over a
-// halo of 69000 in a cell, 1 % active, 2.10 ms, shared 1.74; 27 cells of 16384
-// each 194 us, shared in blocks of a cell each 59.
-constexpr int kTileWaves = 16;  // waves, and cells (or one), per block
+// particles, took 238 / 727 / 1950 us, shared 130 / 174 / 289; a pass over a
+// halo of 69000 in a cell, 1 % active, 2.10 ms, shared 1.71; 27 cells of 16384
+// each 194 us, shared in blocks of a cell each 52.  The fill waits for no other
+// wave: what precedes a cell in its block, and a part in its cell, comes from
+// the count (fill of 144^3 31.8 us with barriers and a second count, 21.9 like
+// this; count 18.2 and 22.3).
 constexpr int kTileBlock = 64 * kTileWaves;
 constexpr int kScanBlock = 1024;
-constexpr int kTileOwn = 1024;  // slots that a wave always takes alone
+constexpr int kTileShared = 4;  // cells that a block shares, at most
 
 // Exclusive scan of v over a block of kScanBlock threads; *total receives
 // the block sum.
@@ -785,58 +787,83 @@ __device__ __forceinline__ int2 cell_part(int lo, int hi, int w) {
   const int a = min(hi, lo + w * part);
   return make_int2(a, min(hi, a + part));
 }
-// Bit q: cell c0 + q of a block's CPB cells is shared by its waves (the same
-// in every wave): at most 4 cells, those with more than a fifth of the block's
-// slots.  (Shared cells are taken one after the other, so more of a size are
-// done sooner by a wave each: 1000 cells of 1024 particles on average took
-// 107 us with every cell above 1024 shared, 70 like this.)
-template <int CPB>
-__device__ __forceinline__ unsigned long long shared_cells(const LoopArgs &la,
-                                                           int ncells, int c0) {
-  const int q = threadIdx.x & 63;
-  const bool in = q < CPB && c0 + q < ncells;
-  const int len =
-      in ? la.cell_start[c0 + q + 1] - la.cell_start[c0 + q] : 0;
-  int all = len;
-  for (int off = CPB / 2; off > 0; off >>= 1) all += __shfl_xor(all, off);
-  return __ballot(len > max(kTileOwn, all / 5));
+// The counts of the parts of a shared cell whose first slot is lo.
+__device__ __forceinline__ int *tile_part(const TileScratch &ts, int lo) {
+  return ts.part + lo / kTileOwn * kTileWaves;
 }
 
+// The block's CPB cells: at most kTileShared of them, those with more than
+// kTileOwn slots and a fifth of the block's, are shared by its waves, the
+// others taken by a wave each.  (Shared cells are taken one after the other,
+// so more of a size are done sooner by a wave each: 1000 cells of 1024
+// particles on average took 107 us with every cell above 1024 shared, 70 like
+// this.)
 template <int CPB>
 __global__ __launch_bounds__(kTileBlock) void k_tile_count(
     DevParts d, LoopArgs la, int mode, const int *flag, int ncells, int C,
     TileScratch ts) {
-  __shared__ unsigned int sum[CPB];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __shared__ int sum[CPB];                       // of a cell
+  __shared__ int parts[kTileShared][kTileWaves]; // of a shared cell's parts
+  const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6));
   const int c0 = blockIdx.x * CPB;
   if (blockIdx.x == 0 && threadIdx.x < 8 * 64) ts.heads[threadIdx.x] = 0;
-  if (threadIdx.x < CPB) sum[threadIdx.x] = 0u;
-  __syncthreads();
-  unsigned long long big = shared_cells<CPB>(la, ncells, c0);
-  auto count = [&](int q, int lo, int hi) {
-    unsigned int k = 0u;
-    for_cell_tiles(d, la, mode, flag, c0 + q, lo, hi,
+  // lane q holds the slots of cell c0 + q
+  const bool in = lane < CPB && c0 + lane < ncells;
+  const int lo = in ? la.cell_start[c0 + lane] : 0;
+  const int hi = in ? la.cell_start[c0 + lane + 1] : 0;
+  unsigned int shared = 0u;  // bit q: cell c0 + q (the same in every wave)
+  if (__any(hi - lo > kTileOwn)) {  // uniform
+    int all = hi - lo;
+    for (int off = CPB / 2; off > 0; off >>= 1) all += __shfl_xor(all, off);
+    shared = (unsigned int)__ballot(
+        hi - lo > max(kTileOwn, all / (kTileShared + 1)));
+  }
+  auto count = [&](int q, int a, int b) -> int {
+    int k = 0;
+    for_cell_tiles(d, la, mode, flag, c0 + q, a, b,
                    [&](int, bool take) { k += __popcll(__ballot(take)); });
-    if (lane == 0 && k != 0u) atomicAdd(&sum[q], k);
+    return k;
   };
-  if (w < CPB && c0 + w < ncells && !(big >> w & 1ull))
-    count(w, la.cell_start[c0 + w], la.cell_start[c0 + w + 1]);
-  for (; big != 0ull; big &= big - 1ull) {
-    const int q = __builtin_ctzll(big);
-    const int2 p =
-        cell_part(la.cell_start[c0 + q], la.cell_start[c0 + q + 1], w);
-    count(q, p.x, p.y);
+  if (w < CPB && c0 + w < ncells && !(shared >> w & 1u)) {
+    const int k = count(w, __builtin_amdgcn_readlane(lo, w),
+                        __builtin_amdgcn_readlane(hi, w));
+    if (lane == 0) sum[w] = k;
+  }
+  int n = 0;
+  for (unsigned int big = shared; big != 0u; big &= big - 1u, n++) {
+    const int q = __builtin_ctz(big);
+    const int lo_q = __builtin_amdgcn_readlane(lo, q);
+    const int2 p = cell_part(lo_q, __builtin_amdgcn_readlane(hi, q), w);
+    const int k = count(q, p.x, p.y);
+    if (lane == 0) {
+      parts[n][w] = k;
+      tile_part(ts, lo_q)[w] = k;
+    }
   }
   __syncthreads();
   if (w > 0) return;
   unsigned long long v = 0ull;  // of cell c0 + lane
-  if (lane < CPB && c0 + lane < ncells) {
-    const unsigned int k = sum[lane];
-    v = ((unsigned long long)k << 32) | ((k + C - 1) / C);
+  if (in) {
+    int k = 0;
+    if (shared >> lane & 1u) {
+      const int at = __popc(shared & ((1u << lane) - 1u));
+      for (int j = 0; j < kTileWaves; j++) k += parts[at][j];
+    } else {
+      k = sum[lane];
+    }
+    v = ((unsigned long long)k << 32) | (unsigned int)((k + C - 1) / C);
     ts.cell[c0 + lane] = v;
   }
-  for (int off = CPB / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  if (lane == 0) ts.blk[blockIdx.x] = v;
+  unsigned long long incl = v;
+  for (int off = 1; off < CPB; off <<= 1) {
+    const unsigned long long t = __shfl_up(incl, off);
+    if (lane >= off) incl += t;
+  }
+  if (in) ts.first[c0 + lane] = incl - v;
+  if (lane == CPB - 1) {
+    ts.blk[blockIdx.x] = incl;
+    ts.big[blockIdx.x] = shared;
+  }
 }
 
 // One block: exclusive scan of the nb block sums in place; the totals close
@@ -867,63 +894,46 @@ template <int CPB>
 __global__ __launch_bounds__(kTileBlock) void k_tile_fill(
     DevParts d, LoopArgs la, int mode, const int *flag, int ncells, int C,
     TileScratch ts) {
-  __shared__ unsigned long long cell[CPB];  // as ts.cell
-  __shared__ unsigned long long at0[CPB];   // list and tiles before the cell
-  __shared__ int sum[kTileWaves];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int c0 = blockIdx.x * CPB;
-  if (w == 0) {
-    const unsigned long long v =
-        lane < CPB && c0 + lane < ncells ? ts.cell[c0 + lane] : 0ull;
-    unsigned long long incl = v;
-    for (int off = 1; off < CPB; off <<= 1) {
-      const unsigned long long t = __shfl_up(incl, off);
-      if (lane >= off) incl += t;
-    }
-    if (lane < CPB) {
-      cell[lane] = v;
-      at0[lane] = ts.blk[blockIdx.x] + incl - v;
-    }
-  }
-  __syncthreads();
-  unsigned long long big = shared_cells<CPB>(la, ncells, c0);
+  const unsigned long long base = ts.blk[blockIdx.x];
+  unsigned int big = ts.big[blockIdx.x];
+  // the wave's own cell (all loads in flight together)
+  const int c = c0 + (w < CPB && c0 + w < ncells ? w : 0);
+  const unsigned long long own = ts.cell[c], at0 = base + ts.first[c];
+  const int lo = la.cell_start[c], hi = la.cell_start[c + 1];
   // the cell's tiles, by `step` threads of which this is number `me`
-  auto tiles = [&](int q, int me, int step) {
-    const int t0 = (int)(unsigned int)at0[q], l0 = (int)(at0[q] >> 32);
-    const int nt = (int)(unsigned int)cell[q];
+  auto tiles = [&](int cell, unsigned long long v, unsigned long long at,
+                   int me, int step) {
+    const int t0 = (int)(unsigned int)at, l0 = (int)(at >> 32);
+    const int nt = (int)(unsigned int)v;
     for (int t = me; t < nt; t += step) {
       ts.tile_start[t0 + t] = l0 + t * C;
-      ts.tile_cell[t0 + t] = c0 + q;
+      ts.tile_cell[t0 + t] = cell;
     }
   };
   const unsigned long long below = (1ull << lane) - 1ull;
-  auto list = [&](int q, int lo, int hi, int at) {
-    for_cell_tiles(d, la, mode, flag, c0 + q, lo, hi, [&](int i, bool take) {
+  auto list = [&](int cell, int a, int b, int at) {
+    for_cell_tiles(d, la, mode, flag, cell, a, b, [&](int i, bool take) {
       const unsigned long long m = __ballot(take);
       if (take) ts.alist[at + __popcll(m & below)] = i;
       at += __popcll(m);
     });
   };
-  if (w < CPB && c0 + w < ncells && !(big >> w & 1ull) && cell[w] != 0ull) {
-    tiles(w, lane, 64);
-    list(w, la.cell_start[c0 + w], la.cell_start[c0 + w + 1],
-         (int)(at0[w] >> 32));
+  if (w < CPB && c0 + w < ncells && !(big >> w & 1u) && own != 0ull) {
+    tiles(c, own, at0, lane, 64);
+    list(c, lo, hi, (int)(at0 >> 32));
   }
-  for (; big != 0ull; big &= big - 1ull) {  // the same in every wave
-    const int q = __builtin_ctzll(big);
-    if (cell[q] == 0ull) continue;
-    tiles(q, (int)threadIdx.x, kTileBlock);
-    const int2 p =
-        cell_part(la.cell_start[c0 + q], la.cell_start[c0 + q + 1], w);
-    int k = 0;
-    for_cell_tiles(d, la, mode, flag, c0 + q, p.x, p.y,
-                   [&](int, bool take) { k += __popcll(__ballot(take)); });
-    if (lane == 0) sum[w] = k;
-    __syncthreads();
-    int at = (int)(at0[q] >> 32);
-    for (int j = 0; j < w; j++) at += sum[j];
-    __syncthreads();  // (sum is written again for the next cell)
-    list(q, p.x, p.y, at);
+  for (; big != 0u; big &= big - 1u) {
+    const int cb = c0 + __builtin_ctz(big);
+    const unsigned long long v = ts.cell[cb], b0 = base + ts.first[cb];
+    const int lo_b = la.cell_start[cb];
+    int before = lane < w ? tile_part(ts, lo_b)[lane] : 0;  // of the list
+    tiles(cb, v, b0, (int)threadIdx.x, kTileBlock);
+    const int2 p = cell_part(lo_b, la.cell_start[cb + 1], w);
+    for (int off = kTileWaves / 2; off > 0; off >>= 1)
+      before += __shfl_xor(before, off);
+    list(cb, p.x, p.y, (int)(b0 >> 32) + uniform(before));
   }
 }
 
@@ -1030,7 +1040,7 @@ hipError_t launch_build_tiles(const DevParts &d, const LoopArgs &la, int n,
   // A block per cell where nearly all cells are shared and their blocks do
   // not outnumber the work (1000 cells of 1024 particles 70 us by 16 cells in
   // a block, 77 by one; of 4096 103 and 85; 512 cells of 1024 61 and 58).
-  const bool wide = n / ncells >= max(kTileOwn, 2 * ncells);
+  const bool wide = n / ncells >= max(kTileWide, 2 * ncells);
   const int nb = wide ? ncells : nblk(ncells, kTileWaves);
   if (wide)
     hipLaunchKernelGGL((k_tile_count<1>), dim3(nb), dim3(kTileBlock), 0, st, d,

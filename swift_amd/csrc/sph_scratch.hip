@@ -24,7 +24,10 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t scratch_bytes(size_t n, size_t nc) {
   const size_t tcap = n / kMinTile + nc + 1;
   return align256(8 * nc)                         // cell
-         + align256(8 * nc)                       // blk
+         + align256(8 * nc)                       // first
+         + align256(8 * tile_blocks(n, nc))       // blk
+         + align256(4 * tile_blocks(n, nc))       // big
+         + align256(4 * tile_parts(n))            // part
          + align256(4 * n)                        // alist
          + 3 * align256(4 * tcap)                 // tile_start, _cell, ids
          + 3 * align256(4)                        // nlist, ntiles, nids
@@ -41,7 +44,7 @@ void *g_ptr[kMaxDevices] = {};
 
 }  // namespace
 
-// The scratch itself (about 16 MB for the limits in sph_kernels.h).
+// The scratch itself (about 17 MB for the limits in sph_kernels.h).
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace sphk {
@@ -86,7 +89,10 @@ hipError_t noalloc_scratch(int device, int64_t n, int ncells, TileScratch *ts,
     return p;
   };
   ts->cell = (unsigned long long *)take(8 * nc);
-  ts->blk = (unsigned long long *)take(8 * nc);
+  ts->first = (unsigned long long *)take(8 * nc);
+  ts->blk = (unsigned long long *)take(8 * tile_blocks(nn, nc));
+  ts->big = (unsigned int *)take(4 * tile_blocks(nn, nc));
+  ts->part = (int *)take(4 * tile_parts(nn));
   ts->alist = (int *)take(4 * nn);
   ts->tile_start = (int *)take(4 * tcap);
   ts->tile_cell = (int *)take(4 * tcap);

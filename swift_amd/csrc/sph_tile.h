@@ -19,8 +19,8 @@
 //
 // Bound: the walk's gathers and VALU issue together, in waves that run as long
 // as their fullest lane (busy share of the cycles, L1 return path / VALU, on
-// modulated 97^3 and clustered 144^3: density 0.92 / 0.81 and 0.89 / 0.95,
-// gradient 0.95 / 0.87 and 0.95 / 0.84, force 0.95 / 0.79 and 0.95 / 0.81).
+// modulated 97^3 and clustered 144^3: density 0.86-0.92 / 0.78-0.81 and 0.88 /
+// 0.95, gradient 0.95 / 0.88 and 0.95 / 0.84, force 0.95 / 0.79 and 0.95 / 0.81).
 // A window of 512 rows evens the lanes out better than the chunk engine's
 // 128 (modulated 97^3 box: 26 -> 21 iterations per tile at 256 for 13.5 hits
 // per lane; 512 rows in lists of 32 against 256 in lists of 44: density -4 %,
